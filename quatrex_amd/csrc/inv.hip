@@ -3,6 +3,9 @@
 // Replaces the batched `linalg.inv` of the reference
 // (src/qttools/kernels/linalg/inv.py:24-40, LAPACK/cuSOLVER getrf+getri).
 //
+// Up to n = 128 (complex128) one workgroup inverts a matrix that stays in MFMA
+// result registers (inv_whole, gj_core.h).  Above, and in complex64:
+//
 // Algorithm: blocked in-place Gauss-Jordan elimination split into kernels so
 // that the O(n^3) part runs on every CU of the chip while the sequential
 // pivoting chain stays short:
@@ -38,6 +41,7 @@
 // D[4(l/16) + e][l%16] (f32).
 #include <cstdlib>
 
+#include "gj_core.h"
 #include "qx_internal.h"
 
 namespace qx {
@@ -932,6 +936,28 @@ __global__ __launch_bounds__(512) void inv_step(PanelArgs pa, UpdArgs ua, int ba
   update_tile<T, 32, 32>(ua, u, in && update_live(ua, u), threadIdx.x & (NT - 1), sh.u[half]);
 }
 
+// Whole matrices in registers (gj_core.h): shapes for n <= 64, 96, 128
+// (GjWhole32 there).
+typedef GjShape<4, 1, 4, 1, 8> GjWhole64;
+typedef GjShape<6, 1, 6, 2, 8> GjWhole96;
+typedef GjShape<8, 1, 8, 2, 8> GjWhole128;
+
+// Whole inverse X = (A - S)^-1 of one n x n matrix per workgroup, n <= G::C.
+// Bound by the pivot chain: at n = 64 a column takes ~900 cycles on the
+// factoring wave (57 k of 94 k cycles), the rank-8 updates on the matrix cores
+// 11 k, the exchange of the pivot rows 13 k; at n = 128 (two rows per lane)
+// 1300 cycles a column, 167 k of 371 k, the updates 131 k.
+template <typename G>
+__global__ __launch_bounds__(G::THREADS) void inv_whole(int n, const z2* A, int64_t sA, int lda,
+                                                        const z2* S, int64_t sS, int lds, z2* X,
+                                                        int64_t sX, int ldx, int* info,
+                                                        const int* mask) {
+  __shared__ GjShared<G> sh;
+  const int64_t e = blockIdx.x;
+  if (mask && !mask[e]) return;  // uniform over the workgroup
+  gj_invert<G>(n, A + e * sA, lda, S ? S + e * sS : nullptr, lds, X + e * sX, ldx, info + e, sh);
+}
+
 // X[r, c] = Y[r, idx c]; X may not alias Y.
 __global__ __launch_bounds__(NT) void inv_gather(int n, const z2* Y, int64_t sY, int ldy, z2* X,
                                                  int64_t sX, int ldx, const int* ints, int64_t sI,
@@ -977,6 +1003,13 @@ int inv_panel_kind() {
   const char* e = std::getenv("QX_INV_PANEL");
   const int v = e ? std::atoi(e) : 0;
   return (v == 1 || v == 4) ? v : 0;
+}
+
+// QX_INV_NB (read per call), 0 when not set to a width there is.
+int forced_panel_width() {
+  const char* e = std::getenv("QX_INV_NB");
+  const int v = e ? std::atoi(e) : 0;
+  return (v == 16 || v == 32 || v == 64) ? v : 0;
 }
 
 int inv_group_width() {
@@ -1131,6 +1164,37 @@ void run_inverse(hipStream_t s, int64_t batch, int n, const Mat& X, const InvScr
                      mask);
 }
 
+// Largest size whose whole inverse runs in one workgroup per matrix: 128 in
+// complex128 unless another panel kernel or panel width is forced
+// (QX_INV_PANEL, QX_INV_NB); QX_INV_WHOLE=<n> (read per call) lowers it (0:
+// none).  At 128 the line is where the matrix still fits the registers of one
+// CU (256 KB of accumulators).  us per call against the split panel and update
+// kernels (n <= 32: against one workgroup of four waves per matrix):
+//   64 x 32^2 20 / 30, 1024 x 32^2 29 / 58, 64 x 64^2 44 / 107, 1024 x 64^2
+//   164 / 330, 32 x 96^2 109 / 159, 256 x 96^2 123 / 241, 32 x 128^2 168 /
+//   224, 512 x 128^2 373 / 618.
+// Panels of larger matrices held and factored the same way (32 columns of 256
+// rows) took 42 us instead of 47, and the step with its own update longer than
+// the look-ahead's: 32 x 256^2 497-553 against 490, so those stay as they are.
+int inv_whole_max() {
+  if (inv_panel_kind() != 0 || forced_panel_width() != 0) return 0;
+  const char* e = std::getenv("QX_INV_WHOLE");
+  return e ? min(std::atoi(e), 128) : 128;
+}
+
+void launch_whole(hipStream_t s, int64_t batch, int n, const Mat& A, const Mat& S, const Mat& X,
+                  int* info, const int* mask) {
+#define QX_WHOLE(G)                                                                          \
+  hipLaunchKernelGGL((inv_whole<G>), dim3((unsigned)batch), dim3(G::THREADS), 0, s, n, A.p,  \
+                     A.stride, A.ld, S.p, S.stride, S.ld, X.p, X.stride, X.ld, info, mask)
+  if (n <= 32) QX_WHOLE(GjWhole32);
+  else if (n <= 64) QX_WHOLE(GjWhole64);
+  else if (n <= 96) QX_WHOLE(GjWhole96);
+  else QX_WHOLE(GjWhole128);
+#undef QX_WHOLE
+  QX_HIP_CHECK(hipGetLastError());
+}
+
 }  // namespace
 
 // Panel width: 32 columns; with the older panel kernels 16 above n = 256
@@ -1139,15 +1203,14 @@ void run_inverse(hipStream_t s, int64_t batch, int n, const Mat& X, const InvScr
 // column-group panel of eight waves of eight columns, whose rank-64 updates
 // pass over the matrix half as often).
 int inv_panel_width(int n) {
-  const char* e = std::getenv("QX_INV_NB");  // read per call
-  const int v = e ? std::atoi(e) : 0;
-  const int forced_nb = (v == 16 || v == 32 || v == 64) ? v : 0;
+  const int forced_nb = forced_panel_width();
   if (n > 256) return inv_panel_kind() == 0 ? 32 : 16;
   if (forced_nb == 64 && inv_panel_kind() != 0) return 32;
   return forced_nb ? forced_nb : 32;
 }
 
-Mat zinv_input(int n, const Mat& X, const InvScratch& scr) {
+Mat zinv_input(int n, const Mat& X, const InvScratch& scr, int precision) {
+  if (precision != QX_PREC_C64 && n <= inv_whole_max()) return X;
   const int NB = inv_panel_width(n);
   const int npan = (n + NB - 1) / NB;
   // the panels ping-pong between X and the scratch buffer, the last one
@@ -1172,8 +1235,9 @@ void zinv(hipStream_t s, int64_t batch, int n, const Mat& A, const Mat& S, const
   hipEvent_t ev0 = nullptr;
   if (timer) timer->begin(s, &ev0);
 
-  // n <= 32 in complex128: one wave per matrix, one launch
-  if (precision != QX_PREC_C64 && inv_small(s, batch, n, A, S, X, info, mask)) {
+  // complex128 up to 128: the whole inverse in one launch
+  if (precision != QX_PREC_C64 && n <= inv_whole_max()) {
+    launch_whole(s, batch, n, A, S, X, info, mask);
     if (timer) timer->end(s, ev0, KernelTimer::INV, 8.0 * (double)n * n * n * batch);
     return;
   }

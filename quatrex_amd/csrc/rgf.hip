@@ -119,7 +119,7 @@ struct OzSubBatch {
 // entries are of the order of the FP32 rounding error and would be lost in
 // FP32), the small correction X R by the FP32 GEMM.  Mc and R are n x n
 // temporaries.
-// X = inv(M) for M in Ain, which is X or zinv_input(n, X, scr): the products
+// X = inv(M) for M in Ain, which is X or zinv_input(n, X, scr, ..): the products
 // that form M write it there, so the inverse starts without a copy.
 //
 // Safety net of the mixed mode: since I - M X1 = (I - M X0)^2 for the
@@ -138,6 +138,12 @@ struct OzSubBatch {
 bool mixed_inverse_c64() {
   const char* e = std::getenv("QX_MIXED_INVERSE");
   return e && std::string(e) == "c64";
+}
+
+// Precision of the (first) block inverse.
+int inv_precision(int prec) {
+  const bool c64 = prec == QX_PREC_C64 || (prec == QX_PREC_MIXED && mixed_inverse_c64());
+  return c64 ? QX_PREC_C64 : QX_PREC_C128;
 }
 
 void block_inv(hipStream_t st, int64_t S, int n, const Mat& Ain, const Mat& X, int* info,
@@ -214,7 +220,7 @@ void rgf_selected_inv(qx_handle* h, hipStream_t st0, const qx_btd_layout* la,
   const Btd A0(la, a), X0(lx, x);
   char* oz_region = reinterpret_cast<char*>(ws) + rgf_slot_bytes(la, false, bmax);
 
-  const int gp = gemm_precision(prec);
+  const int gp = gemm_precision(prec), ip = inv_precision(prec);
   // QX_RGF_PAIR=0 (read per call): one launch per backward product
   const char* pair_env = std::getenv("QX_RGF_PAIR");
   const bool pair_on = !(pair_env && pair_env[0] == '0');
@@ -234,7 +240,7 @@ void rgf_selected_inv(qx_handle* h, hipStream_t st0, const qx_btd_layout* la,
 
     // Forward sweep (rgf.py:70-92).
     {
-      const Mat X0 = W.get(xd[0], bs(0)), M0 = zinv_input(bs(0), X0, scr);
+      const Mat X0 = W.get(xd[0], bs(0)), M0 = zinv_input(bs(0), X0, scr, ip);
       fold(st, S, bs(0), bs(0), A.diag(0), -1.0, OR.get(0, bs(0)), M0);
       block_inv(st, S, bs(0), M0, X0, info, prec, scr, W.get(N + 6, bs(0)), W.get(N + 7, bs(0)),
                 mask);
@@ -243,7 +249,7 @@ void rgf_selected_inv(qx_handle* h, hipStream_t st0, const qx_btd_layout* la,
       const int j = i + 1, bi = bs(i), bj = bs(j);
       const Mat T1 = W.get(t1, bi);
       zgemm(st, S, bj, bi, bi, QX_OP_N, QX_OP_N, kOne, A.lower(i), W.get(xd[i], bi), kZero, T1, gp);
-      const Mat Xj = W.get(xd[j], bj), Mj = zinv_input(bj, Xj, scr);
+      const Mat Xj = W.get(xd[j], bj), Mj = zinv_input(bj, Xj, scr, ip);
       Mat Ajj = A.diag(j);
       if (!OR.get(j, bj).zero()) {
         fold(st, S, bj, bj, A.diag(j), -1.0, OR.get(j, bj), Mj);
@@ -332,7 +338,7 @@ void rgf_selected_solve(qx_handle* h, hipStream_t st0, const qx_btd_layout* la,
   const Btd A0(la, a), SL0(lsl, sl), SG0(lsg, sg), XL0(lxl, xl), XG0(lxg, xg),
       XR0(want_r ? lxr : nullptr, want_r ? xr : nullptr);
 
-  const int gp = gemm_precision(prec);
+  const int gp = gemm_precision(prec), ip = inv_precision(prec);
   // The odd sub-batches start after sub-batch 0's first block inverse, so
   // that the sub-batches' latency-bound inverse phases do not coincide and
   // the GEMMs of one fill the GPU during the inverse of another
@@ -438,7 +444,7 @@ void rgf_selected_solve(qx_handle* h, hipStream_t st0, const qx_btd_layout* la,
   // ---- block 0 (rgf.py:207-231) ----
   {
     const int b0 = bs(0);
-    const Mat X0 = W.get(sr[0], b0), M0 = zinv_input(b0, X0, scr);
+    const Mat X0 = W.get(sr[0], b0), M0 = zinv_input(b0, X0, scr, ip);
     fold(st, S, b0, b0, A.diag(0), -1.0, OR.get(0, b0), M0);
     block_inv(st, S, b0, M0, X0, info, prec, scr, W.get(NS1, b0), W.get(NS2, b0), mask);
     if (release.p) {
@@ -481,7 +487,7 @@ void rgf_selected_solve(qx_handle* h, hipStream_t st0, const qx_btd_layout* la,
     }
     // xr_jj = inv(a_jj - obc - a_ji xr_ii a_ij), the argument formed where
     // the inverse starts
-    const Mat Mj = zinv_input(bj, Xrj, scr);
+    const Mat Mj = zinv_input(bj, Xrj, scr, ip);
     Mat Ajj = A.diag(j);
     if (!OR.get(j, bj).zero()) {
       fold(st, S, bj, bj, A.diag(j), -1.0, OR.get(j, bj), Mj);

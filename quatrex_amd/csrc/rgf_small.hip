@@ -19,20 +19,15 @@
 //   dependent steps, each about a microsecond of one SIMD's matrix-core
 //   work behind a memory round trip and a barrier, so fewer steps make it
 //   shorter.
-// - Block inverse (sinv_wg): the four waves of team 0, eight lanes per row
-//   (four columns each), Gauss-Jordan with partial pivoting and one barrier
-//   per column: the pivot is a DPP wave maximum of 32-bit keys (float
-//   magnitude with the row index in the low bits, as in inv.hip) over each
-//   wave's rows, then the largest of the four published keys; the candidate
-//   rows and row k go through double-buffered LDS; the column interchanges
-//   are undone at the end.  (sinv_wave is the one-wave variant, kept for
-//   QX_INV_SMALL=1.)
+// - Block inverse (sinv): gj_invert (gj_core.h), one factoring and two update
+//   waves, the block in matrix-core registers; the other waves wait.
 // - Elementwise steps (folds, X - X^H parts, traces) as team loops whose
 //   loads are all issued before the first use.
 // - A barrier closes every step, which makes its global writes visible to
 //   the other waves of the workgroup.
 #include <cstdlib>
 
+#include "gj_core.h"
 #include "qx_internal.h"
 
 namespace qx {
@@ -77,45 +72,8 @@ __device__ inline M blk(const z2* base, int64_t stride, int64_t e, int32_t off, 
   return M{const_cast<z2*>(base) + e * stride + off, ld};
 }
 
-// Wave maximum of pivot keys (DPP), as in inv.hip.
-__device__ inline unsigned s_wave_max(unsigned v) {
-  v = max(v, (unsigned)__builtin_amdgcn_mov_dpp((int)v, 0xB1, 0xf, 0xf, false));
-  v = max(v, (unsigned)__builtin_amdgcn_mov_dpp((int)v, 0x4E, 0xf, 0xf, false));
-  v = max(v, (unsigned)__builtin_amdgcn_mov_dpp((int)v, 0x124, 0xf, 0xf, false));
-  v = max(v, (unsigned)__builtin_amdgcn_mov_dpp((int)v, 0x128, 0xf, 0xf, false));
-  const unsigned a = (unsigned)__builtin_amdgcn_readlane((int)v, 0);
-  const unsigned b = (unsigned)__builtin_amdgcn_readlane((int)v, 16);
-  const unsigned c = (unsigned)__builtin_amdgcn_readlane((int)v, 32);
-  const unsigned d = (unsigned)__builtin_amdgcn_readlane((int)v, 48);
-  return max(max(a, b), max(c, d));
-}
-
-// Value of lane QQ of each pair of lanes (DPP quad_perm [0,0,2,2] / [1,1,3,3]).
-template <int QQ>
-__device__ inline double s_pair_bcast(double x) {
-  constexpr int sel = QQ == 0 ? 0xA0 : 0xF5;
-  const int lo = __builtin_amdgcn_mov_dpp(__double2loint(x), sel, 0xf, 0xf, false);
-  const int hi = __builtin_amdgcn_mov_dpp(__double2hiint(x), sel, 0xf, 0xf, false);
-  return __hiloint2double(hi, lo);
-}
-
-// LDS of one wave's inverse.
-struct WaveShared {
-  z2 prow[kSB], krow[kSB];
-  int perm[kSB], idx[kSB];
-  z2 tile[kSB][kSB + 1];
-};
-
-struct WgInvShared {
-  z2 cand[2][kThreads / 64][kSB];
-  z2 krow[2][kSB];
-  unsigned keys[2][kThreads / 64];
-  int perm[kSB], idx[kSB];
-  z2 tile[kSB][kSB + 1];
-};
-
 struct Shared {
-  WgInvShared winv;
+  GjShared<GjWhole32> winv;
   double red[2][kSolveThreads / 64];
 };
 
@@ -350,305 +308,10 @@ __device__ __forceinline__ void strace_diff(int nt, int n, M X, M Y, M Z, M W, z
   __syncthreads();
 }
 
-// X = inv(A - S) for one n x n matrix (n <= 32; S may be null; X may
-// alias A), computed by one whole wave with no workgroup barrier.
-__device__ __forceinline__ void sinv_wave(int n, const z2* A, int lda, const z2* S, int lds, z2* X, int ldx,
-                          int* info, WaveShared& sh) {
-  {
-    const int lane = threadIdx.x & 63, r = lane >> 1, h = lane & 1;
-    double xr[16], xi[16];
-#pragma unroll
-    for (int c = 0; c < 16; ++c) {
-      const int col = 16 * h + c;
-      z2 v = make_double2(0.0, 0.0);
-      if (r < n && col < n) {
-        v = A[r * lda + col];
-        if (S) {
-          const z2 u = S[r * lds + col];
-          v.x -= u.x;
-          v.y -= u.y;
-        }
-      }
-      xr[c] = v.x;
-      xi[c] = v.y;
-    }
-#pragma unroll
-    for (int k = 0; k < kSB; ++k) {
-      if (k < n) {
-        const int hk = k >> 4, ck = k & 15;
-        unsigned key = 0;
-        if (h == hk && r >= k && r < n) key = pivot_key(xr[ck], xi[ck], r);
-        const unsigned kmax = s_wave_max(key);
-        int p = 511 - (int)(kmax & 0x1FFu);
-        if (p < k || p >= n) p = k;
-        if (lane == 0) {
-          sh.perm[k] = p;
-          if ((kmax >> 9) == 0u) *info = 1;  // no nonzero pivot: singular
-        }
-        // publish the pivot row and row k (one wave: LDS keeps program order)
-        if (r == p) {
-#pragma unroll
-          for (int c = 0; c < 16; ++c) sh.prow[16 * h + c] = make_double2(xr[c], xi[c]);
-        }
-        if (r == k) {
-#pragma unroll
-          for (int c = 0; c < 16; ++c) sh.krow[16 * h + c] = make_double2(xr[c], xi[c]);
-        }
-        __builtin_amdgcn_wave_barrier();
-        const z2 x = sh.prow[k];
-        double vr, vi;
-        complex_recip(x.x, x.y, vr, vi);
-        double pr[16], pi[16];  // this lane's half of the scaled pivot row
-#pragma unroll
-        for (int c = 0; c < 16; ++c) {
-          const int col = 16 * h + c;
-          if (col == k) {
-            pr[c] = vr;
-            pi[c] = vi;
-          } else {
-            const z2 v = sh.prow[col];
-            pr[c] = v.x * vr - v.y * vi;
-            pi[c] = v.x * vi + v.y * vr;
-          }
-        }
-        if (r == k) {
-#pragma unroll
-          for (int c = 0; c < 16; ++c) {
-            xr[c] = pr[c];
-            xi[c] = pi[c];
-          }
-        } else if (r == p) {
-#pragma unroll
-          for (int c = 0; c < 16; ++c) {
-            const z2 v = sh.krow[16 * h + c];
-            xr[c] = v.x;
-            xi[c] = v.y;
-          }
-        }
-        // multiplier: the row's (swapped-in) value in column k
-        const double fr = hk == 0 ? s_pair_bcast<0>(xr[ck]) : s_pair_bcast<1>(xr[ck]);
-        const double fi = hk == 0 ? s_pair_bcast<0>(xi[ck]) : s_pair_bcast<1>(xi[ck]);
-        if (r != k && r < n) {
-#pragma unroll
-          for (int c = 0; c < 16; ++c) {
-            const int col = 16 * h + c;
-            if (col == k) {
-              xr[c] = -(fr * pr[c] - fi * pi[c]);
-              xi[c] = -(fr * pi[c] + fi * pr[c]);
-            } else {
-              xr[c] -= fr * pr[c] - fi * pi[c];
-              xi[c] -= fr * pi[c] + fi * pr[c];
-            }
-          }
-        }
-        __builtin_amdgcn_wave_barrier();
-      }
-    }
-    // undo the column interchanges: reverse order of the pivots
-    if (lane == 0) {
-      for (int c = 0; c < n; ++c) sh.idx[c] = c;
-      for (int k = n - 1; k >= 0; --k) {
-        const int pq = sh.perm[k];
-        const int t = sh.idx[k];
-        sh.idx[k] = sh.idx[pq];
-        sh.idx[pq] = t;
-      }
-    }
-#pragma unroll
-    for (int c = 0; c < 16; ++c) {
-      const int col = 16 * h + c;
-      if (r < n && col < n) sh.tile[r][col] = make_double2(xr[c], xi[c]);
-    }
-    __builtin_amdgcn_wave_barrier();
-#pragma unroll
-    for (int c = 0; c < 16; ++c) {
-      const int col = 16 * h + c;
-      if (r < n && col < n) X[r * ldx + col] = sh.tile[r][sh.idx[col]];
-    }
-  }
-}
-
-// X = inv(A - S) for one n x n matrix (n <= 32) by the first four waves of
-// the workgroup (eight lanes per row, four columns per lane; further waves
-// hold no row): Gauss-Jordan with partial pivoting and one barrier per
-// column.  Before the barrier each wave publishes its best candidate row
-// (DPP maximum of the pivot keys over its eight rows) and the lanes of row k
-// publish row k; after it every thread takes the largest of the four keys,
-// reads the pivot row and computes the reciprocal itself (one wave per SIMD,
-// so nothing is serialised).  The buffers alternate between columns: no
-// wave can write a buffer before every wave has passed the barrier that
-// follows its last read.
-
-
-__device__ __forceinline__ void sinv_wg(int n, const z2* A, int lda, const z2* S, int lds,
-                                        z2* X, int ldx, int* info, WgInvShared& sh) {
-  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
-  const int r = tid >> 3, q = tid & 7;  // row, quarter-of-eight within the row
-  double xr[4], xi[4];
-  {
-    // all loads in flight together (clamped addresses, no branch between them)
-    z2 va[4], vs[4];
-#pragma unroll
-    for (int c = 0; c < 4; ++c) {
-      const int col = 4 * q + c;
-      const bool ok = r < n && col < n;
-      va[c] = A[ok ? r * lda + col : 0];
-      vs[c] = S ? S[ok ? r * lds + col : 0] : make_double2(0.0, 0.0);
-    }
-#pragma unroll
-    for (int c = 0; c < 4; ++c) {
-      const bool ok = r < n && 4 * q + c < n;
-      xr[c] = ok ? va[c].x - vs[c].x : 0.0;
-      xi[c] = ok ? va[c].y - vs[c].y : 0.0;
-    }
-  }
-  // Groups of four columns run as a loop, the four columns of a group are
-  // unrolled (register indices stay constants): the fully unrolled 32
-  // columns are ~64 KB of code per call site, beyond the instruction cache.
-#pragma unroll 1
-  for (int kq = 0; kq < kSB / 4; ++kq) {
-#pragma unroll
-    for (int kc = 0; kc < 4; ++kc) {
-      const int k = 4 * kq + kc, b = kc & 1;
-      if (k < n) {
-        unsigned key = 0;
-        if (q == kq && r >= k && r < n) key = pivot_key(xr[kc], xi[kc], r);
-        const unsigned wkey = s_wave_max(key);
-        if (wkey != 0u && r == 511 - (int)(wkey & 0x1FFu)) {
-#pragma unroll
-          for (int c = 0; c < 4; ++c) sh.cand[b][w][4 * q + c] = make_double2(xr[c], xi[c]);
-        }
-        if (lane == 0 && w < kThreads / 64) sh.keys[b][w] = wkey;  // waves 4..7 hold no row
-        if (r == k) {
-#pragma unroll
-          for (int c = 0; c < 4; ++c) sh.krow[b][4 * q + c] = make_double2(xr[c], xi[c]);
-        }
-        __syncthreads();
-        unsigned kmax = sh.keys[b][0];
-        int ws = 0;
-#pragma unroll
-        for (int u = 1; u < kThreads / 64; ++u) {
-          const unsigned v = sh.keys[b][u];
-          if (v > kmax) {
-            kmax = v;
-            ws = u;
-          }
-        }
-        int p = 511 - (int)(kmax & 0x1FFu);
-        if (p < k || p >= n) p = k;
-        if (tid == 0) {
-          sh.perm[k] = p;
-          if ((kmax >> 9) == 0u) *info = 1;  // no nonzero pivot: singular
-        }
-        const z2 x = sh.cand[b][ws][k];
-        double vr, vi;
-        complex_recip(x.x, x.y, vr, vi);
-        double pr[4], pi[4];
-#pragma unroll
-        for (int c = 0; c < 4; ++c) {
-          const int col = 4 * q + c;
-          if (col == k) {
-            pr[c] = vr;
-            pi[c] = vi;
-          } else {
-            const z2 v = sh.cand[b][ws][col];
-            pr[c] = v.x * vr - v.y * vi;
-            pi[c] = v.x * vi + v.y * vr;
-          }
-        }
-        if (r == k) {
-#pragma unroll
-          for (int c = 0; c < 4; ++c) {
-            xr[c] = pr[c];
-            xi[c] = pi[c];
-          }
-        } else if (r == p) {
-#pragma unroll
-          for (int c = 0; c < 4; ++c) {
-            const z2 v = sh.krow[b][4 * q + c];
-            xr[c] = v.x;
-            xi[c] = v.y;
-          }
-        }
-        // multiplier: the row's (swapped-in) value in column k, from the lane
-        // of this row that holds column k
-        const int src = (lane & ~7) + kq;
-        const double fr = __shfl(xr[kc], src, 64), fi = __shfl(xi[kc], src, 64);
-        if (r < n && r != k) {
-#pragma unroll
-          for (int c = 0; c < 4; ++c) {
-            const int col = 4 * q + c;
-            if (col == k) {
-              xr[c] = -(fr * pr[c] - fi * pi[c]);
-              xi[c] = -(fr * pi[c] + fi * pr[c]);
-            } else {
-              xr[c] -= fr * pr[c] - fi * pi[c];
-              xi[c] -= fr * pi[c] + fi * pr[c];
-            }
-          }
-        }
-      }
-    }
-  }
-#pragma unroll
-  for (int c = 0; c < 4; ++c) {
-    const int col = 4 * q + c;
-    if (r < n && col < n) sh.tile[r][col] = make_double2(xr[c], xi[c]);
-  }
-  __syncthreads();  // tile, and the pivot record written by thread 0
-  // Undo the column interchanges (the identity after the swaps (k, perm k)
-  // for k = n - 1 down to 0): position c is traced forward through the
-  // swaps for k = 0 .. n - 1, one position per thread.
-  if (tid < n) {
-    int pos = tid;
-#pragma unroll 8
-    for (int k = 0; k < n; ++k) {
-      const int p = sh.perm[k];
-      pos = (pos == k) ? p : ((pos == p) ? k : pos);
-    }
-    sh.idx[tid] = pos;
-  }
-  __syncthreads();
-#pragma unroll
-  for (int c = 0; c < 4; ++c) {
-    const int col = 4 * q + c;
-    if (r < n && col < n) X[r * ldx + col] = sh.tile[r][sh.idx[col]];
-  }
-  __syncthreads();
-}
-
-
-
 // In-place inverse of the block X by the workgroup.
 __device__ __forceinline__ void sinv(int n, M X, int* info, Shared& sh) {
-  sinv_wg(n, X.p, X.ld, nullptr, 0, X.p, X.ld, info, sh.winv);
-}
-
-// Batched X_e = inv(A_e - S_e), n <= 32: one matrix per workgroup.
-__global__ __launch_bounds__(kThreads) void inv_small_wg_kernel(int n, const z2* A, int64_t sA,
-                                                                int lda, const z2* S, int64_t sS,
-                                                                int lds, z2* X, int64_t sX,
-                                                                int ldx, int* info,
-                                                                const int* mask) {
-  __shared__ WgInvShared sh;
-  const int64_t e = blockIdx.x;
-  if (mask && !mask[e]) return;  // uniform over the workgroup
-  sinv_wg(n, A + e * sA, lda, S ? S + e * sS : nullptr, lds, X + e * sX, ldx, info + e, sh);
-}
-
-// Batched X_e = inv(A_e - S_e), n <= 32: one matrix per wave, four per
-// workgroup (the whole-wave condition e < batch is uniform per wave).
-__global__ __launch_bounds__(kThreads) void inv_small_kernel(int64_t batch, int n, const z2* A,
-                                                             int64_t sA, int lda, const z2* S,
-                                                             int64_t sS, int lds, z2* X,
-                                                             int64_t sX, int ldx, int* info,
-                                                             const int* mask) {
-  __shared__ WaveShared sh[kThreads / 64];
-  const int w = threadIdx.x >> 6;
-  const int64_t e = (int64_t)blockIdx.x * (kThreads / 64) + w;
-  if (e < batch && !(mask && !mask[e]))
-    sinv_wave(n, A + e * sA, lda, S ? S + e * sS : nullptr, lds, X + e * sX, ldx, info + e,
-              sh[w]);
+  gj_invert<GjWhole32>(n, X.p, X.ld, nullptr, 0, X.p, X.ld, info, sh.winv);
+  __syncthreads();  // the inverse is visible to the workgroup
 }
 
 const Cplx kOneS{1.0, 0.0}, kMinusS{-1.0, 0.0}, kZeroS{0.0, 0.0};
@@ -1024,33 +687,6 @@ bool fits32(const qx_btd_layout* l, int N) {
 }
 
 }  // namespace
-
-// Batched inverse X = inv(A - S) of blocks n <= 32 in one launch (complex128
-// arithmetic), one matrix per workgroup: measured at n = 32 it beats both the
-// split panel kernels and one matrix per wave from 16 to 4096 matrices (37 vs
-// 49 / 69 us at 256, 207 vs 623 / 296 us at 4096).  QX_INV_SMALL=0 sends every
-// size to the split panel kernels, 1 to the per-wave kernel.
-bool inv_small(hipStream_t st, int64_t batch, int n, const Mat& A, const Mat& S, const Mat& X,
-               int* info, const int* mask) {
-  const char* env = std::getenv("QX_INV_SMALL");
-  const int mode = env ? std::atoi(env) : -1;
-  if (mode == 0) return false;
-  if (n < 1 || n > kSB) return false;
-  if (batch <= 0) return true;
-  QX_REQUIRE(batch < (int64_t(1) << 31), "inv: batch too large");
-  const bool per_wave = mode == 1;
-  if (per_wave) {
-    const int64_t blocks = (batch + kThreads / 64 - 1) / (kThreads / 64);
-    hipLaunchKernelGGL(inv_small_kernel, dim3((unsigned)blocks), dim3(kThreads), 0, st, batch,
-                       n, A.p, A.stride, A.ld, S.p, S.stride, S.ld, X.p, X.stride, X.ld, info,
-                       mask);
-  } else {
-    hipLaunchKernelGGL(inv_small_wg_kernel, dim3((unsigned)batch), dim3(kThreads), 0, st, n,
-                       A.p, A.stride, A.ld, S.p, S.stride, S.ld, X.p, X.stride, X.ld, info, mask);
-  }
-  QX_HIP_CHECK(hipGetLastError());
-  return true;
-}
 
 // Fused path of rgf_selected_solve for small blocks; returns false (and does
 // nothing) when the call is not eligible: complex128 arithmetic (4M or 3M),

@@ -364,3 +364,52 @@ def test_singular_block_raises(device):
     # the error flag is cleared after it was reported
     A[1] = torch.eye(8, dtype=A.dtype, device=device)
     _inv(device, A, X, 0)
+
+
+@pytest.mark.parametrize("n", [1, 7, 8, 9, 16, 17, 31, 32, 33, 40, 63, 64, 65, 95, 96, 97, 127, 128])
+@pytest.mark.parametrize("in_place", [False, True])
+def test_whole_inverse_edges(device, n, in_place):
+    """n <= 128: one workgroup per matrix with the matrix in registers, at the
+    edges of its shapes (32, 64, 96, 128), tiles (16) and sub-panels (8), with
+    a subtracted matrix and leading dimensions above n, against NumPy and (to
+    rounding, same pivot rule) against the split panel kernels.  Columns past
+    n are left alone."""
+    rng = np.random.default_rng(13 * n)
+    batch, ld = 3, n + 3
+    a = _cplx(rng, (batch, n, ld))
+    s = 0.1 * _cplx(rng, (batch, n, n))
+    a[:, 0, 0] = s[:, 0, 0] if n > 1 else a[:, 0, 0]  # a zero first pivot candidate
+    from quatrex_amd import _lib as ql
+
+    lib, h = ql.load(), ql.handle(device)
+    S = torch.as_tensor(s, device=device)
+    outs = {}
+    for whole in ("128", "0"):
+        with pytest.MonkeyPatch.context() as mp:
+            mp.setenv("QX_INV_WHOLE", whole)
+            A = torch.as_tensor(a, device=device).clone()
+            X = A if in_place else torch.full_like(A, 7.0)
+            rc = lib.qx_inv_batched(h, ql.stream_ptr(device), batch, n, A.data_ptr(), ld, n * ld,
+                                    S.data_ptr(), n, n * n, X.data_ptr(), ld, n * ld, 0)
+            ql.check(rc, h, "inv")
+            ql.sync_check(device, "inv")
+            outs[whole] = X.cpu().numpy()
+    pad = a[:, :, n:] if in_place else 7.0
+    for e in range(batch):
+        m = a[e, :, :n] - s[e]
+        tol = 1e-15 * np.linalg.cond(m) * max(n, 4)
+        assert rel_err(outs["128"][e, :, :n], np.linalg.inv(m)) < tol
+        assert rel_err(outs["128"][e, :, :n], outs["0"][e, :, :n]) < 2 * tol
+    assert np.array_equal(outs["128"][:, :, n:], np.broadcast_to(pad, outs["128"][:, :, n:].shape))
+
+
+@pytest.mark.parametrize("n", [20, 48, 80, 128])
+def test_whole_inverse_singular_raises(device, n):
+    a = np.zeros((2, n, n), complex)
+    a[0] = np.eye(n)
+    a[1, :, : n // 2] = 1.0  # rank 1
+    A = torch.as_tensor(a, device=device)
+    X = torch.empty_like(A)
+    with pytest.raises(np.linalg.LinAlgError):
+        _inv(device, A, X, 0)
+    assert np.array_equal(X[0].cpu().numpy(), np.eye(n))
