@@ -71,6 +71,12 @@ extern "C" {
 #define QX_SOLVE_RETARDED_OFFDIAG 4u /* also write off-diagonal G^R blocks     */
 #define QX_SOLVE_SKIP_LOWER_L 8u     /* lesser output is symmetric-stored      */
 #define QX_SOLVE_SKIP_LOWER_G 16u    /* greater output is symmetric-stored     */
+/* The call may wait for the device once: it checks whether every diagonal
+ * S^{<>} block and lesser / greater boundary block is skew-Hermitian (to 64
+ * eps of its largest entry) and, if so, runs the backward sweep with three
+ * products per quantity and block instead of four (complex128 arithmetic; same
+ * results to rounding).  Ignored while the stream records a graph. */
+#define QX_SOLVE_SKEW_CHECK 32u
 
 typedef struct qx_handle qx_handle;
 

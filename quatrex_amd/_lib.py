@@ -66,6 +66,7 @@ SOLVE_CURRENT = 2
 SOLVE_RETARDED_OFFDIAG = 4
 SOLVE_SKIP_LOWER_L = 8
 SOLVE_SKIP_LOWER_G = 16
+SOLVE_SKEW_CHECK = 32
 
 EXPORTED_SYMBOLS = (
     "qx_abi_version", "qx_create", "qx_destroy", "qx_last_error", "qx_workspace_query",

@@ -272,6 +272,21 @@ int* qx_handle::ensure_info(size_t n) {
   return info;
 }
 
+void qx_handle::ensure_skew() {
+  if (skew_dev) return;
+  while (skew_ev.size() < kMaxParts) {
+    hipEvent_t ev;
+    QX_HIP_CHECK(hipEventCreateWithFlags(&ev, hipEventDisableTiming));
+    skew_ev.push_back(ev);
+  }
+  if (!skew_host && hipHostMalloc(&skew_host, kMaxParts * sizeof(int)) != hipSuccess)
+    throw qx::Error{QX_ENOMEM, "skew flag allocation failed"};
+  if (hipMalloc(&skew_dev, kMaxParts * sizeof(int)) != hipSuccess) {
+    skew_dev = nullptr;
+    throw qx::Error{QX_ENOMEM, "skew flag allocation failed"};
+  }
+}
+
 int* qx_handle::ensure_mask(size_t n) {
   if (n > mask_len) {
     const size_t len = std::max<size_t>(n, 1024);
@@ -341,7 +356,7 @@ int qx_create(qx_handle** handle, int device) {
   h->device = device;
   if (const char* env = std::getenv("QX_RGF_STREAMS")) {
     const int p = std::atoi(env);
-    if (p >= 1 && p <= 8) h->parts = p;
+    if (p >= 1 && p <= qx_handle::kMaxParts) h->parts = p;
   }
   *handle = h;
   return QX_OK;
@@ -410,6 +425,9 @@ int qx_destroy(qx_handle* h) {
   if (h->ws) (void)hipFree(h->ws);
   if (h->info) (void)hipFree(h->info);
   if (h->mask) (void)hipFree(h->mask);
+  if (h->skew_dev) (void)hipFree(h->skew_dev);
+  if (h->skew_host) (void)hipHostFree(h->skew_host);
+  for (hipEvent_t ev : h->skew_ev) (void)hipEventDestroy(ev);
   delete h;
   return QX_OK;
 }
@@ -612,7 +630,8 @@ int qx_assemble_system_matrix(qx_handle* h, void* stream, int64_t n_stack, int64
 int qx_set_tuning(qx_handle* h, int streams, int gemm_tile) {
   return guarded(h, [&]() {
     QX_REQUIRE(h, "null handle");
-    QX_REQUIRE(streams >= 1 && streams <= 8, "set_tuning: streams must be in [1, 8]");
+    QX_REQUIRE(streams >= 1 && streams <= qx_handle::kMaxParts,
+               "set_tuning: streams must be in [1, 8]");
     QX_REQUIRE(gemm_tile == QX_GEMM_AUTO || gemm_tile == QX_GEMM_REG_64x64 ||
                    gemm_tile == QX_GEMM_REG_64x128 || gemm_tile == QX_GEMM_REG_128x64 ||
                    gemm_tile == QX_GEMM_LDS_64 || gemm_tile == QX_GEMM_LDS_128,

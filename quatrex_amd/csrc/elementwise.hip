@@ -5,6 +5,9 @@
 // transposed reads are coalesced.  Reductions (traces, norms) use one
 // workgroup per matrix and a fixed summation order, so results do not
 // depend on how many matrices share a launch.
+#include <algorithm>
+#include <cmath>
+
 #include "qx_internal.h"
 
 namespace qx {
@@ -184,6 +187,158 @@ void herm(hipStream_t s, int64_t batch, int m, int n, double cy, double ca,
   QX_REQUIRE(blocks < (int64_t(1) << 31), "herm: grid too large");
   hipLaunchKernelGGL(herm_kernel, dim3((unsigned)blocks), dim3(NT), 0, s, g);
   QX_HIP_CHECK(hipGetLastError());
+}
+
+// Tile pair t of the upper triangle of tn x tn tiles: (rt, ct), rt <= ct.
+__device__ inline void tile_pair(int t, int tn, int& rt, int& ct) {
+  rt = 0;
+  while (t >= tn - rt) {
+    t -= tn - rt;
+    ++rt;
+  }
+  ct = rt + t;
+}
+
+// Y = (X - X^H) / 2 + (P - P^H) = W - W^H with W = X / 2 + P, on the tile pair
+// (rt, ct), (ct, rt): every element is read once, and Y is skew-Hermitian to
+// the bit.  Streaming: 48 n^2 bytes per matrix (the projection kernel it
+// replaces moved 32 n^2 and read each X twice).
+struct SkewArgs {
+  int n, tn;
+  int64_t half;  // matrices per group
+  const z2 *X[2], *P[2];
+  z2* Y[2];
+  int64_t sX[2], sP[2], sY[2];
+  int lx[2], lp[2], ly[2];
+  double* dens;  // Im diag of group 0's Y, or null
+  int64_t sd;
+};
+
+__global__ __launch_bounds__(NT) void skew_update_kernel(SkewArgs g) {
+  __shared__ z2 wa[TS][TS + 1], wb[TS][TS + 1];
+  const int pairs = g.tn * (g.tn + 1) / 2;
+  const int id = tile_xcd_remap(blockIdx.x, gridDim.x);
+  const int64_t eg = id / pairs;
+  int rt, ct;
+  tile_pair(id - (int)(eg * pairs), g.tn, rt, ct);
+  const int grp = eg >= g.half ? 1 : 0;
+  const int64_t e = eg - grp * g.half;
+  const z2* X = grp ? g.X[1] + e * g.sX[1] : g.X[0] + e * g.sX[0];
+  const z2* P = grp ? g.P[1] + e * g.sP[1] : g.P[0] + e * g.sP[0];
+  z2* Y = grp ? g.Y[1] + e * g.sY[1] : g.Y[0] + e * g.sY[0];
+  const int lx = grp ? g.lx[1] : g.lx[0], lp = grp ? g.lp[1] : g.lp[0],
+            ly = grp ? g.ly[1] : g.ly[0];
+  const int n = g.n, r0 = rt * TS, c0 = ct * TS;
+  const int tx = threadIdx.x & 31, ty = threadIdx.x >> 5;  // 32 x 8
+  z2 xa[4], pa[4], xb[4], pb[4];
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {
+    // all loads in flight together, from addresses clamped into the block
+    const int i = ty + 8 * k;
+    const int ra = min(r0 + i, n - 1), ca = min(c0 + tx, n - 1);
+    const int rb = min(c0 + i, n - 1), cb = min(r0 + tx, n - 1);
+    xa[k] = X[(int64_t)ra * lx + ca];
+    pa[k] = P[(int64_t)ra * lp + ca];
+    xb[k] = X[(int64_t)rb * lx + cb];
+    pb[k] = P[(int64_t)rb * lp + cb];
+  }
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {
+    const int i = ty + 8 * k;
+    wa[i][tx] = make_double2(fma(0.5, xa[k].x, pa[k].x), fma(0.5, xa[k].y, pa[k].y));
+    wb[i][tx] = make_double2(fma(0.5, xb[k].x, pb[k].x), fma(0.5, xb[k].y, pb[k].y));
+  }
+  __syncthreads();
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {
+    const int i = ty + 8 * k;
+    {
+      const int r = r0 + i, c = c0 + tx;
+      if (r < n && c < n) {
+        const z2 u = wa[i][tx], v = wb[tx][i];
+        const z2 y = make_double2(u.x - v.x, u.y + v.y);
+        Y[(int64_t)r * ly + c] = y;
+        if (g.dens && grp == 0 && r == c) g.dens[e * g.sd + r] = y.y;
+      }
+    }
+    if (rt != ct) {
+      const int r = c0 + i, c = r0 + tx;
+      if (r < n && c < n) {
+        const z2 u = wb[i][tx], v = wa[tx][i];
+        Y[(int64_t)r * ly + c] = make_double2(u.x - v.x, u.y + v.y);
+      }
+    }
+  }
+}
+
+// Largest |s| and largest |s_rc + conj s_cr| (|re| + |im|) of one matrix of one
+// block per workgroup; the flag is raised if the second exceeds 64 eps of the
+// first, or if anything is not finite.
+constexpr int kSkewBlocks = 64;  // blocks per launch
+struct SkewCheckArgs {
+  int blocks;
+  const z2* p[kSkewBlocks];
+  int64_t stride[kSkewBlocks];
+  int n[kSkewBlocks];
+  int* flag;
+};
+
+__global__ __launch_bounds__(NT) void skew_check_kernel(SkewCheckArgs g) {
+  __shared__ z2 tile[TS][TS + 1];
+  __shared__ double red[2][NT / 64];
+  const int blk = blockIdx.x % g.blocks;
+  const int64_t e = blockIdx.x / g.blocks;
+  if (e > 0 && g.stride[blk] == 0) return;  // one matrix for the whole stack
+  const z2* S = g.p[blk] + e * g.stride[blk];
+  const int n = g.n[blk], tn = (n + TS - 1) / TS;
+  const int tx = threadIdx.x & 31, ty = threadIdx.x >> 5;  // 32 x 8
+  double m = 0.0, d = 0.0;
+  bool bad = false;
+  for (int rt = 0; rt < tn; ++rt)
+    for (int ct = rt; ct < tn; ++ct) {
+      const int r0 = rt * TS, c0 = ct * TS;
+      z2 a[4];
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        const int i = ty + 8 * k;
+        const int ra = min(r0 + i, n - 1), ca = min(c0 + tx, n - 1);
+        const int rb = min(c0 + i, n - 1), cb = min(r0 + tx, n - 1);
+        a[k] = S[(int64_t)ra * n + ca];
+        tile[i][tx] = S[(int64_t)rb * n + cb];
+      }
+      __syncthreads();
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        const int i = ty + 8 * k;
+        if (r0 + i < n && c0 + tx < n) {
+          const z2 b = tile[tx][i];  // S[c0 + tx][r0 + i]
+          const double ma = fabs(a[k].x) + fabs(a[k].y), mb = fabs(b.x) + fabs(b.y);
+          const double df = fabs(a[k].x + b.x) + fabs(a[k].y - b.y);
+          bad = bad || !(ma < INFINITY) || !(mb < INFINITY);
+          m = fmax(m, fmax(ma, mb));
+          d = fmax(d, df);
+        }
+      }
+      __syncthreads();
+    }
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) {
+    m = fmax(m, __shfl_xor(m, off, 64));
+    d = fmax(d, __shfl_xor(d, off, 64));
+  }
+  const int w = threadIdx.x >> 6;
+  if ((threadIdx.x & 63) == 0) {
+    red[0][w] = m;
+    red[1][w] = d;
+  }
+  __syncthreads();
+  for (int u = 0; u < NT / 64; ++u) {
+    m = fmax(m, red[0][u]);
+    d = fmax(d, red[1][u]);
+  }
+  // 2^-46 = 64 eps: above the rounding of a product C C^H, below the error the
+  // recursion itself makes
+  if (bad || !(d <= 0x1p-46 * m)) *g.flag = 1;
 }
 
 // Contact self-energies from Sigma^R (one 32 x 32 tile per workgroup, the
@@ -427,6 +582,8 @@ __global__ __launch_bounds__(NT) void contour_acc_kernel(AccArgs g, int64_t tota
   }
 }
 
+__global__ void clear_flag_kernel(int* flag) { *flag = 0; }
+
 unsigned grid_for(int64_t total) {
   int64_t b = (total + NT - 1) / NT;
   if (b > 65536 * 4) b = 65536 * 4;
@@ -509,6 +666,47 @@ void ew_antiherm_pair(hipStream_t s, int64_t batch, int n, double scale, const M
     return;
   }
   herm(s, batch, n, n, 0.0, scale, X0, -scale, X0, Y0, 0.0, Mat(), &X1, &X1, &Y1);
+}
+
+void ew_skew_update(hipStream_t s, int64_t batch, int n, const Mat& X0, const Mat& P0,
+                    const Mat& Y0, const Mat* X1, const Mat* P1, const Mat* Y1, double* dens,
+                    int64_t dens_stride) {
+  if (batch <= 0 || n <= 0) return;
+  const bool two = Y1 != nullptr;
+  QX_REQUIRE(!X0.zero() && !P0.zero() && !Y0.zero(), "skew_update: null operand");
+  QX_REQUIRE(!two || (X1 && P1 && !X1->zero() && !P1->zero() && !Y1->zero()),
+             "skew_update: a two-group launch needs all operands");
+  const Mat &x1 = two ? *X1 : X0, &p1 = two ? *P1 : P0, &y1 = two ? *Y1 : Y0;
+  for (const Mat* y : {&Y0, &y1})
+    QX_REQUIRE(y->p != X0.p && y->p != P0.p && y->p != x1.p && y->p != p1.p,
+               "skew_update: the output aliases an operand");
+  const int tn = (n + TS - 1) / TS;
+  SkewArgs g{n, tn, batch, {X0.p, x1.p}, {P0.p, p1.p}, {Y0.p, y1.p},
+             {X0.stride, x1.stride}, {P0.stride, p1.stride}, {Y0.stride, y1.stride},
+             {X0.ld, x1.ld}, {P0.ld, p1.ld}, {Y0.ld, y1.ld}, dens, dens_stride};
+  const int64_t blocks = (two ? 2 : 1) * batch * (tn * (tn + 1) / 2);
+  QX_REQUIRE(blocks < (int64_t(1) << 31), "skew_update: grid too large");
+  hipLaunchKernelGGL(skew_update_kernel, dim3((unsigned)blocks), dim3(NT), 0, s, g);
+  QX_HIP_CHECK(hipGetLastError());
+}
+
+void skew_check(hipStream_t s, int64_t batch, const std::vector<SkewBlock>& blocks, int* flag) {
+  hipLaunchKernelGGL(clear_flag_kernel, dim3(1), dim3(1), 0, s, flag);
+  if (batch <= 0) return;
+  for (size_t b0 = 0; b0 < blocks.size(); b0 += kSkewBlocks) {
+    SkewCheckArgs g;
+    g.blocks = (int)std::min<size_t>(kSkewBlocks, blocks.size() - b0);
+    for (int k = 0; k < g.blocks; ++k) {
+      g.p[k] = blocks[b0 + k].p;
+      g.stride[k] = blocks[b0 + k].stride;
+      g.n[k] = blocks[b0 + k].n;
+    }
+    g.flag = flag;
+    const int64_t wgs = batch * g.blocks;
+    QX_REQUIRE(wgs < (int64_t(1) << 31), "skew_check: grid too large");
+    hipLaunchKernelGGL(skew_check_kernel, dim3((unsigned)wgs), dim3(NT), 0, s, g);
+    QX_HIP_CHECK(hipGetLastError());
+  }
 }
 
 void ew_herm_add(hipStream_t s, int64_t batch, int n, const Mat& D, double scale,

@@ -75,27 +75,31 @@ struct GemmArgs {
   const z2* E;
   int64_t sE;
   int lde;
+  // optional: third output Y = Cin + op(A) op(B) / 2 (C may then be null)
+  z2* Y;
+  int64_t sY;
+  int ldy;
   // Up to three products of one shape in one launch: matrices half <= e <
   // 2 half take every operand from the second set (base, matrix stride,
   // leading dimension) at index e - half, matrices e >= 2 half from the
   // third at e - 2 half.  Sets a launch does not use equal the first.
   int64_t half;
   const z2 *A2, *B2, *Cin2, *E2;
-  z2 *C2, *Ct2;
-  int64_t sA2, sB2, sC2, sCin2, sCt2, sE2;
-  int lda2, ldb2, ldc2, ldcin2, ldct2, lde2;
+  z2 *C2, *Ct2, *Y2;
+  int64_t sA2, sB2, sC2, sCin2, sCt2, sE2, sY2;
+  int lda2, ldb2, ldc2, ldcin2, ldct2, lde2, ldy2;
   const z2 *A3, *B3, *Cin3, *E3;
-  z2 *C3, *Ct3;
-  int64_t sA3, sB3, sC3, sCin3, sCt3, sE3;
-  int lda3, ldb3, ldc3, ldcin3, ldct3, lde3;
+  z2 *C3, *Ct3, *Y3;
+  int64_t sA3, sB3, sC3, sCin3, sCt3, sE3, sY3;
+  int lda3, ldb3, ldc3, ldcin3, ldct3, lde3, ldy3;
 };
 
 // Operands of matrix e of a launch (see GemmArgs::half); uniform over a
 // workgroup.
 struct GemmPtrs {
   const z2 *A, *B, *Cin, *E;
-  z2 *C, *Ct;
-  int lda, ldb, ldc, ldcin, ldct, lde;
+  z2 *C, *Ct, *Y;
+  int lda, ldb, ldc, ldcin, ldct, lde, ldy;
 };
 __device__ __forceinline__ GemmPtrs gemm_ptrs(const GemmArgs& g, int64_t e) {
   const int grp = e >= 2 * g.half ? 2 : (e >= g.half ? 1 : 0);
@@ -105,8 +109,12 @@ __device__ __forceinline__ GemmPtrs gemm_ptrs(const GemmArgs& g, int64_t e) {
   GemmPtrs p;
   p.A = QX_SEL(g.A + l * g.sA, g.A2 + l * g.sA2, g.A3 + l * g.sA3);
   p.B = QX_SEL(g.B + l * g.sB, g.B2 + l * g.sB2, g.B3 + l * g.sB3);
-  p.C = QX_SEL(g.C + l * g.sC, g.C2 + l * g.sC2, g.C3 + l * g.sC3);
-  p.Cin = QX_SEL(g.Cin + l * g.sCin, g.Cin2 + l * g.sCin2, g.Cin3 + l * g.sCin3);
+  p.C = g.C ? QX_SEL(g.C + l * g.sC, g.C2 + l * g.sC2, g.C3 + l * g.sC3) : nullptr;
+  // a group without a beta term has a null Cin of its own
+  const z2* ci = QX_SEL(g.Cin, g.Cin2, g.Cin3);
+  p.Cin = ci ? ci + l * QX_SEL(g.sCin, g.sCin2, g.sCin3) : nullptr;
+  p.Y = g.Y ? QX_SEL(g.Y + l * g.sY, g.Y2 + l * g.sY2, g.Y3 + l * g.sY3) : nullptr;
+  p.ldy = QX_SEL(g.ldy, g.ldy2, g.ldy3);
   p.E = g.E ? QX_SEL(g.E + l * g.sE, g.E2 + l * g.sE2, g.E3 + l * g.sE3) : nullptr;
   p.Ct = g.Ct ? QX_SEL(g.Ct + l * g.sCt, g.Ct2 + l * g.sCt2, g.Ct3 + l * g.sCt3) : nullptr;
   p.lda = QX_SEL(g.lda, g.lda2, g.lda3);
@@ -337,13 +345,14 @@ void zgemm_kernel(GemmArgs g) {
           }
           // explicit fma: the same rounding whatever the compiler contracts
           double outr = fma(g.ar, vr, -(g.ai * vi)), outi = fma(g.ar, vi, g.ai * vr);
-          z2* dst = C + (int64_t)row * P.ldc + col;
-          if (!g.beta_zero) {
+          if (!g.beta_zero && P.Cin) {
             const z2 c = beta_source(P, row, col);
             outr += fma(g.br, c.x, -(g.bi * c.y));
             outi += fma(g.br, c.y, g.bi * c.x);
+            if (P.Y)
+              P.Y[(int64_t)row * P.ldy + col] = make_double2(fma(0.5, vr, c.x), fma(0.5, vi, c.y));
           }
-          *dst = make_double2(outr, outi);
+          if (C) C[(int64_t)row * P.ldc + col] = make_double2(outr, outi);
           if (P.Ct) P.Ct[(int64_t)col * P.ldct + row] = make_double2(-outr, outi);
         }
       }
@@ -597,12 +606,14 @@ void zgemm_reg_kernel(GemmArgs g) {
           }
           // explicit fma, as in zgemm_kernel
           double outr = fma(g.ar, vr, -(g.ai * vi)), outi = fma(g.ar, vi, g.ai * vr);
-          if (!g.beta_zero) {
+          if (!g.beta_zero && P.Cin) {
             const z2 c = beta_source(P, row, col);
             outr += fma(g.br, c.x, -(g.bi * c.y));
             outi += fma(g.br, c.y, g.bi * c.x);
+            if (P.Y)
+              P.Y[(int64_t)row * P.ldy + col] = make_double2(fma(0.5, vr, c.x), fma(0.5, vi, c.y));
           }
-          C[(int64_t)row * P.ldc + col] = make_double2(outr, outi);
+          if (C) C[(int64_t)row * P.ldc + col] = make_double2(outr, outi);
           if (P.Ct) P.Ct[(int64_t)col * P.ldct + row] = make_double2(-outr, outi);
         }
       }
@@ -795,7 +806,10 @@ void zgemm(hipStream_t s, int64_t batch, int m, int n, int k, int opA, int opB,
 namespace {
 
 void check_operands(int m, int n, const GemmOperands& o) {
-  QX_REQUIRE(!o.C.zero(), "zgemm: output is a zero matrix");
+  QX_REQUIRE(!o.C.zero() || !o.Y.zero(), "zgemm: output is a zero matrix");
+  QX_REQUIRE(o.Y.zero() || (!o.Cin.zero() && o.E.zero() && o.Y.p != o.C.p && o.Y.p != o.Ct.p &&
+                            o.Y.p != o.A.p && o.Y.p != o.B.p),
+             "zgemm: the half output needs a beta term and aliases no other operand");
   QX_REQUIRE(o.E.zero() || (m == n && !o.Cin.zero() && o.E.p != o.C.p && o.Cin.p != o.C.p),
              "zgemm: the D + E - E^H beta term needs m == n, a non-zero D and an output "
              "aliasing neither");
@@ -810,9 +824,9 @@ bool same_layout(const Mat& a, const Mat& b) { return a.zero() == b.zero(); }
 
 // An output of one product is no operand of the other.
 bool independent(const GemmOperands& x, const GemmOperands& y) {
-  for (const z2* w : {x.C.p, x.Ct.p}) {
+  for (const z2* w : {x.C.p, x.Ct.p, x.Y.p}) {
     if (!w) continue;
-    for (const z2* r : {y.A.p, y.B.p, y.Cin.p, y.E.p, y.C.p, y.Ct.p})
+    for (const z2* r : {y.A.p, y.B.p, y.Cin.p, y.E.p, y.C.p, y.Ct.p, y.Y.p})
       if (r == w) return false;
   }
   return true;
@@ -835,6 +849,11 @@ void zgemm_impl(hipStream_t s, int64_t batch, int m, int n, int k, int opA, int 
              "zgemm: precision must be QX_PREC_C128, QX_PREC_C64, QX_PREC_C128_3M, "
              "QX_PREC_OZAKI2(8..20) or QX_PREC_OZAKI_BF16(2..7)");
   if (batch <= 0 || m <= 0 || n <= 0) return;
+  for (int a = 0; a < ng; ++a)
+    QX_REQUIRE(gs[a]->Y.zero() || (!gs[a]->A.zero() && !gs[a]->B.zero() && k > 0 &&
+                                   (beta.re != 0.0 || beta.im != 0.0) &&
+                                   !oz2_moduli(precision) && !ozbf_slices(precision)),
+               "zgemm: no half output for this product");
   if (const int nmod = oz2_moduli(precision)) {
     // one launch sequence per product, in order, on the calling thread's
     // residue workspace
@@ -873,8 +892,8 @@ void zgemm_impl(hipStream_t s, int64_t batch, int m, int n, int k, int opA, int 
     for (int a = 1; a < ng; ++a) {
       const GemmOperands& o = *gs[a];
       one_launch = one_launch && same_layout(x.A, o.A) && same_layout(x.B, o.B) &&
-                   same_layout(x.Cin, o.Cin) && same_layout(x.C, o.C) &&
-                   same_layout(x.Ct, o.Ct) && same_layout(x.E, o.E);
+                   same_layout(x.C, o.C) && same_layout(x.Ct, o.Ct) && same_layout(x.E, o.E) &&
+                   same_layout(x.Y, o.Y);
     }
     if (!one_launch) {
       for (int a = 0; a < ng; ++a)
@@ -882,7 +901,8 @@ void zgemm_impl(hipStream_t s, int64_t batch, int m, int n, int k, int opA, int 
       return;
     }
   }
-  const bool beta_zero = (beta.re == 0.0 && beta.im == 0.0) || x.Cin.zero();
+  const bool beta_none = beta.re == 0.0 && beta.im == 0.0;
+  const bool beta_zero = beta_none || x.Cin.zero();
   if (x.A.zero() || x.B.zero() || k <= 0) {
     // op(A) op(B) == 0: C = beta Cin (Cin + E - E^H).
     if (!x.E.zero() && !beta_zero) {
@@ -913,11 +933,13 @@ void zgemm_impl(hipStream_t s, int64_t batch, int m, int n, int k, int opA, int 
   g.C = x.C.p;
   g.sC = x.C.stride;
   g.ldc = x.C.ld;
-  const Mat& ci = x.Cin.zero() ? x.C : x.Cin;
-  g.Cin = ci.p;
-  g.sCin = ci.stride;
-  g.ldcin = ci.ld;
-  g.beta_zero = beta_zero ? 1 : 0;
+  g.Cin = x.Cin.p;
+  g.sCin = x.Cin.stride;
+  g.ldcin = x.Cin.ld;
+  g.beta_zero = beta_none ? 1 : 0;
+  g.Y = x.Y.p;
+  g.sY = x.Y.stride;
+  g.ldy = x.Y.ld;
   g.Ct = x.Ct.p;
   g.sCt = x.Ct.stride;
   g.ldct = x.Ct.ld;
@@ -934,10 +956,12 @@ void zgemm_impl(hipStream_t s, int64_t batch, int m, int n, int k, int opA, int 
   g.C2 = o2.C.p;
   g.sC2 = o2.C.stride;
   g.ldc2 = o2.C.ld;
-  const Mat& ci2 = o2.Cin.zero() ? o2.C : o2.Cin;
-  g.Cin2 = ci2.p;
-  g.sCin2 = ci2.stride;
-  g.ldcin2 = ci2.ld;
+  g.Cin2 = o2.Cin.p;
+  g.sCin2 = o2.Cin.stride;
+  g.ldcin2 = o2.Cin.ld;
+  g.Y2 = o2.Y.p;
+  g.sY2 = o2.Y.stride;
+  g.ldy2 = o2.Y.ld;
   g.Ct2 = o2.Ct.p;
   g.sCt2 = o2.Ct.stride;
   g.ldct2 = o2.Ct.ld;
@@ -954,10 +978,12 @@ void zgemm_impl(hipStream_t s, int64_t batch, int m, int n, int k, int opA, int 
   g.C3 = o3.C.p;
   g.sC3 = o3.C.stride;
   g.ldc3 = o3.C.ld;
-  const Mat& ci3 = o3.Cin.zero() ? o3.C : o3.Cin;
-  g.Cin3 = ci3.p;
-  g.sCin3 = ci3.stride;
-  g.ldcin3 = ci3.ld;
+  g.Cin3 = o3.Cin.p;
+  g.sCin3 = o3.Cin.stride;
+  g.ldcin3 = o3.Cin.ld;
+  g.Y3 = o3.Y.p;
+  g.sY3 = o3.Y.stride;
+  g.ldy3 = o3.Y.ld;
   g.Ct3 = o3.Ct.p;
   g.sCt3 = o3.Ct.stride;
   g.ldct3 = o3.Ct.ld;
@@ -988,11 +1014,9 @@ void zgemm_in(hipStream_t s, int64_t batch, int m, int n, int k, int opA, int op
              nullptr, precision);
 }
 
-void zgemm_hin(hipStream_t s, int64_t batch, int n, int k, int opA, int opB, Cplx alpha,
-               const Mat& A, const Mat& B, Cplx beta, const Mat& D, const Mat& E, const Mat& C,
-               int precision) {
-  zgemm_impl(s, batch, n, n, k, opA, opB, alpha, beta, GemmOperands{A, B, D, C, Mat(), E},
-             nullptr, precision);
+void zgemm_one(hipStream_t s, int64_t batch, int m, int n, int k, int opA, int opB, Cplx alpha,
+               Cplx beta, const GemmOperands& x, int precision) {
+  zgemm_impl(s, batch, m, n, k, opA, opB, alpha, beta, x, nullptr, precision);
 }
 
 void zgemm_pair(hipStream_t s, int64_t batch, int m, int n, int k, int opA, int opB,

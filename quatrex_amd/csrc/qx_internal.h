@@ -110,20 +110,20 @@ void zgemm(hipStream_t s, int64_t batch, int m, int n, int k, int opA, int opB,
 void zgemm_in(hipStream_t s, int64_t batch, int m, int n, int k, int opA, int opB,
               Cplx alpha, const Mat& A, const Mat& B, Cplx beta, const Mat& Cin,
               const Mat& C, int precision, const Mat& Ct = Mat());
-// C = alpha op(A) op(B) + beta (D + E - E^H), n x n: the Hermitian-part sum
-// (ew_herm_add) formed in the product's epilogue, rounded as that kernel
-// rounds it.  C aliases neither D nor E.
-void zgemm_hin(hipStream_t s, int64_t batch, int n, int k, int opA, int opB, Cplx alpha,
-               const Mat& A, const Mat& B, Cplx beta, const Mat& D, const Mat& E, const Mat& C,
-               int precision);
 // Operands of one product C = alpha op(A) op(B) + beta (Cin + E - E^H), E
-// optional (zero Mat), with the optional second output Ct = -C^H.
+// optional (zero Mat; n x n products only, rounded as ew_herm_add rounds the
+// sum; C aliases neither Cin nor E then), with the optional second output Ct = -C^H and the
+// optional third output Y = Cin + op(A) op(B) / 2 (it may alias Cin; C may then
+// be a zero Mat, not stored; not for the split-product precisions).
 struct GemmOperands {
-  Mat A, B, Cin, C, Ct, E;
+  Mat A, B, Cin, C, Ct, E, Y;
 };
+// One product given by its operands.
+void zgemm_one(hipStream_t s, int64_t batch, int m, int n, int k, int opA, int opB, Cplx alpha,
+               Cplx beta, const GemmOperands& x, int precision);
 // Two products of one shape, ops, alpha and beta (x and y, batch matrices
-// each) as a single launch of 2 batch matrices when every operand of x is
-// present exactly when its counterpart in y is (strides and leading
+// each) as a single launch of 2 batch matrices when every operand of x but
+// Cin is present exactly when its counterpart in y is (strides and leading
 // dimensions may differ; an operand shared by both is passed twice), op(A)
 // op(B) is not identically zero, and neither product reads or
 // writes an output of the other; otherwise x, then y, as two launches.  Each
@@ -243,6 +243,21 @@ void ew_antiherm(hipStream_t s, int64_t batch, int n, double scale,
 // as two launches, if an output of one is an operand of the other).
 void ew_antiherm_pair(hipStream_t s, int64_t batch, int n, double scale, const Mat& X0,
                       const Mat& Y0, const Mat& X1, const Mat& Y1);
+// Full G^<> blocks of the backward sweep from skew-Hermitian x and the product
+// P: Y = (X - X^H) / 2 + (P - P^H), one or two groups in one launch; a non-null
+// dens also receives Im diag of the first group's Y (stride dens_stride).
+void ew_skew_update(hipStream_t s, int64_t batch, int n, const Mat& X0, const Mat& P0,
+                    const Mat& Y0, const Mat* X1, const Mat* P1, const Mat* Y1, double* dens,
+                    int64_t dens_stride);
+// One block of skew_check: stride 0 checks a single matrix.
+struct SkewBlock {
+  const z2* p;
+  int64_t stride;
+  int n;
+};
+// flag = 1 if a matrix of any of the blocks differs from skew-Hermitian by
+// more than 64 eps of its largest entry (|re| + |im| in both), else 0.
+void skew_check(hipStream_t s, int64_t batch, const std::vector<SkewBlock>& blocks, int* flag);
 // Y += T^H - T             (square)
 void ew_add_hdiff(hipStream_t s, int64_t batch, int n, const Mat& T,
                   const Mat& Y);
@@ -322,7 +337,13 @@ struct qx_handle {
   std::vector<hipStream_t> streams;   // helper streams (default priority)
   std::vector<hipEvent_t> join;       // one per helper stream
   hipEvent_t fork = nullptr;
+  static constexpr int kMaxParts = 8;
+  // skew-Hermitian checks of selected_solve, one slot per sub-batch
+  int* skew_dev = nullptr;
+  int* skew_host = nullptr;  // pinned
+  std::vector<hipEvent_t> skew_ev;
   void* ensure_ws(size_t bytes);
   int* ensure_info(size_t n);
   int* ensure_mask(size_t n);
+  void ensure_skew();
 };

@@ -347,6 +347,23 @@ void rgf_selected_solve(qx_handle* h, hipStream_t st0, const qx_btd_layout* la,
   const bool stagger = !(stg_env && stg_env[0] == '0');
   const char* pair_env = std::getenv("QX_RGF_PAIR");
   const bool pair_on = !(pair_env && pair_env[0] == '0');
+  // The backward sweep with three products per quantity holds for
+  // skew-Hermitian Σ^≶ and is taken when the device finds them so; the check
+  // needs one wait for the device, so only a caller that allows it
+  // (QX_SOLVE_SKEW_CHECK) and does not record a graph gets it.  The
+  // reduced-precision products keep the reference's sequence.
+  bool skew_on = (flags & QX_SOLVE_SKEW_CHECK) != 0 && N > 1 && xl != xg &&
+                 (prec == QX_PREC_C128 || prec == QX_PREC_C128_3M);
+  if (skew_on) {
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(st0, &cap) != hipSuccess) {
+      // the default stream while another one records
+      (void)hipGetLastError();
+      cap = hipStreamCaptureStatusActive;
+    }
+    skew_on = cap == hipStreamCaptureStatusNone;
+  }
+  if (skew_on) h->ensure_skew();
   hipEvent_t stg_ev = nullptr;
   if (stagger) QX_HIP_CHECK(hipEventCreateWithFlags(&stg_ev, hipEventDisableTiming));
   std::promise<void> stg_set;
@@ -395,7 +412,7 @@ void rgf_selected_solve(qx_handle* h, hipStream_t st0, const qx_btd_layout* la,
     sl_[i] = N + i;
     sg_[i] = 2 * N + i;
   }
-  int spare = 3 * N;
+  int spare = 3 * N, spare_r = 3 * N + 2;
   const int T1s = 3 * N + 1, T3s = 3 * N + 3, T4s = 3 * N + 4, T5s = 3 * N + 5,
             T6s = 3 * N + 6, B1s = 3 * N + 7, B2s = 3 * N + 8, B3s = 3 * N + 9, B4s = 3 * N + 10,
             C1s = 3 * N + 11, C2s = 3 * N + 12, C3s = 3 * N + 13, C4s = 3 * N + 14;
@@ -424,10 +441,7 @@ void rgf_selected_solve(qx_handle* h, hipStream_t st0, const qx_btd_layout* la,
   // are wanted and pairing is on
   auto one = [&](int m, int n, int k, int opA, int opB, Cplx alpha, Cplx beta,
                  const GemmOperands& o) {
-    if (o.E.zero())
-      zgemm_in(st, S, m, n, k, opA, opB, alpha, o.A, o.B, beta, o.Cin, o.C, gp, o.Ct);
-    else
-      zgemm_hin(st, S, n, k, opA, opB, alpha, o.A, o.B, beta, o.Cin, o.E, o.C, gp);
+    zgemm_one(st, S, m, n, k, opA, opB, alpha, beta, o, gp);
   };
   auto prod = [&](bool h0, bool h1, int m, int n, int k, int opA, int opB, Cplx alpha,
                   Cplx beta, const GemmOperands& x, const GemmOperands& y) {
@@ -465,6 +479,22 @@ void rgf_selected_solve(qx_handle* h, hipStream_t st0, const qx_btd_layout* la,
          {X0, T3[0], T6[0], T6[0], none, none}, {X0, T3[1], T6[1], T6[1], none, none});
     prod(true, true, b0, b0, b0, QX_OP_N, QX_OP_C, kOne, kZero,
          {T6[0], X0, X[0], X[0], none, none}, {T6[1], X0, X[1], X[1], none, none});
+  }
+
+  // Σ^≶ and boundary blocks of this sub-batch against skew-Hermitian, on the
+  // stream so early that the answer is there before the forward sweep is
+  if (skew_on) {
+    std::vector<SkewBlock> blocks;
+    for (const Q& q : qs)
+      for (int i = 0; i < N; ++i) {
+        const Mat s = q.sig->diag(i), o = q.obc->get(i, bs(i));
+        if (!s.zero()) blocks.push_back({s.p, s.stride, bs(i)});
+        if (!o.zero()) blocks.push_back({o.p, o.stride, bs(i)});
+      }
+    skew_check(st, S, blocks, h->skew_dev + part);
+    QX_HIP_CHECK(hipMemcpyAsync(h->skew_host + part, h->skew_dev + part, sizeof(int),
+                                hipMemcpyDeviceToHost, st));
+    QX_HIP_CHECK(hipEventRecord(h->skew_ev[part], st));
   }
 
   // ---- forward sweep (rgf.py:234-295) ----
@@ -559,6 +589,19 @@ void rgf_selected_solve(qx_handle* h, hipStream_t st0, const qx_btd_layout* la,
     if (lds) ew_diag_imag(st, S, bn, W.get(sr[N - 1], bn), lds + orb_off[N - 1], n_orb, kLdos);
   }
 
+  bool skew = false;
+  if (skew_on) {
+    QX_HIP_CHECK(hipEventSynchronize(h->skew_ev[part]));
+    skew = h->skew_host[part] == 0;
+  }
+  // full[qi]: G^≶_jj of the step before (the caller's output block, projected,
+  // in the skew-Hermitian sweep where it is written, else a workspace slot)
+  Mat full[2];
+  for (int qi = 0; qi < 2; ++qi) {
+    const Mat d = qs[qi].out->diag(N - 1);
+    full[qi] = skew && !d.zero() ? d : slot(qi, N - 1, bs(N - 1));
+  }
+
   // ---- backward sweep (rgf.py:308-404) ----
   // gr[i]: full G^R_ii once computed (the caller's output block when it is
   // written, else a workspace slot)
@@ -569,18 +612,21 @@ void rgf_selected_solve(qx_handle* h, hipStream_t st0, const qx_btd_layout* la,
     const Mat Xri = W.get(sr[i], bi), Xrj = gr[j];
     const Mat Aij = A.upper(i), Aji = A.lower(i);
     const Mat B1 = W.get(B1s, bj), B2 = W.get(B2s, bi), B3 = W.get(B3s, bj), B4 = W.get(B4s, bi);
-    // B1 = xr_ii a_ij, B2 = xr_jj a_ji, B3 = B1 xr_jj (xr_ii a_ij xr_jj),
-    // B4 = B1 B2 (... a_ji): two pairs of one shape when bi == bj
+    // B1 = xr_ii a_ij, B2 = xr_jj a_ji, B3 = B1 xr_jj (xr_ii a_ij xr_jj; only
+    // Σ_ij terms and G^R_ij need it), B4 = B1 B2 (... a_ji): pairs of one shape
+    // when bi == bj.  The skew-Hermitian sweep forms B4 below.
+    const bool need_b3 = !qs[0].sig->upper(i).zero() || !qs[1].sig->upper(i).zero() ||
+                         (want_r && want_r_off && !XR.upper(i).zero());
     if (bi == bj) {
       prod(true, true, bi, bi, bi, QX_OP_N, QX_OP_N, kOne, kZero,
            {Xri, Aij, B1, B1, none, none}, {Xrj, Aji, B2, B2, none, none});
-      prod(true, true, bi, bi, bi, QX_OP_N, QX_OP_N, kOne, kZero,
+      prod(need_b3, !skew, bi, bi, bi, QX_OP_N, QX_OP_N, kOne, kZero,
            {B1, Xrj, B3, B3, none, none}, {B1, B2, B4, B4, none, none});
     } else {
       zgemm(st, S, bi, bj, bi, QX_OP_N, QX_OP_N, kOne, Xri, Aij, kZero, B1, gp);
       zgemm(st, S, bj, bi, bj, QX_OP_N, QX_OP_N, kOne, Xrj, Aji, kZero, B2, gp);
-      zgemm(st, S, bi, bj, bj, QX_OP_N, QX_OP_N, kOne, B1, Xrj, kZero, B3, gp);
-      zgemm(st, S, bi, bi, bj, QX_OP_N, QX_OP_N, kOne, B1, B2, kZero, B4, gp);
+      if (need_b3) zgemm(st, S, bi, bj, bj, QX_OP_N, QX_OP_N, kOne, B1, Xrj, kZero, B3, gp);
+      if (!skew) zgemm(st, S, bi, bi, bj, QX_OP_N, QX_OP_N, kOne, B1, B2, kZero, B4, gp);
     }
 
     if (want_cur) {
@@ -601,11 +647,81 @@ void rgf_selected_solve(qx_handle* h, hipStream_t st0, const qx_btd_layout* la,
         }
       }
       // tr(sigma_greater_tilde xl_jj - xg_jj sigma_lesser_tilde)
-      trace_diff(st, S, bj, C3, W.get(sl_[j], bj), W.get(sg_[j], bj), C2,
-                 cur + i, N - 1);
+      trace_diff(st, S, bj, C3, full[0], full[1], C2, cur + i, N - 1);
     }
 
-    {
+    const Mat out_r = want_r ? XR.diag(i) : Mat();
+    // G^R_ii goes straight into the output block, which the next step reads
+    const Mat Zr = !out_r.zero() ? out_r : W.get(spare_r, bi);
+
+    if (skew) {
+      // For skew-Hermitian x, with U = B2 x_ii and H = x_jj B1^H:
+      //   -x_ji = U + H, x_ij = (U + H)^H,
+      //   x_ii' = x_ii + (P - P^H), P = B1 (U + H / 2),
+      // three products per quantity instead of four (T = B1 U, and
+      // B1 x_jj B1^H = B1 H is half of itself minus its conjugate transpose).
+      // Every step is linear in x up to its Hermitian part, which rounding
+      // alone makes, so nothing is mixed into the solution; the error against
+      // extended precision is that of the four-product form.
+      Mat Xi[2], U[2], P[2], T5[2], Z[2], sij[2], up[2], low[2], to[2];
+      bool hs[2];
+      for (int qi = 0; qi < 2; ++qi) {
+        const Q& q = qs[qi];
+        Xi[qi] = slot(qi, i, bi);
+        U[qi] = W.get(q.T4, bi);
+        P[qi] = W.get(q.T6 == T6g ? C1s : q.T6, bi);
+        T5[qi] = W.get(q.T5, bj);
+        sij[qi] = q.sig->upper(i);
+        hs[qi] = !sij[qi].zero();
+        up[qi] = q.out->upper(i);
+        low[qi] = (!q.skip_lower) ? q.out->lower(i) : Mat();
+        const Mat d = q.out->diag(i);
+        Z[qi] = !d.zero() ? d : W.get(*q.spare, bi);
+        // with Σ_ij terms x_ij is completed below, its lower block with it
+        to[qi] = hs[qi] ? Mat() : low[qi];
+        if (hs[qi] && up[qi].zero()) up[qi] = W.get(q.T3, bj);
+      }
+      const GemmOperands b4{B1, B2, B4, B4, none, none};
+      const GemmOperands u0{B2, Xi[0], U[0], U[0], none, none},
+          u1{B2, Xi[1], U[1], U[1], none, none};
+      if (bi == bj && pair_on) {
+        zgemm_triple(st, S, bi, bi, bi, QX_OP_N, QX_OP_N, kOne, kZero, b4, u0, u1, gp);
+      } else {
+        one(bi, bi, bj, QX_OP_N, QX_OP_N, kOne, kZero, b4);
+        prod(true, true, bj, bi, bi, QX_OP_N, QX_OP_N, kOne, kZero, u0, u1);
+      }
+      prod(hs[0], hs[1], bi, bj, bi, QX_OP_N, QX_OP_N, kOne, kZero,
+           {Xri, sij[0], T5[0], T5[0], none, none}, {Xri, sij[1], T5[1], T5[1], none, none});
+      // C = -(U + H) (the lower block), -C^H (the upper one), Y = U + H / 2
+      prod(true, true, bj, bi, bj, QX_OP_N, QX_OP_C, kMinus, kMinus,
+           {full[0], B1, U[0], to[0], up[0], none, U[0]},
+           {full[1], B1, U[1], to[1], up[1], none, U[1]});
+      prod(hs[0], hs[1], bi, bj, bj, QX_OP_N, QX_OP_C, kOne, kOne,
+           {T5[0], Xrj, up[0], up[0], low[0], none}, {T5[1], Xrj, up[1], up[1], low[1], none});
+      const GemmOperands r{B4, Xri, Xri, Zr, none, none};
+      const GemmOperands p0{B1, U[0], none, P[0], none, none},
+          p1{B1, U[1], none, P[1], none, none};
+      if (bi == bj && pair_on) {
+        zgemm_triple(st, S, bi, bi, bi, QX_OP_N, QX_OP_N, kOne, kOne, r, p0, p1, gp);
+      } else {
+        one(bi, bi, bi, QX_OP_N, QX_OP_N, kOne, kOne, r);
+        prod(true, true, bi, bi, bj, QX_OP_N, QX_OP_N, kOne, kZero, p0, p1);
+      }
+      prod(hs[0], hs[1], bi, bi, bj, QX_OP_N, QX_OP_C, kMinus, kOne,
+           {T5[0], B3, P[0], P[0], none, none}, {T5[1], B3, P[1], P[1], none, none});
+      double* dst = dens ? dens + orb_off[i] : nullptr;
+      if (pair_on) {
+        ew_skew_update(st, S, bi, Xi[0], P[0], Z[0], &Xi[1], &P[1], &Z[1], dst, n_orb);
+      } else {
+        ew_skew_update(st, S, bi, Xi[0], P[0], Z[0], nullptr, nullptr, nullptr, dst, n_orb);
+        ew_skew_update(st, S, bi, Xi[1], P[1], Z[1], nullptr, nullptr, nullptr, nullptr, 0);
+      }
+      for (int qi = 0; qi < 2; ++qi) {
+        const Q& q = qs[qi];
+        if (q.out->diag(i).zero()) std::swap(*q.spare, (*q.slot)[i]);
+        full[qi] = Z[qi];
+      }
+    } else {
       // G^< temporaries T1, T5, T4 (x_ij when the output has no upper
       // block); G^> ones in its own slots
       Mat Xi[2], Xj[2], T1[2], T5[2], Z[2], Oij[2], low[2], sij[2];
@@ -613,7 +729,7 @@ void rgf_selected_solve(qx_handle* h, hipStream_t st0, const qx_btd_layout* la,
       for (int qi = 0; qi < 2; ++qi) {
         const Q& q = qs[qi];
         Xi[qi] = slot(qi, i, bi);
-        Xj[qi] = slot(qi, j, bj);
+        Xj[qi] = full[qi];
         T1[qi] = W.get(qi == 0 ? T1s : q.T3, bi);
         T5[qi] = W.get(q.T5, bj);
         Z[qi] = W.get(*q.spare, bi);
@@ -649,6 +765,7 @@ void rgf_selected_solve(qx_handle* h, hipStream_t st0, const qx_btd_layout* la,
       for (int qi = 0; qi < 2; ++qi) {
         const Q& q = qs[qi];
         std::swap(*q.spare, (*q.slot)[i]);
+        full[qi] = Z[qi];
         if (!proj2 && !q.out->diag(i).zero()) ew_antiherm(st, S, bi, 0.5, Z[qi], q.out->diag(i));
         if (dens && qi == 0) ew_diag_imag(st, S, bi, Z[qi], dens + orb_off[i], n_orb);
       }
@@ -660,17 +777,10 @@ void rgf_selected_solve(qx_handle* h, hipStream_t st0, const qx_btd_layout* la,
       if (!XR.lower(i).zero())
         zgemm(st, S, bj, bi, bi, QX_OP_N, QX_OP_N, kMinus, B2, Xri, kZero, XR.lower(i), gp);
     }
-    const Mat out_r = want_r ? XR.diag(i) : Mat();
-    if (!out_r.zero()) {
-      // straight into the output block, which the next step reads
-      zgemm_in(st, S, bi, bi, bi, QX_OP_N, QX_OP_N, kOne, B4, Xri, kOne, Xri, out_r, gp);
-      gr[i] = out_r;
-    } else {
-      const Mat Z = W.get(spare, bi);
-      zgemm_in(st, S, bi, bi, bi, QX_OP_N, QX_OP_N, kOne, B4, Xri, kOne, Xri, Z, gp);
-      std::swap(spare, sr[i]);
-      gr[i] = Z;
-    }
+    if (!skew)
+      zgemm_in(st, S, bi, bi, bi, QX_OP_N, QX_OP_N, kOne, B4, Xri, kOne, Xri, Zr, gp);
+    if (out_r.zero()) std::swap(spare_r, sr[i]);
+    gr[i] = Zr;
     if (lds) ew_diag_imag(st, S, bi, gr[i], lds + orb_off[i], n_orb, kLdos);
   }
   });

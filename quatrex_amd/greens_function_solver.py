@@ -318,6 +318,9 @@ class RGF(GFSolver):
             flags |= _lib.SOLVE_SKIP_LOWER_L
         if xg.symmetry:
             flags |= _lib.SOLVE_SKIP_LOWER_G
+        if not _lib.capturing():
+            # the call ends with a wait for the device anyway (sync_check)
+            flags |= _lib.SOLVE_SKEW_CHECK
         h, st = _lib.handle(dev), _lib.stream_ptr(dev)
         prec = _lib.RGF_PRECISIONS[self.precision]
         inner = int(np.prod(a.stack_shape[1:], dtype=np.int64))

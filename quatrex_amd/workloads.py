@@ -161,14 +161,16 @@ def solve_flops(n_blocks: int, b: int) -> float:
 
 def required_flops(n_blocks: int, b: int) -> float:
     """Flops one selected_solve energy (G^R diagonal, G^<, G^>) requires
-    when Sigma^< and Sigma^> are block-diagonal, as in these workloads: the
-    reference's products with Sigma_{i,i+1} (rgf.py:270, 283, 336-346, 358-368)
-    are products with a zero block.  Per block step 10 products and one
-    inverse in the forward sweep (a_ji x^R_ii, a_jj - t a_ij, and per lesser /
-    greater quantity a_ji x_ii, (.) a_ji^H + Sigma_jj, x^R_jj (.),
-    (.) x^R_jj^H) and 13 products in the backward sweep (x^R_ii a_ij,
-    x^R_jj a_ji and the two products with them, per quantity four, and the
-    G^R_ii update); block 0 has 4 products and one inverse.  Each product
-    and each inverse is 8 b^3 real flops.
+    when Sigma^< and Sigma^> are block-diagonal and skew-Hermitian, as in these
+    workloads: the reference's products with Sigma_{i,i+1} (rgf.py:270, 283,
+    336-346, 358-368) are products with a zero block, and for skew-Hermitian
+    x the backward sweep needs three products per quantity instead of four.
+    Per block step 10 products and one inverse in the forward sweep
+    (a_ji x^R_ii, a_jj - t a_ij, and per lesser / greater quantity a_ji x_ii,
+    (.) a_ji^H + Sigma_jj, x^R_jj (.), (.) x^R_jj^H) and 10 products in the
+    backward sweep (B1 = x^R_ii a_ij, B2 = x^R_jj a_ji, B1 B2, the G^R_ii
+    update, and per quantity B2 x_ii, x_jj B1^H and the product of B1 with
+    their sum); block 0 has 4 products and one inverse.  Each product and each
+    inverse is 8 b^3 real flops.  (The reduced-precision arithmetics run 22.)
     """
-    return 8.0 * b ** 3 * ((4 + 23 * (n_blocks - 1)) + n_blocks)
+    return 8.0 * b ** 3 * ((4 + 20 * (n_blocks - 1)) + n_blocks)

@@ -582,3 +582,113 @@ def test_ldos_against_oracle(device, shape):
         ldos = torch.zeros((ne, nb * b), dtype=torch.float64, device=device)
         RGF(ne).selected_solve(a, sl, sg, return_retarded=ret, ldos=ldos)
         assert rel_err(ldos.cpu().numpy(), ref) < 1e-10
+
+
+def _skew_case(device, bs, sigma, outs, ne=6):
+    """System, skew-Hermitian Σ^≶ and boundary blocks, and output containers:
+    sigma "full" has off-diagonal blocks; outs "diag" stores diagonal output
+    blocks only, "upper" lower-skipping containers (symmetric storage)."""
+    rng = np.random.default_rng(31)
+    n = len(bs)
+    oa = ODSDBCOO.from_sparray(sps.coo_matrix(bt_dense(bs, seed=41)), bs, (ne,))
+    oa.data = oa.data * (1.0 + 0.05 * np.arange(ne))[:, None]
+    off = np.hstack(([0], np.cumsum(bs)))
+    mask = np.zeros((off[-1], off[-1]), dtype=bool)
+    for i in range(n):
+        mask[off[i]:off[i + 1], off[i]:off[i + 1]] = True
+    sig = []
+    for q in range(2):
+        m = bt_dense(bs, seed=42 + q)
+        m = m if sigma == "full" else np.where(mask, m, 0)
+        sig.append(ODSDBCOO.from_sparray(sps.coo_matrix(m - m.conj().T), bs, (ne,)))
+    obc = OBCBlocks(n)
+    for i in (0, n - 1):
+        g = 0.05 * (rng.standard_normal((ne, bs[i], bs[i])) + 1j * rng.standard_normal((ne, bs[i], bs[i])))
+        obc.lesser[i] = torch.as_tensor(1j * (g @ g.conj().transpose(0, 2, 1)), device=device)
+        obc.greater[i] = torch.as_tensor(-1j * (g @ g.conj().transpose(0, 2, 1)), device=device)
+    a, sl, sg = (to_gpu(o, device) for o in (oa, *sig))
+
+    def container():
+        pattern = mask if outs == "diag" else bt_dense(bs, seed=41) != 0
+        o = ODSDBCOO.from_sparray(sps.coo_matrix(pattern.astype(np.complex128)), bs, (ne,),
+                                  symmetry=outs == "upper")
+        c = to_gpu(o, device)
+        c.data[...] = 0
+        return c
+    return a, sl, sg, obc, container, int(off[-1])
+
+
+@pytest.mark.parametrize("precision", ["c128", "c128-3m"])
+@pytest.mark.parametrize("sigma", ["diag", "full"])
+@pytest.mark.parametrize("outs", ["btd", "diag", "upper"])
+@pytest.mark.parametrize("bs", [[64, 64, 64, 64], [48, 65, 64, 33, 100]], ids=["equal", "mixed"])
+def test_skew_sweep_matches_general_sweep(device, monkeypatch, bs, outs, sigma, precision):
+    """The backward sweep for skew-Hermitian Σ^≶ (three products per quantity)
+    against the general one (the check not asked for) over everything it
+    accepts: Σ_ij blocks, boundary blocks, outputs without off-diagonal or
+    lower blocks, unequal block sizes, current, density, corner, G^R with
+    off-diagonal blocks.  Equal to rounding; one launch per product
+    (QX_RGF_PAIR=0) gives the same bits as the joint launches."""
+    from quatrex_amd import _lib
+
+    a, sl, sg, obc, container, n_orb = _skew_case(device, np.array(bs), sigma, outs)
+    ne = a.data.shape[0]
+
+    def run(check, pair, retarded):
+        monkeypatch.setattr(_lib, "SOLVE_SKEW_CHECK", 32 if check else 0)
+        monkeypatch.setenv("QX_RGF_PAIR", pair)
+        out = [container(), container()] + ([to_gpu_zeros(a)] if retarded else [])
+        dens = torch.zeros((ne, n_orb), dtype=torch.float64, device=device)
+        corner = torch.zeros((ne, bs[0], bs[-1]), dtype=torch.complex128, device=device)
+        cur = RGF(ne, precision=precision, retarded_offdiag=True).selected_solve(
+            a, sl, sg, obc_blocks=obc, out=tuple(out), return_retarded=retarded,
+            return_current=True, density=dens, corner=corner)
+        return [x.data.cpu().numpy() for x in out] + [t.cpu().numpy() for t in (cur, dens, corner)]
+
+    for retarded in (True, False):
+        new, old, single = run(True, "1", retarded), run(False, "1", retarded), run(True, "0", retarded)
+        for x, y, z in zip(new, old, single):
+            assert np.allclose(x, y, rtol=1e-10, atol=1e-10 * np.abs(y).max())
+            assert np.array_equal(x.view(np.uint64), z.view(np.uint64))
+        assert any(not np.array_equal(x, y) for x, y in zip(new, old))  # another sweep indeed
+
+
+def to_gpu_zeros(m: DSDBCOO) -> DSDBCOO:
+    z = DSDBCOO.zeros_like(m)
+    z.data[...] = 0
+    return z
+
+
+@pytest.mark.parametrize("where", ["sigma", "boundary", "nan"])
+def test_skew_check_keeps_other_inputs_on_the_general_sweep(device, monkeypatch, where):
+    """Σ^≶ or boundary blocks that are not skew-Hermitian (by 1e-12 of one
+    block's largest entry), or not finite, take the general sweep: the bits of
+    a call without the check."""
+    from quatrex_amd import _lib
+
+    bs = np.array([64, 40, 64])
+    a, sl, sg, obc, container, _ = _skew_case(device, bs, "diag", "btd")
+    if where == "sigma":
+        blk = sg.blocks[1, 1]
+        blk[3, 5, 7] += 1e-12 * blk[3].abs().max()
+        sg.blocks[1, 1] = blk
+    elif where == "boundary":
+        obc.lesser[2][2, 1, 0] += 1e-12 * obc.lesser[2][2].abs().max()
+    else:
+        blk = sl.blocks[2, 2]
+        blk[0, 0, 0] = complex("nan")
+        sl.blocks[2, 2] = blk
+    outs = []
+    for check in (32, 0):
+        monkeypatch.setattr(_lib, "SOLVE_SKEW_CHECK", check)
+        # one sub-batch: its check is for all of its energies
+        monkeypatch.setenv("QX_RGF_STREAMS", "1")
+        h = _lib.new_handle(device)
+        _lib.set_tuning(h, streams=1)
+        with _lib.use_handle(h):
+            out = (container(), container())
+            RGF(6).selected_solve(a, sl, sg, obc_blocks=obc, out=out)
+        _lib.load().qx_destroy(h)
+        outs.append([x.data.cpu().numpy() for x in out])
+    for x, y in zip(*outs):
+        assert np.array_equal(x.view(np.uint64), y.view(np.uint64))
