@@ -387,30 +387,46 @@ __global__ __launch_bounds__(NT) void diag_imag_kernel(const z2* X, int64_t sX, 
 }
 
 // System matrix on the nnz pattern: A[e, k] = z_e S_k + T_k - Sig[e, k].
+// A workgroup covers NT consecutive entries of kAsmE energies: S and T are read
+// once for them, the Sigma loads of all are in flight together, and nothing is
+// divided by nnz (one thread per element of a flat grid: two 64-bit divisions
+// each, 3.4 TB/s at 256 energies of 866 k entries).  Streaming, 32 bytes per
+// entry and energy.
+constexpr int kAsmE = 8;
+template <bool SIG>
 __global__ __launch_bounds__(NT) void assemble_kernel(const z2* z, const z2* S, const z2* T,
                                                       const z2* Sig, int64_t sSig, z2* A,
-                                                      int64_t sA, int64_t nnz, int64_t total) {
-  for (int64_t i = blockIdx.x * (int64_t)NT + threadIdx.x; i < total;
-       i += (int64_t)gridDim.x * NT) {
-    const int64_t e = i / nnz;
-    const int64_t k = i - e * nnz;
-    double vr = 0.0, vi = 0.0;
-    if (S) {
-      const z2 ze = z[e], sk = S[k];
-      vr = ze.x * sk.x - ze.y * sk.y;
-      vi = ze.x * sk.y + ze.y * sk.x;
+                                                      int64_t sA, int64_t nnz, int64_t batch) {
+  const int64_t k = blockIdx.x * (int64_t)NT + threadIdx.x;
+  const int64_t e0 = blockIdx.y * (int64_t)kAsmE;
+  if (k >= nnz) return;
+  const int ne = (int)(batch - e0 < kAsmE ? batch - e0 : kAsmE);
+  z2 sg[kAsmE];
+  if constexpr (SIG) {
+#pragma unroll
+    for (int u = 0; u < kAsmE; ++u) sg[u] = Sig[(e0 + (u < ne ? u : 0)) * sSig + k];
+  }
+  const z2 sk = S ? S[k] : make_double2(0.0, 0.0);
+  const z2 tk = T ? T[k] : make_double2(0.0, 0.0);
+#pragma unroll
+  for (int u = 0; u < kAsmE; ++u) {
+    if (u < ne) {
+      double vr = 0.0, vi = 0.0;
+      if (S) {
+        const z2 ze = z[e0 + u];
+        vr = ze.x * sk.x - ze.y * sk.y;
+        vi = ze.x * sk.y + ze.y * sk.x;
+      }
+      if (T) {
+        vr += tk.x;
+        vi += tk.y;
+      }
+      if constexpr (SIG) {
+        vr -= sg[u].x;
+        vi -= sg[u].y;
+      }
+      A[(e0 + u) * sA + k] = make_double2(vr, vi);
     }
-    if (T) {
-      const z2 tk = T[k];
-      vr += tk.x;
-      vi += tk.y;
-    }
-    if (Sig) {
-      const z2 sg = Sig[e * sSig + k];
-      vr -= sg.x;
-      vi -= sg.y;
-    }
-    A[e * sA + k] = make_double2(vr, vi);
   }
 }
 
@@ -635,10 +651,20 @@ void ew_assemble(hipStream_t s, int64_t batch, int64_t nnz, const z2* z, const z
                  const z2* T, const z2* Sig, int64_t sSig, z2* A, int64_t sA) {
   if (batch <= 0 || nnz <= 0) return;
   QX_REQUIRE(A && (z || !S), "assemble: null argument");
-  const int64_t total = batch * nnz;
-  hipLaunchKernelGGL(assemble_kernel, dim3(grid_for(total)), dim3(NT), 0, s, z, S, T, Sig, sSig, A,
-                     sA, nnz, total);
-  QX_HIP_CHECK(hipGetLastError());
+  const int64_t gx = (nnz + NT - 1) / NT;
+  QX_REQUIRE(gx < (int64_t(1) << 31), "assemble: grid too large");
+  constexpr int64_t per = int64_t(65535) * kAsmE;  // energies per launch (grid.y limit)
+  for (int64_t e = 0; e < batch; e += per) {
+    const int64_t n = std::min(per, batch - e);
+    const dim3 grid((unsigned)gx, (unsigned)((n + kAsmE - 1) / kAsmE));
+    if (Sig)
+      hipLaunchKernelGGL(assemble_kernel<true>, grid, dim3(NT), 0, s, z + (S ? e : 0), S, T,
+                         Sig + e * sSig, sSig, A + e * sA, sA, nnz, n);
+    else
+      hipLaunchKernelGGL(assemble_kernel<false>, grid, dim3(NT), 0, s, z + (S ? e : 0), S, T,
+                         Sig, sSig, A + e * sA, sA, nnz, n);
+    QX_HIP_CHECK(hipGetLastError());
+  }
 }
 
 void ew_ident_sub(hipStream_t s, int64_t batch, int n, const Mat& Y) {

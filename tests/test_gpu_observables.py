@@ -98,3 +98,39 @@ def test_system_matrix_assembly(device, with_overlap):
     asm = SystemMatrixAssembler(pattern, sps.csr_matrix(h), overlap=ov, potential=v)
     got = asm(e, 1e-3, gs)
     assert rel_err(got.data.cpu().numpy(), a.data) < 1e-14
+
+
+@pytest.mark.parametrize("batch", [1, 7, 8, 9, 17])
+@pytest.mark.parametrize("nnz", [1, 255, 257])
+@pytest.mark.parametrize("terms", ["zst", "st", "z", "t"])
+def test_assembly_kernel_edges(device, batch, nnz, terms):
+    """A = z S + T - Sigma for stacks and patterns around the kernel's groups of
+    eight energies and 256 entries, with each of the terms absent; entries
+    outside the stack are left alone."""
+    from quatrex_amd import _lib
+
+    rng = np.random.default_rng(batch * 1000 + nnz)
+    cn = lambda *s: rng.standard_normal(s) + 1j * rng.standard_normal(s)  # noqa: E731
+    z, s, t, sig = cn(batch), cn(nnz), cn(nnz), cn(batch, nnz)
+    want = np.zeros((batch, nnz), complex)
+    args = {"z": None, "s": None, "t": None, "sig": None}
+    if "z" in terms:
+        want += z[:, None] * s
+        args["z"], args["s"] = z, s
+    if "t" in terms:
+        want += t
+        args["t"] = t
+    if "s" in terms:
+        want -= sig
+        args["sig"] = sig
+    dev = {k: None if v is None else torch.as_tensor(v, device=device) for k, v in args.items()}
+    out = torch.full((batch + 1, nnz), 7.0, dtype=torch.complex128, device=device)
+    ptr = {k: None if v is None else v.data_ptr() for k, v in dev.items()}
+    h = _lib.handle(device)
+    rc = _lib.load().qx_assemble_system_matrix(h, _lib.stream_ptr(device), batch, nnz, ptr["z"],
+                                               ptr["s"], ptr["t"], ptr["sig"], nnz,
+                                               out.data_ptr(), nnz)
+    _lib.check(rc, h, "assemble")
+    got = out.cpu().numpy()
+    assert np.allclose(got[:batch], want, rtol=1e-15, atol=4e-15)
+    assert np.all(got[batch] == 7.0)
