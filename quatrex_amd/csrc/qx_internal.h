@@ -264,9 +264,10 @@ void ew_add_hdiff(hipStream_t s, int64_t batch, int n, const Mat& T,
 // Y = -X^H                 (X is m x n, Y is n x m)
 void ew_neg_h(hipStream_t s, int64_t batch, int m, int n, const Mat& X,
               const Mat& Y);
-// out[e * out_stride] = tr(X Y - Z W)   (square; complex)
+// out[e * out_stride] = tr(X Y - Z W)   (square; complex); part: scratch of
+// ceil(n / 32) elements per matrix, aliasing no operand
 void trace_diff(hipStream_t s, int64_t batch, int n, const Mat& X, const Mat& Y,
-                const Mat& Z, const Mat& W, z2* out, int64_t out_stride);
+                const Mat& Z, const Mat& W, z2* out, int64_t out_stride, const Mat& part);
 // out[e] = || |A| + |B| ||_F   (square)
 void absnorm2(hipStream_t s, int64_t batch, int n, const Mat& A, const Mat& B,
               double* out);

@@ -632,22 +632,23 @@ void rgf_selected_solve(qx_handle* h, hipStream_t st0, const qx_btd_layout* la,
     if (want_cur) {
       // Meir-Wingreen layer current from the forward (left-connected) blocks
       // of layer i and the full blocks of layer j (rgf.py:381-400).
-      const Mat C1 = W.get(C1s, bi), C2 = W.get(C2s, bj), C3 = W.get(C3s, bj), C4 = W.get(C4s, bj);
-      zgemm(st, S, bj, bi, bi, QX_OP_N, QX_OP_N, kOne, Aji, Xri, kZero, C1, gp);  // a_ji xr_ii
-      Mat tl[2] = {C2, C3};
-      for (int qi = 0; qi < 2; ++qi) {
-        const Q& q = qs[qi];
-        const Mat T4 = W.get(T4s, bi);
-        zgemm(st, S, bj, bi, bi, QX_OP_N, QX_OP_N, kOne, Aji, W.get((*q.slot)[i], bi), kZero, T4, gp);
-        zgemm(st, S, bj, bj, bi, QX_OP_N, QX_OP_C, kOne, T4, Aji, kZero, tl[qi], gp);
-        const Mat sij = q.sig->upper(i);
-        if (!sij.zero()) {
-          zgemm(st, S, bj, bj, bi, QX_OP_N, QX_OP_N, kOne, C1, sij, kZero, C4, gp);
+      const Mat C1 = W.get(C1s, bi), C4 = W.get(C4s, bj);
+      const Mat tl[2] = {W.get(C2s, bj), W.get(C3s, bj)};
+      const Mat T4[2] = {W.get(T4s, bi), W.get(T4g, bi)}, Xi[2] = {slot(0, i, bi), slot(1, i, bi)};
+      const Mat sij[2] = {SL.upper(i), SG.upper(i)};
+      if (!sij[0].zero() || !sij[1].zero())  // a_ji xr_ii
+        zgemm(st, S, bj, bi, bi, QX_OP_N, QX_OP_N, kOne, Aji, Xri, kZero, C1, gp);
+      prod(true, true, bj, bi, bi, QX_OP_N, QX_OP_N, kOne, kZero,
+           {Aji, Xi[0], T4[0], T4[0], none, none}, {Aji, Xi[1], T4[1], T4[1], none, none});
+      prod(true, true, bj, bj, bi, QX_OP_N, QX_OP_C, kOne, kZero,
+           {T4[0], Aji, tl[0], tl[0], none, none}, {T4[1], Aji, tl[1], tl[1], none, none});
+      for (int qi = 0; qi < 2; ++qi)
+        if (!sij[qi].zero()) {
+          zgemm(st, S, bj, bj, bi, QX_OP_N, QX_OP_N, kOne, C1, sij[qi], kZero, C4, gp);
           ew_add_hdiff(st, S, bj, C4, tl[qi]);
         }
-      }
       // tr(sigma_greater_tilde xl_jj - xg_jj sigma_lesser_tilde)
-      trace_diff(st, S, bj, C3, full[0], full[1], C2, cur + i, N - 1);
+      trace_diff(st, S, bj, tl[1], full[0], full[1], tl[0], cur + i, N - 1, C4);
     }
 
     const Mat out_r = want_r ? XR.diag(i) : Mat();
