@@ -42,6 +42,17 @@ struct Btd {
   Mat diag(int i) const { return L ? at(L->diag[i], bs(i)) : Mat(); }
   Mat upper(int i) const { return L ? at(L->upper[i], bs(i + 1)) : Mat(); }  // (i, i+1)
   Mat lower(int i) const { return L ? at(L->lower[i], bs(i)) : Mat(); }      // (i+1, i)
+  // One past the last element any block of any matrix uses.
+  const z2* end() const {
+    int64_t m = 0;
+    for (int i = 0; i < L->n_blocks; ++i) {
+      m = std::max(m, L->diag[i] + (int64_t)bs(i) * bs(i));
+      if (i + 1 < L->n_blocks)
+        m = std::max(m, std::max(L->upper[i], L->lower[i]) + (int64_t)bs(i) * bs(i + 1));
+    }
+    return base + (L->n_stack - 1) * L->stack_stride + m;
+  }
+  bool overlaps(const Btd& o) const { return base < o.end() && o.base < end(); }
 };
 
 void check_layout(const qx_btd_layout* l, const qx_btd_layout* ref, const char* what) {
@@ -224,6 +235,10 @@ void rgf_selected_inv(qx_handle* h, hipStream_t st0, const qx_btd_layout* la,
   // QX_RGF_PAIR=0 (read per call): one launch per backward product
   const char* pair_env = std::getenv("QX_RGF_PAIR");
   const bool pair_on = !(pair_env && pair_env[0] == '0');
+  // a_ji x_ii is kept in the output (see the backward sweep) in complex128
+  // arithmetic, unless the output shares memory with A; the other arithmetics
+  // keep the reference's sequence of products
+  const bool keep = (prec == QX_PREC_C128 || prec == QX_PREC_C128_3M) && !A0.overlaps(X0);
   run_split(h, st0, Stot, [&](hipStream_t st, int64_t e0, int64_t S) {
     const OzSubBatch oz(prec, oz_region, bmax, e0, S);
     const Btd A = A0.sub(e0), X = X0.sub(e0);
@@ -237,6 +252,12 @@ void rgf_selected_inv(qx_handle* h, hipStream_t st0, const qx_btd_layout* la,
     const int t1 = N + 1, t2 = N + 2, t3 = N + 3;
     const InvScratch scr = W.inv(N + 4);  // N + 6, N + 7: Newton-Schulz temporaries
     auto bs = [&](int i) { return A.bs(i); };
+    // a_ji x_ii of the forward sweep, kept for the backward one in the storage
+    // of x_ij (b_j x b_i there), which is written last
+    auto kept = [&](int i) {
+      const Mat u = keep ? X.upper(i) : Mat();
+      return u.zero() ? u : Mat(u.p, u.stride, bs(i));
+    };
 
     // Forward sweep (rgf.py:70-92).
     {
@@ -247,7 +268,7 @@ void rgf_selected_inv(qx_handle* h, hipStream_t st0, const qx_btd_layout* la,
     }
     for (int i = 0; i + 1 < N; ++i) {
       const int j = i + 1, bi = bs(i), bj = bs(j);
-      const Mat T1 = W.get(t1, bi);
+      const Mat T1 = kept(i).zero() ? W.get(t1, bi) : kept(i);
       zgemm(st, S, bj, bi, bi, QX_OP_N, QX_OP_N, kOne, A.lower(i), W.get(xd[i], bi), kZero, T1, gp);
       const Mat Xj = W.get(xd[j], bj), Mj = zinv_input(bj, Xj, scr, ip);
       Mat Ajj = A.diag(j);
@@ -263,14 +284,37 @@ void rgf_selected_inv(qx_handle* h, hipStream_t st0, const qx_btd_layout* la,
       ew_axpby(st, S, bs(N - 1), bs(N - 1), kOne, W.get(xd[N - 1], bs(N - 1)), kZero, Mat(),
                X.diag(N - 1));
 
-    // Backward sweep (rgf.py:97-110).
+    // Backward sweep (rgf.py:97-110).  Xjj: the full block of the step before.
+    Mat Xjj = W.get(xd[N - 1], bs(N - 1));
     for (int i = N - 2; i >= 0; --i) {
       const int j = i + 1, bi = bs(i), bj = bs(j);
-      const Mat Xii = W.get(xd[i], bi), Xjj = W.get(xd[j], bj);
+      const Mat Xii = W.get(xd[i], bi);
       const Mat T1 = W.get(t1, bi), T2 = W.get(t2, bj);
       Mat Xji = X.lower(i);
       if (Xji.zero()) Xji = W.get(t3, bi);
       const Mat Xij = X.upper(i);
+      if (!kept(i).zero()) {
+        // x_ji = -x_jj (a_ji x_ii), t = -x_ii a_ij, then x_ij = t x_jj and
+        // x_ii <- x_ii + t x_ji straight into the output block: four products
+        // and two launches per step where the general form below has five and
+        // three, and no copy of the diagonal block
+        const Mat none, d = X.diag(i), Z = d.zero() ? W.get(spare, bi) : d;
+        const GemmOperands ji{Xjj, kept(i), Xji, Xji, none, none},
+            t{Xii, A.upper(i), T2, T2, none, none}, ij{T2, Xjj, none, Xij, none, none},
+            ii{T2, Xji, Xii, Z, none, none};
+        if (pair_on && bi == bj) {
+          zgemm_pair(st, S, bi, bi, bi, QX_OP_N, QX_OP_N, kMinus, kZero, ji, t, gp);
+          zgemm_pair(st, S, bi, bi, bi, QX_OP_N, QX_OP_N, kOne, kOne, ij, ii, gp);
+        } else {
+          zgemm_one(st, S, bj, bi, bj, QX_OP_N, QX_OP_N, kMinus, kZero, ji, gp);
+          zgemm_one(st, S, bi, bj, bi, QX_OP_N, QX_OP_N, kMinus, kZero, t, gp);
+          zgemm_one(st, S, bi, bj, bj, QX_OP_N, QX_OP_N, kOne, kOne, ij, gp);
+          zgemm_one(st, S, bi, bi, bj, QX_OP_N, QX_OP_N, kOne, kOne, ii, gp);
+        }
+        if (d.zero()) std::swap(spare, xd[i]);
+        Xjj = Z;
+        continue;
+      }
       if (pair_on && bi == bj) {
         // the x_ji and x_ij chains below, each product pair as one launch
         const Mat none;
@@ -295,6 +339,7 @@ void rgf_selected_inv(qx_handle* h, hipStream_t st0, const qx_btd_layout* la,
       const Mat Z = W.get(spare, bi);
       zgemm_in(st, S, bi, bi, bj, QX_OP_N, QX_OP_N, kMinus, T2, Xji, kOne, Xii, Z, gp);
       std::swap(spare, xd[i]);
+      Xjj = Z;
       if (!X.diag(i).zero())
         ew_axpby(st, S, bi, bi, kOne, W.get(xd[i], bi), kZero, Mat(), X.diag(i));
     }

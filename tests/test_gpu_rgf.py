@@ -584,13 +584,20 @@ def test_ldos_against_oracle(device, shape):
         assert rel_err(ldos.cpu().numpy(), ref) < 1e-10
 
 
+def _bt_full(bs, seed):
+    """bt_dense with every entry of the block tridiagonal pattern stored."""
+    m = bt_dense(bs, seed=seed)
+    blk = np.repeat(np.arange(len(bs)), bs)
+    return np.where((np.abs(blk[:, None] - blk) <= 1) & (m == 0), 0.01, m)
+
+
 def _skew_case(device, bs, sigma, outs, ne=6):
     """System, skew-Hermitian Σ^≶ and boundary blocks, and output containers:
     sigma "full" has off-diagonal blocks; outs "diag" stores diagonal output
     blocks only, "upper" lower-skipping containers (symmetric storage)."""
     rng = np.random.default_rng(31)
     n = len(bs)
-    oa = ODSDBCOO.from_sparray(sps.coo_matrix(bt_dense(bs, seed=41)), bs, (ne,))
+    oa = ODSDBCOO.from_sparray(sps.coo_matrix(_bt_full(bs, 41)), bs, (ne,))
     oa.data = oa.data * (1.0 + 0.05 * np.arange(ne))[:, None]
     off = np.hstack(([0], np.cumsum(bs)))
     mask = np.zeros((off[-1], off[-1]), dtype=bool)
@@ -598,7 +605,7 @@ def _skew_case(device, bs, sigma, outs, ne=6):
         mask[off[i]:off[i + 1], off[i]:off[i + 1]] = True
     sig = []
     for q in range(2):
-        m = bt_dense(bs, seed=42 + q)
+        m = _bt_full(bs, 42 + q)
         m = m if sigma == "full" else np.where(mask, m, 0)
         sig.append(ODSDBCOO.from_sparray(sps.coo_matrix(m - m.conj().T), bs, (ne,)))
     obc = OBCBlocks(n)
@@ -609,7 +616,7 @@ def _skew_case(device, bs, sigma, outs, ne=6):
     a, sl, sg = (to_gpu(o, device) for o in (oa, *sig))
 
     def container():
-        pattern = mask if outs == "diag" else bt_dense(bs, seed=41) != 0
+        pattern = mask if outs == "diag" else _bt_full(bs, 41) != 0
         o = ODSDBCOO.from_sparray(sps.coo_matrix(pattern.astype(np.complex128)), bs, (ne,),
                                   symmetry=outs == "upper")
         c = to_gpu(o, device)
@@ -692,3 +699,34 @@ def test_skew_check_keeps_other_inputs_on_the_general_sweep(device, monkeypatch,
         outs.append([x.data.cpu().numpy() for x in out])
     for x, y in zip(*outs):
         assert np.array_equal(x.view(np.uint64), y.view(np.uint64))
+
+
+@pytest.mark.parametrize("precision", ["c128", "c128-3m"])
+@pytest.mark.parametrize("form", ["btd", "diag", "in-place"])
+@pytest.mark.parametrize("bs", [[64, 64, 64, 64], [48, 65, 64, 33, 100]], ids=["equal", "mixed"])
+def test_selected_inv_output_forms(device, monkeypatch, bs, form, precision):
+    """selected_inv keeps a_ji x_ii in the x_ij output block where there is one
+    and the output shares no memory with A: full outputs, outputs with
+    diagonal blocks only and outputs written over A, against the oracle; one
+    launch per product gives the same bits."""
+    bs, ne = np.array(bs), 5
+    oa = ODSDBCOO.from_sparray(sps.coo_matrix(_bt_full(bs, 51)), bs, (ne,))
+    oa.data = oa.data * (1.0 + 0.05 * np.arange(ne))[:, None]
+    ref = orgf.RGF(ne).selected_inv(oa)
+    got = []
+    for pair in ("1", "0"):
+        monkeypatch.setenv("QX_RGF_PAIR", pair)
+        a = to_gpu(oa, device)
+        if form == "in-place":
+            x = a
+        elif form == "btd":
+            x = to_gpu_zeros(a)
+        else:
+            x = _skew_case(device, bs, "diag", "diag", ne)[4]()
+        assert RGF(ne, precision=precision).selected_inv(a, out=x) is None
+        got.append(x)
+    for i in range(len(bs)):
+        for j in (i - 1, i, i + 1):
+            if 0 <= j < len(bs) and (i == j or form != "diag"):
+                assert rel_err(got[0].blocks[i, j].cpu().numpy(), ref.blocks[i, j]) < 1e-10
+    assert torch.equal(torch.view_as_real(got[0].data), torch.view_as_real(got[1].data))
