@@ -33,7 +33,17 @@ const Cplx kOne{1.0, 0.0}, kMinus{-1.0, 0.0}, kZero{0.0, 0.0};
 
 // Sancho-Rubio decimation (sancho_rubio.py:33-86).  Products are formed left
 // to right as in the reference (alpha @ inverse @ beta == (alpha g) beta);
-// the repeated alpha g beta of the reference is computed once.
+// the repeated alpha g beta of the reference is computed once.  Per iteration
+// three product launches: t1 = -alpha g with t2 = -beta g; t1 beta, added to
+// eps and eps_s in the epilogue, with the new alpha = t1 alpha and beta =
+// t2 beta; t2 alpha, added to eps, which the epilogue also writes where the
+// next inverse starts.  (The couplings change sign with every iteration, which
+// no product of two of them sees.)  Bound by the products for large stacks (512
+// x 256 x 256, 13 iterations: 133.7 -> 125.6 ms, of which 79 ms of products and
+// 41 ms of inverses; with seven product and axpby launches more before) and by
+// the chain of launches for small ones (32 x 96 x 96, a device: 5.5 -> 3.8 ms).
+// Sub-batches on streams of their own, the inverse of one beside the products
+// of another, gained nothing at 512 (127 ms) and cost 10 to 40% below 128.
 int sancho_rubio(qx_handle* h, hipStream_t st, int64_t n, int b, const void* a_ii,
                  const void* a_ij, const void* a_ji, void* x_ii, int max_iter, double tol,
                  int* iters) {
@@ -43,45 +53,56 @@ int sancho_rubio(qx_handle* h, hipStream_t st, int64_t n, int b, const void* a_i
   if (n == 0) return QX_OK;
   const int64_t bb = (int64_t)b * b;
   const size_t slot = (size_t)(n * bb) * sizeof(z2);
-  // 10 matrix slots, inverse scratch (buffer + pivot ints), norms
-  z2* ws = static_cast<z2*>(h->ensure_ws(slot * 12 + (size_t)n * sizeof(double) * 2));
+  // 9 matrix slots, inverse scratch (buffer + pivot ints), norms
+  z2* ws = static_cast<z2*>(h->ensure_ws(slot * 11 + (size_t)n * sizeof(double)));
   auto M = [&](int k) { return Mat(ws + (int64_t)k * n * bb, bb, b); };
-  const InvScratch scr{ws + 10 * n * bb, bb, reinterpret_cast<int*>(ws + 11 * n * bb), 4 * bb};
-  double* dnorm = reinterpret_cast<double*>(ws + 12 * n * bb);
+  const Mat none, g = M(2), t1 = M(3), t2 = M(4), xout(x_ii, bb, b);
+  const InvScratch scr{ws + 9 * n * bb, bb, reinterpret_cast<int*>(ws + 10 * n * bb), 4 * bb};
+  double* dnorm = reinterpret_cast<double*>(ws + 11 * n * bb);
   int* info = h->ensure_info(n);
-  const Mat Aii(a_ii, bb, b), Aij(a_ij, bb, b), Aji(a_ji, bb, b), X(x_ii, bb, b);
-  int eps = 0, eps_s = 1, alpha = 2, beta = 3, g = 4, t1 = 5, t2 = 6, p = 7, na = 8, nb = 9;
-  ew_axpby(st, n, b, b, kOne, Aii, kZero, Mat(), M(eps));
-  ew_axpby(st, n, b, b, kOne, Aii, kZero, Mat(), M(eps_s));
-  ew_axpby(st, n, b, b, kOne, Aji, kZero, Mat(), M(alpha));
-  ew_axpby(st, n, b, b, kOne, Aij, kZero, Mat(), M(beta));
-  std::vector<double> hn(n);
-  bool converged = false;
+  h->ensure_words();
   const int prec = QX_PREC_C128;
-  for (int it = 0; it < max_iter; ++it) {
+
+  // the first iteration reads the caller's blocks where the later ones read
+  // their own: none is copied
+  Mat eps(a_ii, bb, b), eps_s = eps, eps_inv = eps;
+  Mat alpha(a_ji, bb, b), beta(a_ij, bb, b), na = M(5), nb = M(6);
+  const Mat start = zinv_input(b, g, scr, prec);
+  bool converged = false;
+  for (int it = 0; it < max_iter && !converged; ++it) {
     if (iters) *iters = it + 1;
-    zinv(st, n, b, M(eps), Mat(), M(g), info, prec, scr);
-    zgemm(st, n, b, b, b, QX_OP_N, QX_OP_N, kOne, M(alpha), M(g), kZero, M(t1), prec);  // a g
-    zgemm(st, n, b, b, b, QX_OP_N, QX_OP_N, kOne, M(beta), M(g), kZero, M(t2), prec);   // b g
-    zgemm(st, n, b, b, b, QX_OP_N, QX_OP_N, kOne, M(t1), M(beta), kZero, M(p), prec);   // a g b
-    // eps -= a g b + b g a ; eps_s -= a g b
-    ew_axpby(st, n, b, b, kOne, M(eps), kMinus, M(p), M(eps));
-    zgemm(st, n, b, b, b, QX_OP_N, QX_OP_N, kMinus, M(t2), M(alpha), kOne, M(eps), prec);
-    ew_axpby(st, n, b, b, kOne, M(eps_s), kMinus, M(p), M(eps_s));
-    zgemm(st, n, b, b, b, QX_OP_N, QX_OP_N, kOne, M(t1), M(alpha), kZero, M(na), prec);  // a g a
-    zgemm(st, n, b, b, b, QX_OP_N, QX_OP_N, kOne, M(t2), M(beta), kZero, M(nb), prec);   // b g b
-    std::swap(alpha, na);
-    std::swap(beta, nb);
-    absnorm2(st, n, b, M(alpha), M(beta), dnorm);
-    QX_HIP_CHECK(hipMemcpyAsync(hn.data(), dnorm, n * sizeof(double), hipMemcpyDeviceToHost, st));
-    QX_HIP_CHECK(hipStreamSynchronize(st));
-    const double delta = *std::max_element(hn.begin(), hn.end()) / 2.0;
-    if (delta < tol) {
-      converged = true;
-      break;
+    zinv(st, n, b, eps_inv, none, g, info, prec, scr);
+    zgemm_pair(st, n, b, b, b, QX_OP_N, QX_OP_N, kMinus, kZero, {alpha, g, none, t1, none, none},
+               {beta, g, none, t2, none, none}, prec);
+    GemmOperands ab{t1, beta, eps, M(0), none, none, M(1), eps_s};
+    const GemmOperands aa{t1, alpha, none, na, none, none, none, none, 1.0},
+        bb2{t2, beta, none, nb, none, none, none, none, 1.0};
+    eps = M(0);
+    eps_s = M(1);
+    GemmOperands ba{t2, alpha, eps, eps, none, none};
+    // (an inverse without panels starts from eps itself: its output is g)
+    eps_inv = start.p == g.p ? eps : start;
+    if (start.p != g.p) {
+      ba.Y = start;
+      ba.Yin = eps;
     }
+    ab.ys = ba.ys = 1.0;
+    zgemm_triple(st, n, b, b, b, QX_OP_N, QX_OP_N, kOne, kOne, ab, aa, bb2, prec);
+    zgemm_one(st, n, b, b, b, QX_OP_N, QX_OP_N, kOne, kOne, ba, prec);
+    absnorm2(st, n, b, na, nb, dnorm);
+    max_value(st, n, dnorm, h->word_dev);
+    QX_HIP_CHECK(hipMemcpyAsync(h->word_host, h->word_dev, sizeof(double), hipMemcpyDeviceToHost,
+                                st));
+    QX_HIP_CHECK(hipStreamSynchronize(st));
+    converged = *static_cast<volatile double*>(h->word_host) / 2.0 < tol;
+    // the couplings of the next iteration; the caller's are never written
+    const Mat fa = it == 0 ? M(7) : alpha, fb = it == 0 ? M(8) : beta;
+    alpha = na;
+    beta = nb;
+    na = fa;
+    nb = fb;
   }
-  zinv(st, n, b, M(eps_s), Mat(), X, info, prec, scr);
+  zinv(st, n, b, eps_s, none, xout, info, prec, scr);
   return converged ? QX_OK : QX_NOT_CONVERGED;
 }
 
@@ -272,18 +293,20 @@ int* qx_handle::ensure_info(size_t n) {
   return info;
 }
 
-void qx_handle::ensure_skew() {
-  if (skew_dev) return;
-  while (skew_ev.size() < kMaxParts) {
+void qx_handle::ensure_words() {
+  if (word_dev) return;
+  while (part_ev.size() < kMaxParts) {
     hipEvent_t ev;
     QX_HIP_CHECK(hipEventCreateWithFlags(&ev, hipEventDisableTiming));
-    skew_ev.push_back(ev);
+    part_ev.push_back(ev);
   }
-  if (!skew_host && hipHostMalloc(&skew_host, kMaxParts * sizeof(int)) != hipSuccess)
-    throw qx::Error{QX_ENOMEM, "skew flag allocation failed"};
-  if (hipMalloc(&skew_dev, kMaxParts * sizeof(int)) != hipSuccess) {
-    skew_dev = nullptr;
-    throw qx::Error{QX_ENOMEM, "skew flag allocation failed"};
+  if (!word_host && hipHostMalloc(&word_host, kMaxParts * sizeof(double)) != hipSuccess) {
+    word_host = nullptr;
+    throw qx::Error{QX_ENOMEM, "pinned memory allocation failed"};
+  }
+  if (hipMalloc(&word_dev, kMaxParts * sizeof(double)) != hipSuccess) {
+    word_dev = nullptr;
+    throw qx::Error{QX_ENOMEM, "flag allocation failed"};
   }
 }
 
@@ -425,9 +448,9 @@ int qx_destroy(qx_handle* h) {
   if (h->ws) (void)hipFree(h->ws);
   if (h->info) (void)hipFree(h->info);
   if (h->mask) (void)hipFree(h->mask);
-  if (h->skew_dev) (void)hipFree(h->skew_dev);
-  if (h->skew_host) (void)hipHostFree(h->skew_host);
-  for (hipEvent_t ev : h->skew_ev) (void)hipEventDestroy(ev);
+  if (h->word_dev) (void)hipFree(h->word_dev);
+  if (h->word_host) (void)hipHostFree(h->word_host);
+  for (hipEvent_t ev : h->part_ev) (void)hipEventDestroy(ev);
   delete h;
   return QX_OK;
 }

@@ -526,21 +526,57 @@ __global__ __launch_bounds__(NT) void trace_sum_kernel(const z2* part, int64_t s
   out[e * so] = make_double2(sr, si);
 }
 
-__global__ __launch_bounds__(NT) void absnorm_kernel(int n, const z2* A, int64_t sA, int lda,
-                                                     const z2* B, int64_t sB, int ldb,
-                                                     double* out) {
-  __shared__ double red[NT / 64];
+// One workgroup of NTN threads per matrix, four elements of both in flight per
+// thread (NT threads and one element: 21 us for 32 matrices of 96).
+constexpr int NTN = 1024;
+__global__ __launch_bounds__(NTN) void absnorm_kernel(int n, const z2* A, int64_t sA, int lda,
+                                                      const z2* B, int64_t sB, int ldb,
+                                                      double* out) {
+  __shared__ double red[NTN / 64];
   const int64_t e = blockIdx.x;
+  const int nn = n * n;
   double acc = 0.0;
-  for (int idx = threadIdx.x; idx < n * n; idx += NT) {
-    const int r = idx / n, c = idx - r * n;
-    const z2 a = A[e * sA + (int64_t)r * lda + c];
-    const z2 b = B[e * sB + (int64_t)r * ldb + c];
-    const double v = hypot(a.x, a.y) + hypot(b.x, b.y);
-    acc += v * v;
+  for (int i0 = threadIdx.x; i0 < nn; i0 += 4 * NTN) {
+    z2 a[4], b[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const int idx = min(i0 + u * NTN, nn - 1);
+      const int r = idx / n, c = idx - r * n;
+      a[u] = A[e * sA + (int64_t)r * lda + c];
+      b[u] = B[e * sB + (int64_t)r * ldb + c];
+    }
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const double v = hypot(a[u].x, a[u].y) + hypot(b[u].x, b[u].y);
+      if (i0 + u * NTN < nn) acc += v * v;
+    }
   }
-  acc = block_sum(acc, red);
-  if (threadIdx.x == 0) out[e] = sqrt(acc);
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) acc += __shfl_xor(acc, off, 64);
+  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = acc;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    double s = 0.0;
+    for (int q = 0; q < NTN / 64; ++q) s += red[q];
+    out[e] = sqrt(s);
+  }
+}
+
+__global__ __launch_bounds__(NT) void max_kernel(int64_t n, const double* v, double* out) {
+  __shared__ double red[NT / 64];
+  double m = -INFINITY;
+  for (int64_t i = threadIdx.x; i < n; i += NT) {
+    const double x = v[i];
+    m = x > m ? x : m;  // a NaN is passed over
+  }
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) m = fmax(m, __shfl_xor(m, off, 64));
+  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = m;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    for (int q = 1; q < NT / 64; ++q) m = fmax(m, red[q]);
+    *out = v[0] == v[0] ? m : v[0];
+  }
 }
 
 // Newton-Schulz check of one complex64 block inverse per workgroup (see
@@ -821,8 +857,14 @@ void trace_diff(hipStream_t s, int64_t batch, int n, const Mat& X, const Mat& Y,
 void absnorm2(hipStream_t s, int64_t batch, int n, const Mat& A, const Mat& B,
               double* out) {
   if (batch <= 0) return;
-  hipLaunchKernelGGL(absnorm_kernel, dim3((unsigned)batch), dim3(NT), 0, s, n, A.p,
+  hipLaunchKernelGGL(absnorm_kernel, dim3((unsigned)batch), dim3(NTN), 0, s, n, A.p,
                      A.stride, A.ld, B.p, B.stride, B.ld, out);
+  QX_HIP_CHECK(hipGetLastError());
+}
+
+void max_value(hipStream_t s, int64_t n, const double* v, double* out) {
+  QX_REQUIRE(n > 0 && v && out, "max_value: nothing to compare");
+  hipLaunchKernelGGL(max_kernel, dim3(1), dim3(NT), 0, s, n, v, out);
   QX_HIP_CHECK(hipGetLastError());
 }
 

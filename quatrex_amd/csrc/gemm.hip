@@ -75,7 +75,11 @@ struct GemmArgs {
   const z2* E;
   int64_t sE;
   int lde;
-  // optional: third output Y = Cin + op(A) op(B) / 2 (C may then be null)
+  // optional: third output Y = Yin + ys op(A) op(B) (C may then be null)
+  double ys;
+  const z2* Yin;
+  int64_t sYin;
+  int ldyin;
   z2* Y;
   int64_t sY;
   int ldy;
@@ -84,22 +88,22 @@ struct GemmArgs {
   // leading dimension) at index e - half, matrices e >= 2 half from the
   // third at e - 2 half.  Sets a launch does not use equal the first.
   int64_t half;
-  const z2 *A2, *B2, *Cin2, *E2;
+  const z2 *A2, *B2, *Cin2, *E2, *Yin2;
   z2 *C2, *Ct2, *Y2;
-  int64_t sA2, sB2, sC2, sCin2, sCt2, sE2, sY2;
-  int lda2, ldb2, ldc2, ldcin2, ldct2, lde2, ldy2;
-  const z2 *A3, *B3, *Cin3, *E3;
+  int64_t sA2, sB2, sC2, sCin2, sCt2, sE2, sY2, sYin2;
+  int lda2, ldb2, ldc2, ldcin2, ldct2, lde2, ldy2, ldyin2;
+  const z2 *A3, *B3, *Cin3, *E3, *Yin3;
   z2 *C3, *Ct3, *Y3;
-  int64_t sA3, sB3, sC3, sCin3, sCt3, sE3, sY3;
-  int lda3, ldb3, ldc3, ldcin3, ldct3, lde3, ldy3;
+  int64_t sA3, sB3, sC3, sCin3, sCt3, sE3, sY3, sYin3;
+  int lda3, ldb3, ldc3, ldcin3, ldct3, lde3, ldy3, ldyin3;
 };
 
 // Operands of matrix e of a launch (see GemmArgs::half); uniform over a
 // workgroup.
 struct GemmPtrs {
-  const z2 *A, *B, *Cin, *E;
+  const z2 *A, *B, *Cin, *E, *Yin;
   z2 *C, *Ct, *Y;
-  int lda, ldb, ldc, ldcin, ldct, lde, ldy;
+  int lda, ldb, ldc, ldcin, ldct, lde, ldy, ldyin;
 };
 __device__ __forceinline__ GemmPtrs gemm_ptrs(const GemmArgs& g, int64_t e) {
   const int grp = e >= 2 * g.half ? 2 : (e >= g.half ? 1 : 0);
@@ -110,11 +114,14 @@ __device__ __forceinline__ GemmPtrs gemm_ptrs(const GemmArgs& g, int64_t e) {
   p.A = QX_SEL(g.A + l * g.sA, g.A2 + l * g.sA2, g.A3 + l * g.sA3);
   p.B = QX_SEL(g.B + l * g.sB, g.B2 + l * g.sB2, g.B3 + l * g.sB3);
   p.C = g.C ? QX_SEL(g.C + l * g.sC, g.C2 + l * g.sC2, g.C3 + l * g.sC3) : nullptr;
-  // a group without a beta term has a null Cin of its own
+  // a group without a beta term or third output has null pointers of its own
   const z2* ci = QX_SEL(g.Cin, g.Cin2, g.Cin3);
   p.Cin = ci ? ci + l * QX_SEL(g.sCin, g.sCin2, g.sCin3) : nullptr;
-  p.Y = g.Y ? QX_SEL(g.Y + l * g.sY, g.Y2 + l * g.sY2, g.Y3 + l * g.sY3) : nullptr;
+  z2* y = QX_SEL(g.Y, g.Y2, g.Y3);
+  p.Y = y ? y + l * QX_SEL(g.sY, g.sY2, g.sY3) : nullptr;
   p.ldy = QX_SEL(g.ldy, g.ldy2, g.ldy3);
+  p.Yin = y ? QX_SEL(g.Yin, g.Yin2, g.Yin3) + l * QX_SEL(g.sYin, g.sYin2, g.sYin3) : nullptr;
+  p.ldyin = QX_SEL(g.ldyin, g.ldyin2, g.ldyin3);
   p.E = g.E ? QX_SEL(g.E + l * g.sE, g.E2 + l * g.sE2, g.E3 + l * g.sE3) : nullptr;
   p.Ct = g.Ct ? QX_SEL(g.Ct + l * g.sCt, g.Ct2 + l * g.sCt2, g.Ct3 + l * g.sCt3) : nullptr;
   p.lda = QX_SEL(g.lda, g.lda2, g.lda3);
@@ -349,8 +356,10 @@ void zgemm_kernel(GemmArgs g) {
             const z2 c = beta_source(P, row, col);
             outr += fma(g.br, c.x, -(g.bi * c.y));
             outi += fma(g.br, c.y, g.bi * c.x);
-            if (P.Y)
-              P.Y[(int64_t)row * P.ldy + col] = make_double2(fma(0.5, vr, c.x), fma(0.5, vi, c.y));
+          }
+          if (P.Y) {
+            const z2 y = P.Yin[(int64_t)row * P.ldyin + col];
+            P.Y[(int64_t)row * P.ldy + col] = make_double2(fma(g.ys, vr, y.x), fma(g.ys, vi, y.y));
           }
           if (C) C[(int64_t)row * P.ldc + col] = make_double2(outr, outi);
           if (P.Ct) P.Ct[(int64_t)col * P.ldct + row] = make_double2(-outr, outi);
@@ -610,8 +619,10 @@ void zgemm_reg_kernel(GemmArgs g) {
             const z2 c = beta_source(P, row, col);
             outr += fma(g.br, c.x, -(g.bi * c.y));
             outi += fma(g.br, c.y, g.bi * c.x);
-            if (P.Y)
-              P.Y[(int64_t)row * P.ldy + col] = make_double2(fma(0.5, vr, c.x), fma(0.5, vi, c.y));
+          }
+          if (P.Y) {
+            const z2 y = P.Yin[(int64_t)row * P.ldyin + col];
+            P.Y[(int64_t)row * P.ldy + col] = make_double2(fma(g.ys, vr, y.x), fma(g.ys, vi, y.y));
           }
           if (C) C[(int64_t)row * P.ldc + col] = make_double2(outr, outi);
           if (P.Ct) P.Ct[(int64_t)col * P.ldct + row] = make_double2(-outr, outi);
@@ -807,9 +818,9 @@ namespace {
 
 void check_operands(int m, int n, const GemmOperands& o) {
   QX_REQUIRE(!o.C.zero() || !o.Y.zero(), "zgemm: output is a zero matrix");
-  QX_REQUIRE(o.Y.zero() || (!o.Cin.zero() && o.E.zero() && o.Y.p != o.C.p && o.Y.p != o.Ct.p &&
-                            o.Y.p != o.A.p && o.Y.p != o.B.p),
-             "zgemm: the half output needs a beta term and aliases no other operand");
+  QX_REQUIRE(o.Y.zero() || (!o.Yin.zero() && o.Y.p != o.C.p && o.Y.p != o.Ct.p &&
+                            o.Y.p != o.A.p && o.Y.p != o.B.p && o.Y.p != o.E.p),
+             "zgemm: the third output needs its summand and aliases no other operand");
   QX_REQUIRE(o.E.zero() || (m == n && !o.Cin.zero() && o.E.p != o.C.p && o.Cin.p != o.C.p),
              "zgemm: the D + E - E^H beta term needs m == n, a non-zero D and an output "
              "aliasing neither");
@@ -826,7 +837,7 @@ bool same_layout(const Mat& a, const Mat& b) { return a.zero() == b.zero(); }
 bool independent(const GemmOperands& x, const GemmOperands& y) {
   for (const z2* w : {x.C.p, x.Ct.p, x.Y.p}) {
     if (!w) continue;
-    for (const z2* r : {y.A.p, y.B.p, y.Cin.p, y.E.p, y.C.p, y.Ct.p, y.Y.p})
+    for (const z2* r : {y.A.p, y.B.p, y.Cin.p, y.E.p, y.C.p, y.Ct.p, y.Y.p, y.Yin.p})
       if (r == w) return false;
   }
   return true;
@@ -851,9 +862,9 @@ void zgemm_impl(hipStream_t s, int64_t batch, int m, int n, int k, int opA, int 
   if (batch <= 0 || m <= 0 || n <= 0) return;
   for (int a = 0; a < ng; ++a)
     QX_REQUIRE(gs[a]->Y.zero() || (!gs[a]->A.zero() && !gs[a]->B.zero() && k > 0 &&
-                                   (beta.re != 0.0 || beta.im != 0.0) &&
-                                   !oz2_moduli(precision) && !ozbf_slices(precision)),
-               "zgemm: no half output for this product");
+                                   gs[a]->ys == x.ys && !oz2_moduli(precision) &&
+                                   !ozbf_slices(precision)),
+               "zgemm: no third output for this product");
   if (const int nmod = oz2_moduli(precision)) {
     // one launch sequence per product, in order, on the calling thread's
     // residue workspace
@@ -892,8 +903,7 @@ void zgemm_impl(hipStream_t s, int64_t batch, int m, int n, int k, int opA, int 
     for (int a = 1; a < ng; ++a) {
       const GemmOperands& o = *gs[a];
       one_launch = one_launch && same_layout(x.A, o.A) && same_layout(x.B, o.B) &&
-                   same_layout(x.C, o.C) && same_layout(x.Ct, o.Ct) && same_layout(x.E, o.E) &&
-                   same_layout(x.Y, o.Y);
+                   same_layout(x.C, o.C) && same_layout(x.Ct, o.Ct) && same_layout(x.E, o.E);
     }
     if (!one_launch) {
       for (int a = 0; a < ng; ++a)
@@ -937,9 +947,13 @@ void zgemm_impl(hipStream_t s, int64_t batch, int m, int n, int k, int opA, int 
   g.sCin = x.Cin.stride;
   g.ldcin = x.Cin.ld;
   g.beta_zero = beta_none ? 1 : 0;
+  g.ys = x.ys;
   g.Y = x.Y.p;
   g.sY = x.Y.stride;
   g.ldy = x.Y.ld;
+  g.Yin = x.Yin.p;
+  g.sYin = x.Yin.stride;
+  g.ldyin = x.Yin.ld;
   g.Ct = x.Ct.p;
   g.sCt = x.Ct.stride;
   g.ldct = x.Ct.ld;
@@ -962,6 +976,9 @@ void zgemm_impl(hipStream_t s, int64_t batch, int m, int n, int k, int opA, int 
   g.Y2 = o2.Y.p;
   g.sY2 = o2.Y.stride;
   g.ldy2 = o2.Y.ld;
+  g.Yin2 = o2.Yin.p;
+  g.sYin2 = o2.Yin.stride;
+  g.ldyin2 = o2.Yin.ld;
   g.Ct2 = o2.Ct.p;
   g.sCt2 = o2.Ct.stride;
   g.ldct2 = o2.Ct.ld;
@@ -984,6 +1001,9 @@ void zgemm_impl(hipStream_t s, int64_t batch, int m, int n, int k, int opA, int 
   g.Y3 = o3.Y.p;
   g.sY3 = o3.Y.stride;
   g.ldy3 = o3.Y.ld;
+  g.Yin3 = o3.Yin.p;
+  g.sYin3 = o3.Yin.stride;
+  g.ldyin3 = o3.Yin.ld;
   g.Ct3 = o3.Ct.p;
   g.sCt3 = o3.Ct.stride;
   g.ldct3 = o3.Ct.ld;

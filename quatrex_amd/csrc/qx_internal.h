@@ -113,17 +113,19 @@ void zgemm_in(hipStream_t s, int64_t batch, int m, int n, int k, int opA, int op
 // Operands of one product C = alpha op(A) op(B) + beta (Cin + E - E^H), E
 // optional (zero Mat; n x n products only, rounded as ew_herm_add rounds the
 // sum; C aliases neither Cin nor E then), with the optional second output Ct = -C^H and the
-// optional third output Y = Cin + op(A) op(B) / 2 (it may alias Cin; C may then
-// be a zero Mat, not stored; not for the split-product precisions).
+// optional third output Y = Yin + ys op(A) op(B) (Y may be Yin, and Yin may be
+// Cin; C may then be a zero Mat, not stored; not for the split-product
+// precisions; one ys per launch).
 struct GemmOperands {
-  Mat A, B, Cin, C, Ct, E, Y;
+  Mat A, B, Cin, C, Ct, E, Y, Yin;
+  double ys = 0.5;
 };
 // One product given by its operands.
 void zgemm_one(hipStream_t s, int64_t batch, int m, int n, int k, int opA, int opB, Cplx alpha,
                Cplx beta, const GemmOperands& x, int precision);
 // Two products of one shape, ops, alpha and beta (x and y, batch matrices
 // each) as a single launch of 2 batch matrices when every operand of x but
-// Cin is present exactly when its counterpart in y is (strides and leading
+// Cin and Y is present exactly when its counterpart in y is (strides and leading
 // dimensions may differ; an operand shared by both is passed twice), op(A)
 // op(B) is not identically zero, and neither product reads or
 // writes an output of the other; otherwise x, then y, as two launches.  Each
@@ -271,6 +273,9 @@ void trace_diff(hipStream_t s, int64_t batch, int n, const Mat& X, const Mat& Y,
 // out[e] = || |A| + |B| ||_F   (square)
 void absnorm2(hipStream_t s, int64_t batch, int n, const Mat& A, const Mat& B,
               double* out);
+// *out = the largest of v[0 .. n - 1] as std::max_element finds it: a NaN is
+// passed over unless it is the first.
+void max_value(hipStream_t s, int64_t n, const double* v, double* out);
 // Beyn: T = a_ji / z + a_ii + a_ij z for each (e, q) node; result stacks
 // ordered e-major then node.
 void contour_operator(hipStream_t s, int64_t batch, int nq, int b,
@@ -339,12 +344,13 @@ struct qx_handle {
   std::vector<hipEvent_t> join;       // one per helper stream
   hipEvent_t fork = nullptr;
   static constexpr int kMaxParts = 8;
-  // skew-Hermitian checks of selected_solve, one slot per sub-batch
-  int* skew_dev = nullptr;
-  int* skew_host = nullptr;  // pinned
-  std::vector<hipEvent_t> skew_ev;
+  // one word and one event per sub-batch, for answers read back by the host
+  // (skew-Hermitian checks of selected_solve, the Sancho-Rubio stop rule)
+  double* word_dev = nullptr;
+  double* word_host = nullptr;  // pinned
+  std::vector<hipEvent_t> part_ev;
   void* ensure_ws(size_t bytes);
   int* ensure_info(size_t n);
   int* ensure_mask(size_t n);
-  void ensure_skew();
+  void ensure_words();
 };

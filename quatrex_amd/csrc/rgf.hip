@@ -408,7 +408,7 @@ void rgf_selected_solve(qx_handle* h, hipStream_t st0, const qx_btd_layout* la,
     }
     skew_on = cap == hipStreamCaptureStatusNone;
   }
-  if (skew_on) h->ensure_skew();
+  if (skew_on) h->ensure_words();
   hipEvent_t stg_ev = nullptr;
   if (stagger) QX_HIP_CHECK(hipEventCreateWithFlags(&stg_ev, hipEventDisableTiming));
   std::promise<void> stg_set;
@@ -536,10 +536,11 @@ void rgf_selected_solve(qx_handle* h, hipStream_t st0, const qx_btd_layout* la,
         if (!s.zero()) blocks.push_back({s.p, s.stride, bs(i)});
         if (!o.zero()) blocks.push_back({o.p, o.stride, bs(i)});
       }
-    skew_check(st, S, blocks, h->skew_dev + part);
-    QX_HIP_CHECK(hipMemcpyAsync(h->skew_host + part, h->skew_dev + part, sizeof(int),
-                                hipMemcpyDeviceToHost, st));
-    QX_HIP_CHECK(hipEventRecord(h->skew_ev[part], st));
+    int* flag = reinterpret_cast<int*>(h->word_dev + part);
+    skew_check(st, S, blocks, flag);
+    QX_HIP_CHECK(hipMemcpyAsync(h->word_host + part, flag, sizeof(int), hipMemcpyDeviceToHost,
+                                st));
+    QX_HIP_CHECK(hipEventRecord(h->part_ev[part], st));
   }
 
   // ---- forward sweep (rgf.py:234-295) ----
@@ -636,8 +637,8 @@ void rgf_selected_solve(qx_handle* h, hipStream_t st0, const qx_btd_layout* la,
 
   bool skew = false;
   if (skew_on) {
-    QX_HIP_CHECK(hipEventSynchronize(h->skew_ev[part]));
-    skew = h->skew_host[part] == 0;
+    QX_HIP_CHECK(hipEventSynchronize(h->part_ev[part]));
+    skew = *reinterpret_cast<const volatile int*>(h->word_host + part) == 0;
   }
   // full[qi]: G^≶_jj of the step before (the caller's output block, projected,
   // in the skew-Hermitian sweep where it is written, else a workspace slot)
@@ -740,8 +741,8 @@ void rgf_selected_solve(qx_handle* h, hipStream_t st0, const qx_btd_layout* la,
            {Xri, sij[0], T5[0], T5[0], none, none}, {Xri, sij[1], T5[1], T5[1], none, none});
       // C = -(U + H) (the lower block), -C^H (the upper one), Y = U + H / 2
       prod(true, true, bj, bi, bj, QX_OP_N, QX_OP_C, kMinus, kMinus,
-           {full[0], B1, U[0], to[0], up[0], none, U[0]},
-           {full[1], B1, U[1], to[1], up[1], none, U[1]});
+           {full[0], B1, U[0], to[0], up[0], none, U[0], U[0]},
+           {full[1], B1, U[1], to[1], up[1], none, U[1], U[1]});
       prod(hs[0], hs[1], bi, bj, bj, QX_OP_N, QX_OP_C, kOne, kOne,
            {T5[0], Xrj, up[0], up[0], low[0], none}, {T5[1], Xrj, up[1], up[1], low[1], none});
       const GemmOperands r{B4, Xri, Xri, Zr, none, none};

@@ -35,6 +35,25 @@ def test_sancho_rubio_matches_oracle(device, b, ne):
     assert rel_err(np_(x), ref) < 1e-10
 
 
+# Sizes at the edges of the inverse's paths (whole matrix, panels whose input
+# the last product writes in place) and of the largest-norm reduction; eta 0.3
+# keeps the decimation well conditioned, so the module's bar of 1e-10 holds.
+# One iteration reads the caller's blocks alone, two and more the workspace.
+@pytest.mark.parametrize("b,ne", [(1, 300), (33, 257), (128, 2), (129, 3), (161, 1)])
+@pytest.mark.parametrize("limit", [1, 2, 100])
+@pytest.mark.filterwarnings("ignore:Surface Green's function")
+def test_sancho_rubio_iterations(device, b, ne, limit):
+    a_ji, a_ii, a_ij = lead(b=b, energies=np.linspace(-0.8, 0.8, ne), eta=0.3, seed=b)
+    blocks = [torch.as_tensor(a, device=device) for a in (a_ii, a_ij, a_ji)]
+    o = oobc.SanchoRubio(max_iterations=limit, convergence_tol=1e-12)
+    ref = o(a_ii, a_ij, a_ji)
+    g = SanchoRubio(max_iterations=limit, convergence_tol=1e-12)
+    x = g(*blocks)
+    assert g.iterations == o.iterations
+    assert rel_err(np_(x), ref) < 1e-10
+    assert all(np.array_equal(np_(t), a) for t, a in zip(blocks, (a_ii, a_ij, a_ji)))
+
+
 def test_sancho_rubio_chain_closed_form(device):
     z = np.array([-1.5, -0.3, 0.0, 0.7, 2.5]) + 1e-3j
     a_ii = (z - 0.2)[:, None, None]
