@@ -40,6 +40,7 @@
 // B[l/16][l%16]; result element e of lane l is D[l/16 + 4e][l%16] (f64) or
 // D[4(l/16) + e][l%16] (f32).
 #include <cstdlib>
+#include <type_traits>
 
 #include "gj_core.h"
 #include "qx_internal.h"
@@ -483,16 +484,26 @@ __device__ inline unsigned wave_max_bcast(unsigned v) {
 // it linearly, so scaling it once at the end gives the same row.  Nothing
 // then has to be written into the register slot of a runtime row.
 //
-// Per column, with one barrier:
-//   - the wave owning the column has published the column (all rows), the
-//     pivot key (wave max of the candidates' keys) and the pivot value to
-//     LDS, double-buffered by column parity so no second barrier guards the
-//     reuse;
-//   - after the barrier every wave reads the pivot key and value and the
-//     multipliers of its rows, and takes its part of row p (and the row's
-//     position) from the lane that holds it (v_readlane, p being uniform);
-//     1 / x_pk, the scaled pivot row and the elimination follow;
-//   - the owner of the next column computes and publishes its pivot data.
+// The owner of a column group runs one column ahead of the other waves: in one
+// step, ended by one barrier, it finds the pivot of its next column, publishes
+// the column's multipliers, pivot row and reciprocal in LDS (the multipliers
+// double-buffered by column parity) and applies the column to its own group,
+// at a raised wave priority, while the others apply the column published
+// before.  So the pivot search, the exchange of the pivot row's entries
+// (v_readlane, the row being uniform) and the reciprocal are off the path of
+// the waves that only follow, and a step costs the longer of the two instead
+// of their sum.  The column positions pass from owner to owner in LDS.
+//
+// Bound by the owner's chain, about 230 instructions per column at 256 rows:
+// 2500 -> 1850 cycles per column (2700 at a change of owner), of which the
+// key and its wave maximum take 450, the pivot row 500, the reciprocal 350
+// and the elimination 350.  Inverses with every wave in step before -> now
+// (with 64 RPL rows fitted to n): 32 x 256^2
+// 489 -> 440 us, 48 x 416^2 1547 -> 1416, 8 x 320^2 784 -> 575, 32 x 160^2
+// 286 -> 235, 512 x 256^2 2990 -> 2910.  Columns dealt out cyclically, each
+// published by a flag instead of a barrier, were slower (32 x 256^2: 513): every
+// wave then repeats the exchange of the pivot row.
+//
 // Pivot choice (largest |re| + |im| through the 32-bit key, ties to the lower
 // row), arithmetic and outputs are those of the other panel kernels up to
 // rounding; ties are broken by the row's index at the start of the panel.
@@ -510,10 +521,10 @@ __device__ inline float lane_read(float v, int l) {
 template <typename T, int RPL, int CW, int NB>
 struct PanelCgShared {
   T col_r[2][64 * RPL], col_i[2][64 * RPL];
-  T piv_r[2], piv_i[2];
-  unsigned key_b[2];
-  double rcp_r[NB], rcp_i[NB];
-  int perm_l[NB];
+  double rcp_r[NB], rcp_i[NB];  // reciprocal of each column's pivot
+  int piv[NB];                  // its row at the start of the panel
+  int perm_l[NB];               // and its position when it was chosen
+  int pos[64 * RPL];            // row positions, handed from owner to owner
 };
 
 // The panel of matrix e, by a workgroup of 64 NB / CW threads.
@@ -521,13 +532,6 @@ template <typename T, int RPL, int CW, int NB>
 __device__ __forceinline__ void panel_cg(const PanelArgs& g, int64_t e,
                                          PanelCgShared<T, RPL, CW, NB>& sh) {
   constexpr int NW = NB / CW, NTH = 64 * NW;
-  auto& col_r = sh.col_r;
-  auto& col_i = sh.col_i;
-  auto& piv_r = sh.piv_r;
-  auto& piv_i = sh.piv_i;
-  auto& key_b = sh.key_b;
-  auto& rcp_r = sh.rcp_r;
-  auto& rcp_i = sh.rcp_i;
   auto& perm_l = sh.perm_l;
   if (g.mask && !g.mask[e]) return;  // uniform over the workgroup
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
@@ -542,7 +546,7 @@ __device__ __forceinline__ void panel_cg(const PanelArgs& g, int64_t e,
 #pragma unroll
   for (int j = 0; j < RPL; ++j) {
     const int r = lane + 64 * j;
-    pos[j] = r;
+    pos[j] = r < n ? r : -1;  // rows beyond the matrix are no candidates
 #pragma unroll
     for (int c = 0; c < CW; ++c) {
       // unconditional loads from a clamped address, so that all of them are
@@ -554,38 +558,112 @@ __device__ __forceinline__ void panel_cg(const PanelArgs& g, int64_t e,
       xi[j][c] = ok ? (T)v.y : (T)0;
     }
   }
-  // Pivot data of panel column cn (register cn of the owner wave) into
-  // buffer b: the column, the key of the candidates (rows at position > kb)
-  // and the pivot value; the pivot row's entry of the published column (its
-  // multiplier in the elimination) is then zeroed, as the deferred scaling
-  // requires.
-  auto publish = [&](int cn, int b, int kb) {
+  // The elimination by column kk, whose column is in buffer b, of the wave's
+  // columns.  own: the wave's register of that column, -1 if it has none (a
+  // constant once inlined).
+  auto eliminate = [&](int p, const T (&fr)[RPL], const T (&fi)[RPL], double vr, double vi,
+                       int own) {
+    // this wave's part of row p, read from the lane that holds it (p is
+    // uniform: register row p >> 6 of lane p & 63)
+    const int pl = p & 63, pj = p >> 6;
+    T ar[CW], ai[CW];
+#pragma unroll
+    for (int c = 0; c < CW; ++c) ar[c] = ai[c] = (T)0;
+#pragma unroll
+    for (int j = 0; j < RPL; ++j) {
+      if (j == pj) {  // uniform: a scalar branch
+#pragma unroll
+        for (int c = 0; c < CW; ++c) {
+          if (c == own) continue;
+          ar[c] = lane_read(xr[j][c], pl);
+          ai[c] = lane_read(xi[j][c], pl);
+        }
+      }
+    }
+    T sr[CW], si[CW];
+#pragma unroll
+    for (int c = 0; c < CW; ++c) {
+      const double a = (double)ar[c], b = (double)ai[c];
+      sr[c] = (T)(a * vr - b * vi);
+      si[c] = (T)(a * vi + b * vr);
+      if (c == own) {
+        // active column: -f / x_pk for the other rows, 1 (scaled at the end)
+        // for the pivot row
+        sr[c] = (T)vr;
+        si[c] = (T)vi;
+#pragma unroll
+        for (int j = 0; j < RPL; ++j) {
+          xr[j][c] = (lane + 64 * j == p) ? (T)1 : (T)0;
+          xi[j][c] = (T)0;
+        }
+      }
+    }
+#pragma unroll
+    for (int j = 0; j < RPL; ++j) {
+#pragma unroll
+      for (int c = 0; c < CW; ++c) {
+        xr[j][c] = fma(-fr[j], sr[c], fma(fi[j], si[c], xr[j][c]));
+        xi[j][c] = fma(-fr[j], si[c], fma(-fi[j], sr[c], xi[j][c]));
+      }
+    }
+  };
+  // a published column applied to this wave's columns
+  auto apply = [&](int kk, int b) {
+    T fr[RPL], fi[RPL];
+#pragma unroll
+    for (int j = 0; j < RPL; ++j) {
+      fr[j] = sh.col_r[b][lane + 64 * j];  // zero for the pivot row
+      fi[j] = sh.col_i[b][lane + 64 * j];
+    }
+    eliminate(__builtin_amdgcn_readfirstlane(sh.piv[kk]), fr, fi, sh.rcp_r[kk], sh.rcp_i[kk], -1);
+  };
+  // column kk factored by its owner (register ca) and published in buffer b
+  auto factor = [&](int ca, int kk, int b) {
+    const int k = k0 + kk;
     unsigned key = 0;
 #pragma unroll
     for (int j = 0; j < RPL; ++j) {
       const int r = lane + 64 * j;
-      col_r[b][r] = xr[j][cn];
-      col_i[b][r] = xi[j][cn];
-      if (pos[j] > kb && r < n) {
-        const unsigned kj = pivot_key((double)xr[j][cn], (double)xi[j][cn], r);
-        key = kj > key ? kj : key;
-      }
+      const unsigned kj = pivot_key((double)xr[j][ca], (double)xi[j][ca], r);
+      key = max(key, pos[j] >= k ? kj : 0u);
     }
     key = wave_max_bcast(key);
-    const int pn = min(511 - (int)(key & 0x1FFu), n - 1);
+    // a candidate always exists (n - k rows), so p < n; min() keeps every
+    // index inside the panel whatever the key holds
+    const int p = min(511 - (int)(key & 0x1FFu), n - 1);
+    const int pl = p & 63, pj = p >> 6;
+    T fr[RPL], fi[RPL];
+    double pvr = 0.0, pvi = 0.0;
+    int q = 0;
 #pragma unroll
     for (int j = 0; j < RPL; ++j) {
-      if (lane + 64 * j == pn) {
-        piv_r[b] = xr[j][cn];
-        piv_i[b] = xi[j][cn];
-        col_r[b][pn] = (T)0;
-        col_i[b][pn] = (T)0;
+      if (j == pj) {
+        pvr = (double)lane_read(xr[j][ca], pl);
+        pvi = (double)lane_read(xi[j][ca], pl);
+        q = __builtin_amdgcn_readlane(pos[j], pl);
       }
     }
-    if (lane == 0) key_b[b] = key;
+#pragma unroll
+    for (int j = 0; j < RPL; ++j) {
+      const bool prow = lane + 64 * j == p;
+      fr[j] = prow ? (T)0 : xr[j][ca];
+      fi[j] = prow ? (T)0 : xi[j][ca];
+      sh.col_r[b][lane + 64 * j] = fr[j];
+      sh.col_i[b][lane + 64 * j] = fi[j];
+      // interchange k <-> q: row p moves to position k, the row at k to q
+      pos[j] = prow ? k : (pos[j] == k ? q : pos[j]);
+    }
+    double vr, vi;
+    complex_recip(pvr, pvi, vr, vi);
+    if (lane == 0) {
+      sh.piv[kk] = p;
+      sh.rcp_r[kk] = vr;
+      sh.rcp_i[kk] = vi;
+      perm_l[kk] = q;
+      if ((key >> 9) == 0u) g.info[e] = 1;  // no nonzero pivot: singular
+    }
+    eliminate(p, fr, fi, vr, vi, ca);
   };
-  if (w == 0) publish(0, 0, k0 - 1);
-  __syncthreads();
 
   // The column groups run as a loop and only the CW columns of a group are
   // unrolled (register indices stay compile-time constants).
@@ -595,85 +673,29 @@ __device__ __forceinline__ void panel_cg(const PanelArgs& g, int64_t e,
     for (int ca = 0; ca < CW; ++ca) {
       const int kk = qa * CW + ca;
       if (kk < nbw) {
-        const int k = k0 + kk;
         const int buf = ca & 1;  // kk & 1 (CW is even)
-        const unsigned kmax = __builtin_amdgcn_readfirstlane(key_b[buf]);
-        // a candidate always exists (n - k rows), so p < n; min() keeps every
-        // index inside the panel whatever the key holds
-        const int p = min(511 - (int)(kmax & 0x1FFu), n - 1);
-        const double pvr = (double)piv_r[buf], pvi = (double)piv_i[buf];
-        T fr[RPL], fi[RPL];
+        const bool owner = w == qa;
+        if (kk > 0 && (ca == 0 ? w != qa - 1 : !owner)) apply(kk - 1, buf ^ 1);
+        if (owner) {
+          __builtin_amdgcn_s_setprio(3);
+          if (ca == 0 && qa > 0) {
 #pragma unroll
-        for (int j = 0; j < RPL; ++j) {
-          fr[j] = col_r[buf][lane + 64 * j];  // zero for the pivot row
-          fi[j] = col_i[buf][lane + 64 * j];
-        }
-        // this wave's part of row p and its position, read from the lane
-        // that holds them (p is uniform: register row p >> 6 of lane p & 63)
-        const int pl = p & 63, pj = p >> 6;
-        T ar[CW], ai[CW];
-        int q = 0;
+            for (int j = 0; j < RPL; ++j) pos[j] = sh.pos[lane + 64 * j];
+          }
+          factor(ca, kk, buf);
+          if (ca == CW - 1 || kk == nbw - 1) {
 #pragma unroll
-        for (int c = 0; c < CW; ++c) ar[c] = ai[c] = (T)0;
-#pragma unroll
-        for (int j = 0; j < RPL; ++j) {
-          if (j == pj) {  // uniform: a scalar branch
-#pragma unroll
-            for (int c = 0; c < CW; ++c) {
-              ar[c] = lane_read(xr[j][c], pl);
-              ai[c] = lane_read(xi[j][c], pl);
-            }
-            q = __builtin_amdgcn_readlane(pos[j], pl);
+            for (int j = 0; j < RPL; ++j) sh.pos[lane + 64 * j] = pos[j];
+            __builtin_amdgcn_s_setprio(0);
           }
         }
-        double vr, vi;
-        complex_recip(pvr, pvi, vr, vi);
-        T sr[CW], si[CW];
-#pragma unroll
-        for (int c = 0; c < CW; ++c) {
-          const double a = (double)ar[c], b = (double)ai[c];
-          sr[c] = (T)(a * vr - b * vi);
-          si[c] = (T)(a * vi + b * vr);
-        }
-        if (w == qa) {
-          // active column: -f / x_pk for the other rows, 1 (scaled at the
-          // end) for the pivot row
-          sr[ca] = (T)vr;
-          si[ca] = (T)vi;
-#pragma unroll
-          for (int j = 0; j < RPL; ++j) {
-            xr[j][ca] = (lane + 64 * j == p) ? (T)1 : (T)0;
-            xi[j][ca] = (T)0;
-          }
-        }
-#pragma unroll
-        for (int j = 0; j < RPL; ++j) {
-#pragma unroll
-          for (int c = 0; c < CW; ++c) {
-            xr[j][c] = fma(-fr[j], sr[c], fma(fi[j], si[c], xr[j][c]));
-            xi[j][c] = fma(-fr[j], si[c], fma(-fi[j], sr[c], xi[j][c]));
-          }
-        }
-        // interchange k <-> q: row p moves to position k, the row at k to q
-#pragma unroll
-        for (int j = 0; j < RPL; ++j) {
-          const int r = lane + 64 * j;
-          pos[j] = (r == p) ? k : ((pos[j] == k) ? q : pos[j]);
-        }
-        if (tid == 0) {
-          perm_l[kk] = q;
-          rcp_r[kk] = vr;
-          rcp_i[kk] = vi;
-          if ((kmax >> 9) == 0u) g.info[e] = 1;  // no nonzero pivot: singular
-        }
-        if (kk + 1 < nbw) {
-          if (w == qa + (ca + 1) / CW) publish((ca + 1) % CW, buf ^ 1, k);
-          __syncthreads();
-        }
+        __syncthreads();
       }
     }
   }
-  __syncthreads();  // perm_l and the pivot reciprocals complete
+  if (w != (nbw - 1) / CW) apply(nbw - 1, (nbw - 1) & 1);
+#pragma unroll
+  for (int j = 0; j < RPL; ++j) pos[j] = sh.pos[lane + 64 * j];
 
 #pragma unroll
   for (int j = 0; j < RPL; ++j) {
@@ -685,8 +707,8 @@ __device__ __forceinline__ void panel_cg(const PanelArgs& g, int64_t e,
       const bool pivot = st >= 0 && st < nbw;
       double ar = 1.0, ai = 0.0;
       if (pivot) {
-        ar = rcp_r[st];
-        ai = rcp_i[st];
+        ar = sh.rcp_r[st];
+        ai = sh.rcp_i[st];
       }
 #pragma unroll
       for (int c = 0; c < CW; ++c) {
@@ -1029,21 +1051,35 @@ bool narrow_update(int64_t batch) {
   return batch >= 256;
 }
 
+// f(std::integral_constant<int, R>) with R = ceil(n / 64), the rows per lane of
+// the column-group panels (n <= 512; 3 at least): rows past n would cost as
+// much as the others.
+template <typename F>
+void with_rows_per_lane(int n, const F& f) {
+  switch ((n + 63) / 64) {
+    case 8: f(std::integral_constant<int, 8>{}); break;
+    case 7: f(std::integral_constant<int, 7>{}); break;
+    case 6: f(std::integral_constant<int, 6>{}); break;
+    case 5: f(std::integral_constant<int, 5>{}); break;
+    case 4: f(std::integral_constant<int, 4>{}); break;
+    default: f(std::integral_constant<int, 3>{});
+  }
+}
+
 template <typename T, int NB>
 void launch_panel_cg(hipStream_t s, int64_t batch, int n, const PanelArgs& pa) {
+  const dim3 grid((unsigned)batch);
   if constexpr (NB == 64) {
     // eight waves of eight columns, four rows per lane (n <= 256)
-    hipLaunchKernelGGL((inv_panel_cg<T, 4, 8, 64>), dim3((unsigned)batch), dim3(512), 0, s, pa);
-    return;
+    hipLaunchKernelGGL((inv_panel_cg<T, 4, 8, 64>), grid, dim3(512), 0, s, pa);
+  } else if (inv_group_width() == 4) {
+    with_rows_per_lane(n, [&](auto r) {
+      hipLaunchKernelGGL((inv_panel_cg<T, r(), 4, 32>), grid, dim3(512), 0, s, pa);
+    });
+  } else if (n <= 256) {
+    hipLaunchKernelGGL((inv_panel_cg<T, 4, 8, 32>), grid, dim3(256), 0, s, pa);
   } else {
-    const bool narrow = inv_group_width() == 4;
-    if (n <= 256) {
-      if (narrow) hipLaunchKernelGGL((inv_panel_cg<T, 4, 4, 32>), dim3((unsigned)batch), dim3(512), 0, s, pa);
-      else hipLaunchKernelGGL((inv_panel_cg<T, 4, 8, 32>), dim3((unsigned)batch), dim3(256), 0, s, pa);
-    } else {
-      if (narrow) hipLaunchKernelGGL((inv_panel_cg<T, 8, 4, 32>), dim3((unsigned)batch), dim3(512), 0, s, pa);
-      else hipLaunchKernelGGL((inv_panel_cg<T, 8, 8, 32>), dim3((unsigned)batch), dim3(256), 0, s, pa);
-    }
+    hipLaunchKernelGGL((inv_panel_cg<T, 8, 8, 32>), grid, dim3(256), 0, s, pa);
   }
 }
 
@@ -1109,12 +1145,10 @@ void run_inverse_lookahead(hipStream_t s, int64_t batch, int n, const Mat (&B)[2
     const int64_t blocks = np + (total + 1) / 2;
     QX_REQUIRE(blocks < (int64_t(1) << 31), "inv: grid too large");
     const PanelArgs pn = panel_args(p + 1);
-    if (n <= 256)
-      hipLaunchKernelGGL((inv_step<T, 4>), dim3((unsigned)blocks), dim3(512), 0, s, pn, ur,
+    with_rows_per_lane(n, [&](auto r) {
+      hipLaunchKernelGGL((inv_step<T, r()>), dim3((unsigned)blocks), dim3(512), 0, s, pn, ur,
                          (int)batch, np, total);
-    else
-      hipLaunchKernelGGL((inv_step<T, 8>), dim3((unsigned)blocks), dim3(512), 0, s, pn, ur,
-                         (int)batch, np, total);
+    });
   }
 }
 

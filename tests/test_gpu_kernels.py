@@ -366,6 +366,36 @@ def test_singular_block_raises(device):
     _inv(device, A, X, 0)
 
 
+@pytest.mark.parametrize("n", [129, 160, 161, 191, 192, 193, 255, 257, 320, 321, 384, 385, 448, 449,
+                               511, 512])
+def test_column_panel_edges(device, n):
+    """n > 128: panels of eight waves, at the edges of the rows a lane holds (64)
+    and with full and nearly empty last panels (32).  Residual of elimination
+    with partial pivoting, 16 n eps |A| |X| (growth of a random matrix well
+    below n); the same bits with and without look-ahead; row permuted input
+    with a zero first pivot candidate; a singular matrix is reported."""
+    rng = np.random.default_rng(n)
+    a = _cplx(rng, (3, n, n))
+    a[0] = a[0][rng.permutation(n)]
+    a[:, 0, 0] = 0.0
+    A = torch.as_tensor(a, device=device)
+    outs = []
+    for look in ("1", "0"):
+        with pytest.MonkeyPatch.context() as mp:
+            mp.setenv("QX_INV_LOOKAHEAD", look)
+            X = torch.empty_like(A)
+            _inv(device, A, X, 0)
+            outs.append(X.cpu().numpy())
+    assert np.array_equal(outs[0], outs[1])
+    for e in range(3):
+        x = outs[0][e]
+        res = np.linalg.norm(x @ a[e] - np.eye(n))
+        assert res <= 16 * n * np.finfo(float).eps * np.linalg.norm(x) * np.linalg.norm(a[e])
+    A[1, :, n - 1] = 0.0
+    with pytest.raises(np.linalg.LinAlgError):
+        _inv(device, A, X, 0)
+
+
 @pytest.mark.parametrize("n", [1, 7, 8, 9, 16, 17, 31, 32, 33, 40, 63, 64, 65, 95, 96, 97, 127, 128])
 @pytest.mark.parametrize("in_place", [False, True])
 def test_whole_inverse_edges(device, n, in_place):
