@@ -51,93 +51,52 @@ constexpr int BK = 16, PAD = 1;
 typedef double d4 __attribute__((ext_vector_type(4)));
 typedef float f4 __attribute__((ext_vector_type(4)));
 
-struct GemmArgs {
-  int m, n, k;
-  double ar, ai, br, bi;
-  const z2* A;
-  int64_t sA;
-  int lda;
-  const z2* B;
-  int64_t sB;
-  int ldb;
-  z2* C;
-  int64_t sC;
-  int ldc;
-  const z2* Cin;  // beta term source (== C for the in-place form)
-  int64_t sCin;
-  int ldcin;
-  int tilesM, tilesN;
-  int beta_zero;
-  z2* Ct;  // optional second output Ct = -C^H (n x m), or null
-  int64_t sCt;
-  int ldct;
-  // optional: the beta term is Cin + E - E^H (m == n), E n x n
-  const z2* E;
-  int64_t sE;
-  int lde;
-  // optional: third output Y = Yin + ys op(A) op(B) (C may then be null)
-  double ys;
-  const z2* Yin;
-  int64_t sYin;
-  int ldyin;
+// One product of a launch: base pointers, matrix strides, leading dimensions.
+struct GemmSet {
+  const z2 *A, *B;
+  z2* C;          // null: not stored
+  const z2* Cin;  // beta term source (== C for the in-place form), or null
+  z2* Ct;         // optional second output Ct = -C^H (n x m), or null
+  const z2* E;    // optional: the beta term is Cin + E - E^H (m == n), E n x n
+  const z2* Yin;  // optional: third output Y = Yin + ys op(A) op(B)
   z2* Y;
-  int64_t sY;
-  int ldy;
-  // Up to three products of one shape in one launch: matrices half <= e <
-  // 2 half take every operand from the second set (base, matrix stride,
-  // leading dimension) at index e - half, matrices e >= 2 half from the
-  // third at e - 2 half.  Sets a launch does not use equal the first.
-  int64_t half;
-  const z2 *A2, *B2, *Cin2, *E2, *Yin2;
-  z2 *C2, *Ct2, *Y2;
-  int64_t sA2, sB2, sC2, sCin2, sCt2, sE2, sY2, sYin2;
-  int lda2, ldb2, ldc2, ldcin2, ldct2, lde2, ldy2, ldyin2;
-  const z2 *A3, *B3, *Cin3, *E3, *Yin3;
-  z2 *C3, *Ct3, *Y3;
-  int64_t sA3, sB3, sC3, sCin3, sCt3, sE3, sY3, sYin3;
-  int lda3, ldb3, ldc3, ldcin3, ldct3, lde3, ldy3, ldyin3;
+  int64_t sA, sB, sC, sCin, sCt, sE, sYin, sY;
+  int lda, ldb, ldc, ldcin, ldct, lde, ldyin, ldy;
 };
 
-// Operands of matrix e of a launch (see GemmArgs::half); uniform over a
-// workgroup.
-struct GemmPtrs {
-  const z2 *A, *B, *Cin, *E, *Yin;
-  z2 *C, *Ct, *Y;
-  int lda, ldb, ldc, ldcin, ldct, lde, ldy, ldyin;
+struct GemmArgs {
+  int m, n, k;
+  int tilesM, tilesN;
+  int beta_zero;
+  unsigned count;  // matrices of the launch (register-direct kernel)
+  double ar, ai, br, bi, ys;
+  // Up to three products of one shape in one launch: matrix e is matrix
+  // e - grp half of set grp = min(e / half, 2).
+  unsigned half;
+  GemmSet set[3];
 };
-__device__ __forceinline__ GemmPtrs gemm_ptrs(const GemmArgs& g, int64_t e) {
-  const int grp = e >= 2 * g.half ? 2 : (e >= g.half ? 1 : 0);
+
+// Operands of matrix e of a launch (see GemmArgs::half); uniform over a wave.
+__device__ __forceinline__ GemmSet gemm_ptrs(const GemmArgs& g, unsigned e) {
+  const unsigned grp = e >= 2 * g.half ? 2 : (e >= g.half ? 1 : 0);
   const int64_t l = e - grp * g.half;
-  // field of the group's set
-#define QX_SEL(f1, f2, f3) (grp == 2 ? (f3) : grp == 1 ? (f2) : (f1))
-  GemmPtrs p;
-  p.A = QX_SEL(g.A + l * g.sA, g.A2 + l * g.sA2, g.A3 + l * g.sA3);
-  p.B = QX_SEL(g.B + l * g.sB, g.B2 + l * g.sB2, g.B3 + l * g.sB3);
-  p.C = g.C ? QX_SEL(g.C + l * g.sC, g.C2 + l * g.sC2, g.C3 + l * g.sC3) : nullptr;
-  // a group without a beta term or third output has null pointers of its own
-  const z2* ci = QX_SEL(g.Cin, g.Cin2, g.Cin3);
-  p.Cin = ci ? ci + l * QX_SEL(g.sCin, g.sCin2, g.sCin3) : nullptr;
-  z2* y = QX_SEL(g.Y, g.Y2, g.Y3);
-  p.Y = y ? y + l * QX_SEL(g.sY, g.sY2, g.sY3) : nullptr;
-  p.ldy = QX_SEL(g.ldy, g.ldy2, g.ldy3);
-  p.Yin = y ? QX_SEL(g.Yin, g.Yin2, g.Yin3) + l * QX_SEL(g.sYin, g.sYin2, g.sYin3) : nullptr;
-  p.ldyin = QX_SEL(g.ldyin, g.ldyin2, g.ldyin3);
-  p.E = g.E ? QX_SEL(g.E + l * g.sE, g.E2 + l * g.sE2, g.E3 + l * g.sE3) : nullptr;
-  p.Ct = g.Ct ? QX_SEL(g.Ct + l * g.sCt, g.Ct2 + l * g.sCt2, g.Ct3 + l * g.sCt3) : nullptr;
-  p.lda = QX_SEL(g.lda, g.lda2, g.lda3);
-  p.ldb = QX_SEL(g.ldb, g.ldb2, g.ldb3);
-  p.ldc = QX_SEL(g.ldc, g.ldc2, g.ldc3);
-  p.ldcin = QX_SEL(g.ldcin, g.ldcin2, g.ldcin3);
-  p.ldct = QX_SEL(g.ldct, g.ldct2, g.ldct3);
-  p.lde = QX_SEL(g.lde, g.lde2, g.lde3);
-#undef QX_SEL
+  GemmSet p = g.set[grp];
+  p.A += l * p.sA;
+  p.B += l * p.sB;
+  // an offset only where there is an operand
+  p.C += p.C ? l * p.sC : 0;
+  p.Cin += p.Cin ? l * p.sCin : 0;
+  p.Ct += p.Ct ? l * p.sCt : 0;
+  p.E += p.E ? l * p.sE : 0;
+  p.Yin += p.Yin ? l * p.sYin : 0;
+  p.Y += p.Y ? l * p.sY : 0;
   return p;
 }
 
 // beta-term source of element (row, col) of matrix e: Cin, or Cin + E - E^H
 // with the additions in the order of the Hermitian-part kernel
 // ((E - E^H) + Cin), so that the fused form rounds like the separate pass.
-__device__ __forceinline__ z2 beta_source(const GemmPtrs& P, int row, int col) {
+__device__ __forceinline__ z2 beta_source(const GemmSet& P, int row, int col) {
   const z2 c = P.Cin[(int64_t)row * P.ldcin + col];
   if (!P.E) return c;
   const z2 a = P.E[(int64_t)row * P.lde + col], b = P.E[(int64_t)col * P.lde + row];
@@ -193,7 +152,7 @@ void zgemm_kernel(GemmArgs g) {
   const int64_t e = id / tiles;
   const int t = id - (int)(e * tiles);
   const int m0 = (t / g.tilesN) * BM, n0 = (t % g.tilesN) * BN;
-  const GemmPtrs P = gemm_ptrs(g, e);
+  const GemmSet P = gemm_ptrs(g, e);
   const z2* __restrict__ A = P.A;
   const z2* __restrict__ B = P.B;
   z2* C = P.C;
@@ -372,9 +331,9 @@ void zgemm_kernel(GemmArgs g) {
 // Each wave loads its MFMA fragments straight from global memory (through
 // L1/L2) into a ring of D register slots and multiplies k-step kk while the
 // loads for k-steps kk+1 .. kk+D-1 are in flight (one k-step = 4 values of
-// k).  The four waves of a workgroup (2 x 2) never wait for each other, so a
-// SIMD's matrix core is not idled by workgroup barriers.  Wave tile is
-// (16 TM) x (16 TN); workgroup tile (32 TM) x (32 TN).
+// k).  The waves of a workgroup never wait for each other, so a SIMD's matrix
+// core is not idled by workgroup barriers.  Wave tile is (16 TM) x (16 TN),
+// its first element (m0, n0).
 //
 // Fragment layout of v_mfma_f64_16x16x4_f64: lane l supplies
 // op(A)[row l % 16][k l / 16] and op(B)[k l / 16][col l % 16].
@@ -382,7 +341,7 @@ void zgemm_kernel(GemmArgs g) {
 // negates its imaginary part through the instruction's neg modifier (bits
 // 0, 1, 2 of the last builtin operand negate the A, B, C sources).
 //
-// CHECK = false requires m % BM == 0, n % BN == 0 and k % (4 D) == 0.
+// CHECK = false requires m % 16 TM == 0, n % 16 TN == 0 and k % (4 D) == 0.
 // CHECK = true clamps every address into the matrix (rows of A past m and
 // columns of B past n only feed outputs that are not stored); the pipelined
 // loop then covers whole groups of D full k-steps and a short tail loop the
@@ -400,21 +359,12 @@ void zgemm_kernel(GemmArgs g) {
 // in float, as zgemm_kernel<float> forms them on its LDS store; the result
 // rows follow the f32 layout.
 template <typename T, int OPA, int OPB, int SPLIT, int TM, int TN, int D, bool CHECK>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2)))
-void zgemm_reg_kernel(GemmArgs g) {
+__device__ __forceinline__ void zgemm_wave(const GemmArgs& g, const GemmSet& P, int m0, int n0) {
   constexpr bool F64 = sizeof(T) == 8;
   typedef typename MfmaTraits<T>::acc_t acc_t;
-  constexpr int BM = 32 * TM, BN = 32 * TN;
   // neg-modifier masks: s_a = -1 when op(A) = C (imag part negated), s_b ditto
   constexpr bool CA = OPA == QX_OP_C, CB = OPB == QX_OP_C;
-  const int id = xcd_remap(blockIdx.x, gridDim.x);
-  const int tiles = g.tilesM * g.tilesN;
-  const int64_t e = id / tiles;
-  const int t = id - (int)(e * tiles);
-  const int m0 = (t / g.tilesN) * BM, n0 = (t % g.tilesN) * BN;
-  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-  const int wm = w >> 1, wn = w & 1;
-  const GemmPtrs P = gemm_ptrs(g, e);
+  const int lane = threadIdx.x & 63;
   const z2* __restrict__ A = P.A;
   const z2* __restrict__ B = P.B;
   const int r16 = lane & 15, k4 = lane >> 4;
@@ -424,13 +374,13 @@ void zgemm_reg_kernel(GemmArgs g) {
   const z2* pb[TN];
 #pragma unroll
   for (int i = 0; i < TM; ++i) {
-    int row = m0 + wm * 16 * TM + i * 16 + r16;
+    int row = m0 + i * 16 + r16;
     if (CHECK) row = min(row, g.m - 1);
     pa[i] = CA ? A + row : A + (int64_t)row * P.lda;
   }
 #pragma unroll
   for (int j = 0; j < TN; ++j) {
-    int col = n0 + wn * 16 * TN + j * 16 + r16;
+    int col = n0 + j * 16 + r16;
     if (CHECK) col = min(col, g.n - 1);
     pb[j] = CB ? B + (int64_t)col * P.ldb : B + col;
   }
@@ -569,6 +519,9 @@ void zgemm_reg_kernel(GemmArgs g) {
 #pragma unroll
       for (int s = 0; s < D; ++s) {
         fetch(kb + s + D - 1, fa[(s + D - 1) % D], fb[(s + D - 1) % D]);
+        // keeps the loads ahead of the k-step: left to itself the compiler
+        // moves some of them behind it, which shortens their lead
+        __builtin_amdgcn_sched_barrier(0);
         step(fa[s], fb[s]);
       }
     }
@@ -601,8 +554,8 @@ void zgemm_reg_kernel(GemmArgs g) {
     for (int j = 0; j < TN; ++j)
 #pragma unroll
       for (int q = 0; q < 4; ++q) {
-        const int row = m0 + wm * 16 * TM + i * 16 + (F64 ? k4 + 4 * q : 4 * k4 + q);
-        const int col = n0 + wn * 16 * TN + j * 16 + r16;
+        const int row = m0 + i * 16 + (F64 ? k4 + 4 * q : 4 * k4 + q);
+        const int col = n0 + j * 16 + r16;
         if (!CHECK || (row < g.m && col < g.n)) {
           double vr, vi;
           if constexpr (SPLIT == 3) {
@@ -628,6 +581,38 @@ void zgemm_reg_kernel(GemmArgs g) {
           if (P.Ct) P.Ct[(int64_t)col * P.ldct + row] = make_double2(-outr, outi);
         }
       }
+}
+
+// The waves of a launch in order: matrix after matrix, within a matrix bands of
+// two tile rows, within a band 2 x 2 groups of tiles, so that the four waves of
+// a workgroup load every operand value twice where the tile counts are even.
+// Waves, not workgroups, are the unit of the split (they share nothing but L1):
+// a matrix takes ceil(m / 16 TM) x ceil(n / 16 TN) of them, and only its last
+// 32 rows and columns are padded, not its last 64.  96 products of n x n,
+// padded to 64 -> to 32: n = 80 25 -> 17 us, 96 30 -> 18, 132 71 -> 54,
+// 160 84 -> 64, 205 160 -> 135, 416 930 -> 777; multiples of 64 as before.
+// Half tiles for the waves at the edges (padding to 16) gained nothing: the
+// time of a wave with few MFMAs is the latency of its loads, and the four waves
+// drift apart in L1 (176: 91 -> 92 us, 161: 86 -> 90).
+template <typename T, int OPA, int OPB, int SPLIT, int TM, int TN, int D, bool CHECK>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2)))
+void zgemm_reg_kernel(GemmArgs g) {
+  const unsigned id = __builtin_amdgcn_readfirstlane(
+      4u * (unsigned)xcd_remap(blockIdx.x, gridDim.x) + (threadIdx.x >> 6));
+  const unsigned waves = g.tilesM * g.tilesN;
+  const unsigned e = id / waves;
+  if (e >= g.count) return;  // uniform over the wave; the kernel has no barrier
+  const unsigned t = id - e * waves;
+  const int band = t / (2 * g.tilesN), r = t - band * 2 * g.tilesN;
+  int tr = 2 * band, tc = r;
+  if (tr + 1 < g.tilesM) {
+    const int pairs = 2 * (g.tilesN & ~1);  // waves of whole 2 x 2 groups
+    tr += r < pairs ? (r >> 1) & 1 : r - pairs;
+    tc = r < pairs ? 2 * (r >> 2) + (r & 1) : g.tilesN - 1;
+  }
+  const int m0 = tr * 16 * TM, n0 = tc * 16 * TN;
+  const GemmSet P = gemm_ptrs(g, e);
+  zgemm_wave<T, OPA, OPB, SPLIT, TM, TN, D, CHECK>(g, P, m0, n0);
 }
 
 template <typename T, int SPLIT, int BM, int BN, int WM, int WN>
@@ -671,13 +656,14 @@ int gemm_tile(int m, int n, int64_t batch) {
 
 template <typename T, int SPLIT, int TM, int TN, int D>
 void launch_reg(hipStream_t s, int64_t batch, int opA, int opB, GemmArgs g) {
-  constexpr int BM = 32 * TM, BN = 32 * TN;
+  constexpr int BM = 16 * TM, BN = 16 * TN;
   g.tilesM = (g.m + BM - 1) / BM;
   g.tilesN = (g.n + BN - 1) / BN;
-  const int64_t blocks = batch * g.tilesM * g.tilesN;
-  QX_REQUIRE(blocks < (int64_t(1) << 31), "zgemm: grid too large");
+  g.count = (unsigned)batch;
+  const int64_t waves = batch * g.tilesM * g.tilesN;
+  QX_REQUIRE(waves < (int64_t(1) << 31), "zgemm: grid too large");
   const bool full = g.m % BM == 0 && g.n % BN == 0 && g.k % (4 * D) == 0;
-  dim3 grid((unsigned)blocks), block(256);
+  dim3 grid((unsigned)((waves + 3) / 4)), block(256);
   KernelTimer* timer = active_timer;
   hipEvent_t ev0 = nullptr;
   if (timer) timer->begin(s, &ev0);
@@ -700,8 +686,8 @@ void launch_reg(hipStream_t s, int64_t batch, int opA, int opB, GemmArgs g) {
   if (timer) timer->end(s, ev0, KernelTimer::GEMM, 8.0 * g.m * g.n * (double)g.k * batch);
 }
 
-// Shapes of the register-direct kernel, as (TM, TN, D): workgroup tile
-// (32 TM) x (32 TN), D register slots.  3M keeps three accumulator sets and
+// Shapes of the register-direct kernel, as (TM, TN, D): wave tile
+// (16 TM) x (16 TN), D register slots.  3M keeps three accumulator sets and
 // only fits 2 x 2 without spilling.
 enum RegShape { REG_2x2x4 = 0, REG_2x4x2, REG_4x2x2, REG_NSHAPES };
 
@@ -934,82 +920,17 @@ void zgemm_impl(hipStream_t s, int64_t batch, int m, int n, int k, int opA, int 
   g.ai = alpha.im;
   g.br = beta.re;
   g.bi = beta.im;
-  g.A = x.A.p;
-  g.sA = x.A.stride;
-  g.lda = x.A.ld;
-  g.B = x.B.p;
-  g.sB = x.B.stride;
-  g.ldb = x.B.ld;
-  g.C = x.C.p;
-  g.sC = x.C.stride;
-  g.ldc = x.C.ld;
-  g.Cin = x.Cin.p;
-  g.sCin = x.Cin.stride;
-  g.ldcin = x.Cin.ld;
   g.beta_zero = beta_none ? 1 : 0;
   g.ys = x.ys;
-  g.Y = x.Y.p;
-  g.sY = x.Y.stride;
-  g.ldy = x.Y.ld;
-  g.Yin = x.Yin.p;
-  g.sYin = x.Yin.stride;
-  g.ldyin = x.Yin.ld;
-  g.Ct = x.Ct.p;
-  g.sCt = x.Ct.stride;
-  g.ldct = x.Ct.ld;
-  g.E = x.E.p;
-  g.sE = x.E.stride;
-  g.lde = x.E.ld;
-  g.half = batch;
-  g.A2 = o2.A.p;
-  g.sA2 = o2.A.stride;
-  g.lda2 = o2.A.ld;
-  g.B2 = o2.B.p;
-  g.sB2 = o2.B.stride;
-  g.ldb2 = o2.B.ld;
-  g.C2 = o2.C.p;
-  g.sC2 = o2.C.stride;
-  g.ldc2 = o2.C.ld;
-  g.Cin2 = o2.Cin.p;
-  g.sCin2 = o2.Cin.stride;
-  g.ldcin2 = o2.Cin.ld;
-  g.Y2 = o2.Y.p;
-  g.sY2 = o2.Y.stride;
-  g.ldy2 = o2.Y.ld;
-  g.Yin2 = o2.Yin.p;
-  g.sYin2 = o2.Yin.stride;
-  g.ldyin2 = o2.Yin.ld;
-  g.Ct2 = o2.Ct.p;
-  g.sCt2 = o2.Ct.stride;
-  g.ldct2 = o2.Ct.ld;
-  g.E2 = o2.E.p;
-  g.sE2 = o2.E.stride;
-  g.lde2 = o2.E.ld;
-  const GemmOperands& o3 = z ? *z : x;
-  g.A3 = o3.A.p;
-  g.sA3 = o3.A.stride;
-  g.lda3 = o3.A.ld;
-  g.B3 = o3.B.p;
-  g.sB3 = o3.B.stride;
-  g.ldb3 = o3.B.ld;
-  g.C3 = o3.C.p;
-  g.sC3 = o3.C.stride;
-  g.ldc3 = o3.C.ld;
-  g.Cin3 = o3.Cin.p;
-  g.sCin3 = o3.Cin.stride;
-  g.ldcin3 = o3.Cin.ld;
-  g.Y3 = o3.Y.p;
-  g.sY3 = o3.Y.stride;
-  g.ldy3 = o3.Y.ld;
-  g.Yin3 = o3.Yin.p;
-  g.sYin3 = o3.Yin.stride;
-  g.ldyin3 = o3.Yin.ld;
-  g.Ct3 = o3.Ct.p;
-  g.sCt3 = o3.Ct.stride;
-  g.ldct3 = o3.Ct.ld;
-  g.E3 = o3.E.p;
-  g.sE3 = o3.E.stride;
-  g.lde3 = o3.E.ld;
+  g.half = (unsigned)batch;
+  const GemmOperands* of[3] = {&x, &o2, z ? z : &o2};
+  for (int a = 0; a < 3; ++a) {
+    const GemmOperands& o = *of[a];
+    g.set[a] = {o.A.p, o.B.p, o.C.p, o.Cin.p, o.Ct.p, o.E.p, o.Yin.p, o.Y.p,
+                o.A.stride, o.B.stride, o.C.stride, o.Cin.stride, o.Ct.stride, o.E.stride,
+                o.Yin.stride, o.Y.stride,
+                o.A.ld, o.B.ld, o.C.ld, o.Cin.ld, o.Ct.ld, o.E.ld, o.Yin.ld, o.Y.ld};
+  }
   const int64_t nb = ng * batch;
   const int split = gemm_split(precision);
   if (precision == QX_PREC_C64) {

@@ -366,6 +366,27 @@ def test_singular_block_raises(device):
     _inv(device, A, X, 0)
 
 
+@pytest.mark.parametrize("m,n,k", [(32, 32, 16), (96, 32, 16), (32, 160, 48), (96, 96, 96),
+                                   (97, 65, 33), (33, 161, 20), (160, 224, 64), (288, 320, 32),
+                                   (320, 257, 17)])
+@pytest.mark.parametrize("opb", [0, 2])
+def test_zgemm_wave_tiles(device, m, n, k, opb):
+    """Waves as the unit of the split: odd counts of 32-wide tiles (workgroups
+    that hold tiles of two matrices, a last band of one tile row, a last odd
+    tile column) with and without a partial tile, for an odd number of
+    matrices.  Bound: the k-term dot products, 4 k eps |A| |B|."""
+    rng = np.random.default_rng(m * 1000 + n)
+    a = _cplx(rng, (5, m, k))
+    b = _cplx(rng, (5, k, n) if opb == 0 else (5, n, k))
+    c = _cplx(rng, (5, m, n))
+    C = torch.as_tensor(c, device=device).clone()
+    _zgemm(device, torch.as_tensor(a, device=device), torch.as_tensor(b, device=device), C, 0, opb,
+           -1.0 + 0j, 1.0 + 0j, 0)
+    bo = b if opb == 0 else b.conj().transpose(0, 2, 1)
+    bound = 4 * (k + 2) * np.finfo(float).eps * (np.abs(a) @ np.abs(bo) + np.abs(c))
+    assert (np.abs(C.cpu().numpy() - (c - a @ bo)) <= bound).all()
+
+
 @pytest.mark.parametrize("n", [129, 160, 161, 191, 192, 193, 255, 257, 320, 321, 384, 385, 448, 449,
                                511, 512])
 def test_column_panel_edges(device, n):
