@@ -1,30 +1,38 @@
 // Fused selected solve for small blocks (gfx950): one workgroup per energy.
 //
-// Same algorithm, outputs and operation order as rgf_selected_solve in
-// rgf.hip (reference src/qttools/greens_function_solver/rgf.py:164-414), for
-// stacks whose blocks are all at most kSB = 32 wide and at most kSN = 16 long.
-// At such sizes every block product is a few microseconds of matrix-core
-// work, so the general path (one launch per product over the whole stack)
-// is bound by launch latency; here the whole sweep of one energy runs in one
-// workgroup of two teams of four waves (one wave of each team per SIMD),
-// with every intermediate block in a per-energy workspace that stays in L2.
+// Same algorithm, outputs and operation order as the general sweep of
+// rgf_selected_solve in rgf.hip (reference
+// src/qttools/greens_function_solver/rgf.py:164-414), for stacks whose blocks
+// are all at most kSB = 32 wide and at most kSN = 32 long.  At such sizes every
+// block product is a few microseconds of matrix-core work, so the general path
+// (one launch per product over the whole stack) is bound by launch latency;
+// here the whole sweep of one energy runs in one workgroup of two teams of
+// four waves (one wave of each team per SIMD).
 //
+// - The blocks that one step writes and the next reads stay in LDS; the forward
+//   blocks, which the backward sweep reads again, go to a per-energy workspace
+//   as well, and their lines and those of A are touched one layer ahead.
 // - Block products (sgemm): the four waves of a team each own a 16 x 16
-//   quarter of the output and load their MFMA fragments straight from
+//   quarter of the output and load their MFMA fragments straight from LDS or
 //   memory, all k-steps issued before the first v_mfma_f64_16x16x4_f64.
 //   4M or 3M split, summed over k in the same order as the batched kernels.
 // - The two teams run independent products of one step side by side: the
 //   lesser and greater chains of a layer, pairs of retarded products
-//   (rgf_small_kernel describes the schedule).  The sweep is a chain of
-//   dependent steps, each about a microsecond of one SIMD's matrix-core
-//   work behind a memory round trip and a barrier, so fewer steps make it
-//   shorter.
+//   (rgf_small_kernel describes the schedule).
 // - Block inverse (sinv): gj_invert (gj_core.h), one factoring and two update
 //   waves, the block in matrix-core registers; the other waves wait.
 // - Elementwise steps (folds, X - X^H parts, traces) as team loops whose
 //   loads are all issued before the first use.
-// - A barrier closes every step, which makes its global writes visible to
-//   the other waves of the workgroup.
+// - A barrier closes every step, which makes its writes visible to the other
+//   waves of the workgroup.
+//
+// Bound by the chain of steps: of about 65 us per layer of 32 the inverse takes
+// 17 and each of the 15 product steps 1.5 to 5, for under 1 of matrix-core
+// work.  With all blocks in L2 and 16 blocks at most, before -> now: 16
+// energies of 8 blocks of 32 677 -> 536 us, 300 of 11 blocks of 20 1101 -> 879;
+// against one launch per product: 16 of 32 x 32 2.0 ms (4.9), 512 of 32 x 32
+// 4.3 (9.4), 64 of 24 x 16 0.9 (2.6), 1024 of 16 x 32 4.2 (6.3).
+#include <algorithm>
 #include <cstdlib>
 
 #include "gj_core.h"
@@ -35,7 +43,7 @@ namespace {
 
 // (the workspace bound of rgf_workspace_bytes in rgf.hip follows these)
 constexpr int kSB = 32;   // largest block size
-constexpr int kSN = 16;   // largest block count
+constexpr int kSN = 32;   // largest block count
 constexpr int kThreads = 256;       // a team: four waves, one per SIMD
 constexpr int kSolveThreads = 512;  // the fused kernels: two teams
 
@@ -47,6 +55,7 @@ struct SLay {
 
 struct SmallArgs {
   int N, flags, NS, split;
+  int bmax, slot;  // largest block, elements of a workspace slot (bmax^2)
   int bs[kSN];
   int orb[kSN];  // first orbital of each block (density row offsets)
   int64_t n_orb;
@@ -55,12 +64,14 @@ struct SmallArgs {
   z2 *XL, *XG, *XR;
   SLay lA, lSL, lSG, lXL, lXG, lXR;
   const z2* obc[3][kSN];  // retarded, lesser, greater boundary blocks or null
-  z2* ws;                 // per energy NS slots of kSB * kSB
+  z2* ws;                 // per energy NS slots
   int* info;
   z2* current;   // (S, N - 1) or null
   z2* corner;    // (S, b_0, b_{N-1}) or null
   double* density;  // (S, n_orb) or null
 };
+
+static_assert(sizeof(SmallArgs) <= 4096, "kernel arguments");
 
 struct M {
   z2* p;
@@ -72,52 +83,88 @@ __device__ inline M blk(const z2* base, int64_t stride, int64_t e, int32_t off, 
   return M{const_cast<z2*>(base) + e * stride + off, ld};
 }
 
+constexpr int kLd = kSB + 1;  // rows of a block in LDS: columns fall into different banks
+typedef z2 LdsBlock[kSB * kLd];
+
 struct Shared {
-  GjShared<GjWhole32> winv;
+  LdsBlock blk[7];
+  union {  // the backward sweep inverts nothing
+    GjShared<GjWhole32> winv;
+    LdsBlock tail[2];
+  };
   double red[2][kSolveThreads / 64];
 };
+static_assert(sizeof(Shared) <= 160 * 1024, "LDS of a CU");
 
-// C = alpha op(A) op(B) + beta Cin, m, n, k <= 32, by one team of four waves
+// Touches the cache lines of a block that a later step reads (threads t of the
+// workgroup, each line once); the value is dropped by prefetched().
+struct Touch {
+  unsigned v = 0;
+};
+__device__ __forceinline__ void prefetch(Touch& x, int t, int lines0, M A, int elems) {
+  const int i = (t - lines0) * 8;  // 128 bytes
+  if (A.p && i >= 0 && i < elems) x.v = *reinterpret_cast<const unsigned*>(A.p + i);
+}
+__device__ __forceinline__ void prefetched(const Touch& x) { asm volatile("" ::"v"(x.v)); }
+
+// Element at a byte offset (32 bits, so that it is an address's lane part).
+__device__ __forceinline__ z2& at(z2* p, unsigned byte) {
+  return *reinterpret_cast<z2*>(reinterpret_cast<char*>(p) + byte);
+}
+
+// C = s op(A) op(B) + D, s = 1 or -1, m, n, k <= 32, by one team of four waves
 // (tt: the thread's index in the team), each wave owning a 16 x 16 quarter
-// of C; a null A or B is zero.  Every load (the fragments of all k-steps and
-// the Cin values) is issued before the first v_mfma_f64_16x16x4_f64, from
+// of C; a null A or B is zero.  D is zero, Cin, Cin + Cin2, or (E - E^H) + Cin
+// (m == n), null terms zero; C2: a second place for C.  Every load (the fragments of all k-steps
+// and the values of D) is issued before the first v_mfma_f64_16x16x4_f64, from
 // clamped addresses, with no branch between the loads.  A lane whose row of
 // A (column of B) lies outside the block feeds only output rows (columns)
 // that are not stored, so its value is left as loaded; only a partial last
 // k-step (k not a multiple of 4) has its fragments beyond k zeroed.  No
 // barrier.
+//
+// A step is bound by the instructions around its 32 MFMAs (2048 cycles): with
+// clamped indexes per element and general complex factors about 500 of them,
+// 6500 cycles a step; one clamp per k-step, byte offsets and signs took 16
+// energies of 8 blocks of 32 from 560 to 536 us.
 __device__ __forceinline__ void sgemm(int tt, int split, int m, int n, int k, int opa, int opb,
-                                      Cplx al, M A, M B, Cplx be, M Cin, M C) {
+                                      double sign, M A, M B, M Cin, M C, M C2 = M{nullptr, 0},
+                                      M Cin2 = M{nullptr, 0}, M E = M{nullptr, 0}) {
   const int w = tt >> 6, lane = tt & 63;
   const int r0 = (w >> 1) * 16, c0 = (w & 1) * 16;
   const int r16 = lane & 15, k4 = lane >> 4;
   if (r0 >= m || c0 >= n) return;
-  const bool use_b = Cin.p && (be.re != 0.0 || be.im != 0.0);
+  const int row0 = r0 + k4, col = c0 + r16;  // result element q: row row0 + 4 q
   z2 cin[4];
-  if (use_b) {
+  const bool use_d = Cin.p || Cin2.p;
+  if (use_d) {
+    const int cc = min(col, n - 1);
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
-      const int row = r0 + k4 + 4 * q, col = c0 + r16;
-      const bool ok = row < m && col < n;
-      cin[q] = Cin.p[ok ? row * Cin.ld + col : 0];
+      const int rr = min(row0 + 4 * q, m - 1);
+      cin[q] = make_double2(0.0, 0.0);
+      if (Cin.p) cin[q] = at(Cin.p, 16u * (rr * Cin.ld + cc));
+      if (Cin2.p) {
+        const z2 v = at(Cin2.p, 16u * (rr * Cin2.ld + cc));
+        cin[q] = make_double2(cin[q].x + v.x, cin[q].y + v.y);
+      }
+      if (E.p) {
+        const z2 a = at(E.p, 16u * (rr * E.ld + cc)), b = at(E.p, 16u * (cc * E.ld + rr));
+        cin[q] = make_double2((a.x - b.x) + cin[q].x, (a.y + b.y) + cin[q].y);
+      }
     }
   }
   d4 a1 = {0, 0, 0, 0}, a2 = {0, 0, 0, 0}, a3 = {0, 0, 0, 0};
   if (A.p && B.p) {
+    const unsigned sa = opa == QX_OP_N ? 16u : 16u * A.ld, sb = opb == QX_OP_N ? 16u * B.ld : 16u;
+    const unsigned ba = min(r0 + r16, m - 1) * (opa == QX_OP_N ? 16u * A.ld : 16u);
+    const unsigned bb = min(col, n - 1) * (opb == QX_OP_N ? 16u : 16u * B.ld);
     z2 fa[kSB / 4], fb[kSB / 4];
 #pragma unroll
     for (int s = 0; s < kSB / 4; ++s) {
-      const int kk = 4 * s + k4;
-      const bool oka = kk < k && r0 + r16 < m, okb = kk < k && c0 + r16 < n;
-      const int ia = opa == QX_OP_N ? (r0 + r16) * A.ld + kk : kk * A.ld + r0 + r16;
-      const int ib = opb == QX_OP_N ? kk * B.ld + c0 + r16 : (c0 + r16) * B.ld + kk;
-      fa[s] = A.p[oka ? ia : 0];
-      fb[s] = B.p[okb ? ib : 0];
-    }
-#pragma unroll
-    for (int s = 0; s < kSB / 4; ++s) {
-      if (opa != QX_OP_N) fa[s].y = -fa[s].y;
-      if (opb != QX_OP_N) fb[s].y = -fb[s].y;
+      const unsigned kk = min(4 * s + k4, k - 1);
+      fa[s] = at(A.p, ba + kk * sa);
+      fb[s] = at(B.p, bb + kk * sb);
     }
     if (k & 3) {
       const int s = k >> 2;  // the partial k-step
@@ -129,42 +176,48 @@ __device__ __forceinline__ void sgemm(int tt, int split, int m, int n, int k, in
         }
       }
     }
+    // the conjugations, as the instructions' neg modifiers (bit 0: A, 1: B)
+    const bool ca = opa != QX_OP_N, cb = opb != QX_OP_N;
 #pragma unroll
     for (int s = 0; s < kSB / 4; ++s) {
       if (4 * s < k) {
+        const z2 x = fa[s], y = fb[s];
         if (split == 3) {
-          a1 = __builtin_amdgcn_mfma_f64_16x16x4f64(fa[s].x, fb[s].x, a1, 0, 0, 0);
-          a2 = __builtin_amdgcn_mfma_f64_16x16x4f64(fa[s].y, fb[s].y, a2, 0, 0, 0);
-          a3 = __builtin_amdgcn_mfma_f64_16x16x4f64(fa[s].x + fa[s].y, fb[s].x + fb[s].y, a3,
-                                                    0, 0, 0);
+          const double xs = ca ? x.x - x.y : x.x + x.y, ys = cb ? y.x - y.y : y.x + y.y;
+          a1 = __builtin_amdgcn_mfma_f64_16x16x4f64(x.x, y.x, a1, 0, 0, 0);
+          a2 = ca != cb ? __builtin_amdgcn_mfma_f64_16x16x4f64(x.y, y.y, a2, 0, 0, 1)
+                        : __builtin_amdgcn_mfma_f64_16x16x4f64(x.y, y.y, a2, 0, 0, 0);
+          a3 = __builtin_amdgcn_mfma_f64_16x16x4f64(xs, ys, a3, 0, 0, 0);
         } else {
-          a1 = __builtin_amdgcn_mfma_f64_16x16x4f64(fa[s].x, fb[s].x, a1, 0, 0, 0);
-          a2 = __builtin_amdgcn_mfma_f64_16x16x4f64(fa[s].x, fb[s].y, a2, 0, 0, 0);
-          a1 = __builtin_amdgcn_mfma_f64_16x16x4f64(fa[s].y, fb[s].y, a1, 0, 0, 1);
-          a2 = __builtin_amdgcn_mfma_f64_16x16x4f64(fa[s].y, fb[s].x, a2, 0, 0, 0);
+          a1 = __builtin_amdgcn_mfma_f64_16x16x4f64(x.x, y.x, a1, 0, 0, 0);
+          a2 = cb ? __builtin_amdgcn_mfma_f64_16x16x4f64(x.x, y.y, a2, 0, 0, 2)
+                  : __builtin_amdgcn_mfma_f64_16x16x4f64(x.x, y.y, a2, 0, 0, 0);
+          a1 = ca == cb ? __builtin_amdgcn_mfma_f64_16x16x4f64(x.y, y.y, a1, 0, 0, 1)
+                        : __builtin_amdgcn_mfma_f64_16x16x4f64(x.y, y.y, a1, 0, 0, 0);
+          a2 = ca ? __builtin_amdgcn_mfma_f64_16x16x4f64(x.y, y.x, a2, 0, 0, 1)
+                  : __builtin_amdgcn_mfma_f64_16x16x4f64(x.y, y.x, a2, 0, 0, 0);
         }
       }
     }
   }
 #pragma unroll
   for (int q = 0; q < 4; ++q) {
-    const int row = r0 + k4 + 4 * q, col = c0 + r16;
+    const int row = row0 + 4 * q;
     if (row < m && col < n) {
-      double vr, vi;
+      double vr = a1[q], vi = a2[q];
       if (split == 3) {
         vr = a1[q] - a2[q];
         vi = a3[q] - a1[q] - a2[q];
-      } else {
-        vr = a1[q];
-        vi = a2[q];
       }
-      double outr = al.re * vr - al.im * vi, outi = al.re * vi + al.im * vr;
-      if (use_b) {
-        const z2 c = cin[q];
-        outr += be.re * c.x - be.im * c.y;
-        outi += be.re * c.y + be.im * c.x;
+      if (use_d) {
+        vr = sign < 0 ? cin[q].x - vr : cin[q].x + vr;
+        vi = sign < 0 ? cin[q].y - vi : cin[q].y + vi;
+      } else if (sign < 0) {
+        vr = -vr;
+        vi = -vi;
       }
-      C.p[row * C.ld + col] = make_double2(outr, outi);
+      at(C.p, 16u * (row * C.ld + col)) = make_double2(vr, vi);
+      if (C2.p) at(C2.p, 16u * (row * C2.ld + col)) = make_double2(vr, vi);
     }
   }
 }
@@ -309,8 +362,8 @@ __device__ __forceinline__ void strace_diff(int nt, int n, M X, M Y, M Z, M W, z
 }
 
 // In-place inverse of the block X by the workgroup.
-__device__ __forceinline__ void sinv(int n, M X, int* info, Shared& sh) {
-  gj_invert<GjWhole32>(n, X.p, X.ld, nullptr, 0, X.p, X.ld, info, sh.winv);
+__device__ __forceinline__ void sinv(int n, M X, int* info, GjShared<GjWhole32>& sh) {
+  gj_invert<GjWhole32>(n, X.p, X.ld, nullptr, 0, X.p, X.ld, info, sh);
   __syncthreads();  // the inverse is visible to the workgroup
 }
 
@@ -341,28 +394,30 @@ __global__ __launch_bounds__(kSolveThreads) void rgf_small_kernel(SmallArgs g) {
   const bool skip_lower[2] = {(g.flags & QX_SOLVE_SKIP_LOWER_L) != 0,
                               (g.flags & QX_SOLVE_SKIP_LOWER_G) != 0};
   int* info = g.info + e;
-  z2* W = g.ws + e * (int64_t)g.NS * kSB * kSB;
+  z2* W = g.ws + e * (int64_t)g.NS * g.slot;
   const int team = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 8));
   const int tt = threadIdx.x & (kThreads - 1);  // thread index in the team
   const int tq = 1 + team;                     // the team's chain: 1 lesser, 2 greater
   auto sync = [] { __syncthreads(); };
-  auto slot = [&](int s, int ld) { return M{W + (int64_t)s * kSB * kSB, ld}; };
+  auto slot = [&](int s, int ld) { return M{W + (int64_t)s * g.slot, ld}; };
   auto bs = [&](int i) { return g.bs[i]; };
-  // slots: forward x^R, x^<, x^> (0..3N-1), full G^R, G^<, G^> from the
-  // backward sweep (3N..6N-1), then temporaries (per chain where both
-  // chains need one at the same time)
+  // Workspace slots: forward x^R, x^<, x^> (0..3N-1), which the backward sweep
+  // reads again, and the temporaries of the optional terms.  Everything else
+  // stays in LDS: x^R_jj and x^R_ii in lds(0), lds(1) (swapped every layer),
+  // x^< and x^> of the current layer in lds(2), lds(3), where the forward sweep
+  // also forms t3 and the backward sweep leaves the full block, further
+  // temporaries of the two chains in lds(4), lds(5), and lds(6..8).
   auto F = [&](int q, int i) { return q * N + i; };  // q: 0 r, 1 l, 2 g
-  auto full = [&](int q, int i) { return i == N - 1 ? q * N + i : (3 + q) * N + i; };
-  const int R0 = 6 * N, T1 = R0;
-  auto T3 = [&](int q) { return R0 + q; };
-  auto T4 = [&](int q) { return R0 + 2 + q; };
-  auto T5 = [&](int q) { return R0 + 4 + q; };
-  auto T6 = [&](int q) { return R0 + 6 + q; };
-  auto TB = [&](int q) { return R0 + 8 + q; };
-  auto C4 = [&](int q) { return R0 + 10 + q; };
-  auto CT = [&](int q) { return R0 + 12 + q; };
-  const int B1 = R0 + 15, B2 = R0 + 16, B3 = R0 + 17, B4 = R0 + 18, C1 = R0 + 19,
-            GC0 = R0 + 20, GC1 = R0 + 21, GCT = R0 + 22;  // 6 N + 23 slots
+  const int R0 = 3 * N;
+  auto T4 = [&](int q) { return R0 + q; };
+  auto T5 = [&](int q) { return R0 + 2 + q; };
+  auto C4 = [&](int q) { return R0 + 4 + q; };
+  auto CT = [&](int q) { return R0 + 6 + q; };
+  const int PG = R0 + 9, B3 = R0 + 10, C1 = R0 + 11, GC0 = R0 + 12, GC1 = R0 + 13,
+            GCT = R0 + 14;  // 3 N + 15 slots
+  auto lds = [&](int k) { return M{k < 7 ? sh.blk[k] : sh.tail[k - 7], kLd}; };
+  auto XQ = [&](int q) { return lds(1 + q); };
+  auto PQ = [&](int q) { return lds(3 + q); };
   auto Ad = [&](int i) { return blk(g.A, g.sA, e, g.lA.diag[i], bs(i)); };
   auto Au = [&](int i) { return blk(g.A, g.sA, e, g.lA.up[i], bs(i + 1)); };   // (i, i+1)
   auto Al = [&](int i) { return blk(g.A, g.sA, e, g.lA.lo[i], bs(i)); };       // (i+1, i)
@@ -392,69 +447,77 @@ __global__ __launch_bounds__(kSolveThreads) void rgf_small_kernel(SmallArgs g) {
 
   // ---- block 0 (rgf.py:207-231) ----
   {
-    const M X0 = slot(F(0, 0), b0);
+    const M X0 = lds(0), t3 = XQ(tq), t6 = PQ(tq);
     saxpby(threadIdx.x, kSolveThreads, b0, b0, kOneS, Ad(0), kMinusS, obc(0, 0), X0);
     sync();
-    sinv(b0, X0, info, sh);
-    const M t3 = slot(T3(tq), b0), t6 = slot(T6(tq), b0);
+    sinv(b0, X0, info, sh.winv);
     saxpby(tt, kThreads, b0, b0, kOneS, Sd(tq, 0), kOneS, obc(tq, 0), t3);
-    if (g.corner && team == 0) saxpby(tt, kThreads, b0, b0, kOneS, X0, kZeroS, none, slot(gc_cur, kSB));
+    if (g.corner && team == 0) saxpby(tt, kThreads, b0, b0, kOneS, X0, kZeroS, none, slot(gc_cur, g.bmax));
     sync();
-    sgemm(tt, sp, b0, b0, b0, QX_OP_N, QX_OP_N, kOneS, X0, t3, kZeroS, none, t6);
+    sgemm(tt, sp, b0, b0, b0, QX_OP_N, QX_OP_N, 1.0, X0, t3, none, t6);
+    saxpby(threadIdx.x, kSolveThreads, b0, b0, kOneS, X0, kZeroS, none, slot(F(0, 0), b0));
     sync();
-    sgemm(tt, sp, b0, b0, b0, QX_OP_N, QX_OP_C, kOneS, t6, X0, kZeroS, none, slot(F(tq, 0), b0));
+    sgemm(tt, sp, b0, b0, b0, QX_OP_N, QX_OP_C, 1.0, t6, X0, none, XQ(tq),
+          slot(F(tq, 0), b0));
     sync();
   }
 
   // ---- forward sweep (rgf.py:234-295) ----
   for (int i = 0; i + 1 < N; ++i) {
     const int j = i + 1, bi = bs(i), bj = bs(j);
-    const M Xri = slot(F(0, i), bi), Xrj = slot(F(0, j), bj), t1 = slot(T1, bi);
+    const M Xri = lds(i & 1), Xrj = lds(j & 1), t1 = lds(6);
     const bool ob0 = obc(0, j).p != nullptr;
+    Touch touch;  // the blocks of A of the next layer
+    if (j + 1 < N) {
+      prefetch(touch, threadIdx.x, 0, Al(j), bs(j + 1) * bj);
+      prefetch(touch, threadIdx.x, 128, Au(j), bj * bs(j + 1));
+      prefetch(touch, threadIdx.x, 256, Ad(j + 1), bs(j + 1) * bs(j + 1));
+    }
     // team 0: a_ji x^R_ii, then x^R_jj's argument a_jj - a_ji x^R_ii a_ij;
-    // team 1 meanwhile: a_ji x^<_ii, then a_ji x^>_ii (and the boundary folds)
+    // team 1 meanwhile: a_ji x^<_ii, then a_ji x^>_ii
 #pragma unroll 1
     for (int s = 0; s < 2; ++s) {
       if (team == 0) {
         if (s == 0) {
-          sgemm(tt, sp, bj, bi, bi, QX_OP_N, QX_OP_N, kOneS, Al(i), Xri, kZeroS, none, t1);
+          sgemm(tt, sp, bj, bi, bi, QX_OP_N, QX_OP_N, 1.0, Al(i), Xri, none, t1);
           if (ob0) saxpby(tt, kThreads, bj, bj, kOneS, Ad(j), kMinusS, obc(0, j), Xrj);
+        } else if (ob0) {
+          sgemm(tt, sp, bj, bj, bi, QX_OP_N, QX_OP_N, -1.0, t1, Au(i), Xrj, Xrj);
         } else {
-          sgemm(tt, sp, bj, bj, bi, QX_OP_N, QX_OP_N, kMinusS, t1, Au(i), kOneS,
-                ob0 ? Xrj : Ad(j), Xrj);
+          sgemm(tt, sp, bj, bj, bi, QX_OP_N, QX_OP_N, -1.0, t1, Au(i), Ad(j), Xrj);
         }
       } else {
-        const int q = 1 + s;
-        sgemm(tt, sp, bj, bi, bi, QX_OP_N, QX_OP_N, kOneS, Al(i), slot(F(q, i), bi), kZeroS, none,
-              slot(T4(q), bi));
-        if (obc(q, j).p)
-          saxpby(tt, kThreads, bj, bj, kOneS, Sd(q, j), kOneS, obc(q, j), slot(T3(q), bj));
+        sgemm(tt, sp, bj, bi, bi, QX_OP_N, QX_OP_N, 1.0, Al(i), XQ(1 + s), none,
+              PQ(1 + s));
       }
       sync();
     }
     // each chain: t3 = a_ji x_ii a_ji^H + s_jj (+ boundary); team 0 also the
     // corner's g_c a_ij
-    const M t3 = slot(T3(tq), bj), t5 = slot(T5(tq), bj), t6 = slot(T6(tq), bj);
-    sgemm(tt, sp, bj, bj, bi, QX_OP_N, QX_OP_C, kOneS, slot(T4(tq), bi), Al(i), kOneS,
-          obc(tq, j).p ? t3 : Sd(tq, j), t3);
+    const M t3 = XQ(tq), t5 = PQ(tq), t6 = PQ(tq);
+    sgemm(tt, sp, bj, bj, bi, QX_OP_N, QX_OP_C, 1.0, PQ(tq), Al(i), Sd(tq, j), t3, none,
+          obc(tq, j));
     if (g.corner && team == 0)
-      sgemm(tt, sp, b0, bj, bi, QX_OP_N, QX_OP_N, kOneS, slot(gc_cur, kSB), Au(i), kZeroS, none,
-            slot(GCT, kSB));
+      sgemm(tt, sp, b0, bj, bi, QX_OP_N, QX_OP_N, 1.0, slot(gc_cur, g.bmax), Au(i), none,
+            slot(GCT, g.bmax));
     sync();
     if (Su(1, i).p || Su(2, i).p) {
       const M sij = Su(tq, i);
-      if (sij.p) sgemm(tt, sp, bj, bj, bi, QX_OP_N, QX_OP_N, kOneS, t1, sij, kZeroS, none, t5);
+      if (sij.p) sgemm(tt, sp, bj, bj, bi, QX_OP_N, QX_OP_N, 1.0, t1, sij, none, t5);
       sync();
       if (sij.p) sherm(tt, kThreads, bj, bj, 1.0, -1.0, t5, 1.0, t5, t3);  // t3 += t5^H - t5
       sync();
     }
-    sinv(bj, Xrj, info, sh);
-    sgemm(tt, sp, bj, bj, bj, QX_OP_N, QX_OP_N, kOneS, Xrj, t3, kZeroS, none, t6);
+    sinv(bj, Xrj, info, sh.winv);
+    sgemm(tt, sp, bj, bj, bj, QX_OP_N, QX_OP_N, 1.0, Xrj, t3, none, t6);
+    saxpby(threadIdx.x, kSolveThreads, bj, bj, kOneS, Xrj, kZeroS, none, slot(F(0, j), bj));
     sync();
-    sgemm(tt, sp, bj, bj, bj, QX_OP_N, QX_OP_C, kOneS, t6, Xrj, kZeroS, none, slot(F(tq, j), bj));
+    sgemm(tt, sp, bj, bj, bj, QX_OP_N, QX_OP_C, 1.0, t6, Xrj, none, XQ(tq),
+          slot(F(tq, j), bj));
     if (g.corner && team == 1)
-      sgemm(tt, sp, b0, bj, bj, QX_OP_N, QX_OP_N, kMinusS, slot(GCT, kSB), Xrj, kZeroS, none,
-            slot(gc_nxt, kSB));
+      sgemm(tt, sp, b0, bj, bj, QX_OP_N, QX_OP_N, -1.0, slot(GCT, g.bmax), Xrj, none,
+            slot(gc_nxt, g.bmax));
+    prefetched(touch);
     sync();
     if (g.corner) {
       const int t = gc_cur;
@@ -464,17 +527,18 @@ __global__ __launch_bounds__(kSolveThreads) void rgf_small_kernel(SmallArgs g) {
   }
 
   // ---- last diagonal blocks (rgf.py:297-305), the corner ----
+  int rj = (N - 1) & 1;  // LDS block of the full x^R_jj
   {
     const int bn = bs(N - 1);
-    const M Xq = slot(F(tq, N - 1), bn), od = Od(tq, N - 1);
+    const M Xq = XQ(tq), od = Od(tq, N - 1);
     if (g.density && team == 0) sdiag_imag(tt, kThreads, bn, Xq, g.density + e * g.n_orb + g.orb[N - 1]);
     if (od.p) sherm(tt, kThreads, bn, bn, 0.0, 0.5, Xq, -0.5, Xq, od);
     if (want_r && team == 0) {
       const M xr = blk(g.XR, g.sXR, e, g.lXR.diag[N - 1], bn);
-      if (xr.p) saxpby(tt, kThreads, bn, bn, kOneS, slot(F(0, N - 1), bn), kZeroS, none, xr);
+      if (xr.p) saxpby(tt, kThreads, bn, bn, kOneS, lds(rj), kZeroS, none, xr);
     }
     if (g.corner && team == 1)
-      saxpby(tt, kThreads, b0, bl, kOneS, slot(gc_cur, kSB), kZeroS, none,
+      saxpby(tt, kThreads, b0, bl, kOneS, slot(gc_cur, g.bmax), kZeroS, none,
              M{g.corner + e * (int64_t)b0 * bl, bl});
     sync();
   }
@@ -482,70 +546,81 @@ __global__ __launch_bounds__(kSolveThreads) void rgf_small_kernel(SmallArgs g) {
   // ---- backward sweep (rgf.py:308-404) ----
   for (int i = N - 2; i >= 0; --i) {
     const int j = i + 1, bi = bs(i), bj = bs(j);
-    const M Xri = slot(F(0, i), bi), Xrj = slot(full(0, j), bj);
-    const M Aij = Au(i), Aji = Al(i);
-    const M b1 = slot(B1, bj), b2 = slot(B2, bi), b3 = slot(B3, bj), b4 = slot(B4, bi);
-    if (team == 0)
-      sgemm(tt, sp, bi, bj, bi, QX_OP_N, QX_OP_N, kOneS, Xri, Aij, kZeroS, none, b1);  // xr_ii a_ij
-    else
-      sgemm(tt, sp, bj, bi, bj, QX_OP_N, QX_OP_N, kOneS, Xrj, Aji, kZeroS, none, b2);  // xr_jj a_ji
-    sync();
-    if (team == 0)
-      sgemm(tt, sp, bi, bj, bj, QX_OP_N, QX_OP_N, kOneS, b1, Xrj, kZeroS, none, b3);  // b1 xr_jj
-    else
-      sgemm(tt, sp, bi, bi, bj, QX_OP_N, QX_OP_N, kOneS, b1, b2, kZeroS, none, b4);  // b1 b2
-    sync();
-
     const bool any_s = Su(1, i).p || Su(2, i).p;
     const M sij = Su(tq, i);
+    const M Xri = slot(F(0, i), bi), Xrj = lds(rj), Zr = lds(1 - rj);
+    const M Aij = Au(i), Aji = Al(i);
+    const M b1 = lds(6), b2 = lds(7), b3 = slot(B3, bj), b4 = lds(8);
+    Touch touch, touch2;  // what the next layer reads
+    if (i > 0) {
+      const int h = i - 1, eh = bs(h) * bs(h);
+      prefetch(touch, threadIdx.x, 0, Al(h), bi * bs(h));
+      prefetch(touch, threadIdx.x, 128, Au(h), bs(h) * bi);
+      prefetch(touch, threadIdx.x, 256, slot(F(0, h), bs(h)), eh);
+      prefetch(touch, threadIdx.x, 384, slot(F(1, h), bs(h)), eh);
+      prefetch(touch2, threadIdx.x, 0, slot(F(2, h), bs(h)), eh);
+    }
+    if (team == 0)
+      sgemm(tt, sp, bi, bj, bi, QX_OP_N, QX_OP_N, 1.0, Xri, Aij, none, b1);  // xr_ii a_ij
+    else
+      sgemm(tt, sp, bj, bi, bj, QX_OP_N, QX_OP_N, 1.0, Xrj, Aji, none, b2);  // xr_jj a_ji
+    sync();
+    if (team == 1)
+      sgemm(tt, sp, bi, bi, bj, QX_OP_N, QX_OP_N, 1.0, b1, b2, none, b4);  // b1 b2
+    else if (any_s || (want_r && want_r_off))
+      sgemm(tt, sp, bi, bj, bj, QX_OP_N, QX_OP_N, 1.0, b1, Xrj, none, b3);  // b1 xr_jj
+    sync();
+
     if (want_cur) {
       // layer current from the forward blocks of layer i and the full blocks
       // of layer j (rgf.py:381-400): tl = a_ji x_ii a_ji^H (+ the Σ_ij terms)
       const M c1 = slot(C1, bi), t4 = slot(T4(tq), bi), tl = slot(CT(tq), bj),
               c4 = slot(C4(tq), bj);
-      sgemm(tt, sp, bj, bi, bi, QX_OP_N, QX_OP_N, kOneS, Aji, slot(F(tq, i), bi), kZeroS, none, t4);
-      if (team == 0)
-        sgemm(tt, sp, bj, bi, bi, QX_OP_N, QX_OP_N, kOneS, Aji, Xri, kZeroS, none, c1);  // a_ji xr_ii
+      sgemm(tt, sp, bj, bi, bi, QX_OP_N, QX_OP_N, 1.0, Aji, slot(F(tq, i), bi), none, t4);
+      if (any_s && team == 0)
+        sgemm(tt, sp, bj, bi, bi, QX_OP_N, QX_OP_N, 1.0, Aji, Xri, none, c1);  // a_ji xr_ii
       sync();
-      sgemm(tt, sp, bj, bj, bi, QX_OP_N, QX_OP_C, kOneS, t4, Aji, kZeroS, none, tl);
+      sgemm(tt, sp, bj, bj, bi, QX_OP_N, QX_OP_C, 1.0, t4, Aji, none, tl);
       sync();
       if (any_s) {
-        if (sij.p) sgemm(tt, sp, bj, bj, bi, QX_OP_N, QX_OP_N, kOneS, c1, sij, kZeroS, none, c4);
+        if (sij.p) sgemm(tt, sp, bj, bj, bi, QX_OP_N, QX_OP_N, 1.0, c1, sij, none, c4);
         sync();
         if (sij.p) sherm(tt, kThreads, bj, bj, 1.0, -1.0, c4, 1.0, c4, tl);
         sync();
       }
-      strace_diff(kSolveThreads, bj, slot(CT(2), bj), slot(full(1, j), bj), slot(full(2, j), bj),
-                  slot(CT(1), bj), g.current + e * (int64_t)(N - 1) + i, sh);
+      strace_diff(kSolveThreads, bj, slot(CT(2), bj), XQ(1), XQ(2), slot(CT(1), bj),
+                  g.current + e * (int64_t)(N - 1) + i, sh);
     }
 
     // each chain (q = tq): G_ii, G_ij and the outputs
     const int q = tq;
-    const M Xi = slot(F(q, i), bi), Xj = slot(full(q, j), bj);
-    const M t1 = slot(TB(q), bi), t5 = slot(T5(q), bj), P = slot(T6(q), bj);
-    const M Z = slot(full(q, i), bi), Zr = slot(full(0, i), bi);
+    const M Xi = slot(F(q, i), bi), Xj = XQ(q), t1 = PQ(q), t5 = slot(T5(q), bj), Z = XQ(q);
+    // P of the lesser chain replaces b4, P of the greater chain x^R_jj, unless
+    // a Σ_ij term needs that below
+    const M P = q == 1 ? b4 : any_s ? slot(PG, bj) : Xrj;
     // temp_1x = B4 x_ii; team 0 also G^R_ii = xr_ii + B4 xr_ii
-    sgemm(tt, sp, bi, bi, bi, QX_OP_N, QX_OP_N, kOneS, b4, Xi, kZeroS, none, t1);
-    if (team == 0) sgemm(tt, sp, bi, bi, bi, QX_OP_N, QX_OP_N, kOneS, b4, Xri, kOneS, Xri, Zr);
+    sgemm(tt, sp, bi, bi, bi, QX_OP_N, QX_OP_N, 1.0, b4, Xi, none, t1);
+    if (team == 0) sgemm(tt, sp, bi, bi, bi, QX_OP_N, QX_OP_N, 1.0, b4, Xri, Xri, Zr);
     sync();
     if (any_s) {  // temp_1x -= xr_ii s_ij B3^H
-      if (sij.p) sgemm(tt, sp, bi, bj, bi, QX_OP_N, QX_OP_N, kOneS, Xri, sij, kZeroS, none, t5);
+      if (sij.p) sgemm(tt, sp, bi, bj, bi, QX_OP_N, QX_OP_N, 1.0, Xri, sij, none, t5);
       sync();
-      if (sij.p) sgemm(tt, sp, bi, bi, bj, QX_OP_N, QX_OP_C, kMinusS, t5, b3, kOneS, t1, t1);
+      if (sij.p) sgemm(tt, sp, bi, bi, bj, QX_OP_N, QX_OP_C, -1.0, t5, b3, t1, t1);
       sync();
     }
-    // x_ii' = x_ii + (temp_1x - temp_1x^H); P = -temp_2x = -B1 x_jj
-    sherm(tt, kThreads, bi, bi, 0.0, 1.0, t1, -1.0, t1, Z, 1.0, Xi);
-    sgemm(tt, sp, bi, bj, bj, QX_OP_N, QX_OP_N, kMinusS, b1, Xj, kZeroS, none, P);
+    sgemm(tt, sp, bi, bj, bj, QX_OP_N, QX_OP_N, -1.0, b1, Xj, none, P);  // -temp_2x
     sync();
-    // x_ii' += temp_2x B1^H;  x_ij = -temp_2x - x_ii B2^H (+ xr_ii s_ij xr_jj^H)
+    // x_ii' = x_ii + (temp_1x - temp_1x^H) + temp_2x B1^H;
+    // x_ij = -temp_2x - x_ii B2^H (+ xr_ii s_ij xr_jj^H)
     M Oij = Ou(q, i);
     if (!Oij.p) Oij = slot(T4(q), bj);
-    sgemm(tt, sp, bi, bi, bj, QX_OP_N, QX_OP_C, kMinusS, P, b1, kOneS, Z, Z);
-    sgemm(tt, sp, bi, bj, bi, QX_OP_N, QX_OP_C, kMinusS, Xi, b2, kOneS, P, Oij);
+    sgemm(tt, sp, bi, bi, bj, QX_OP_N, QX_OP_C, -1.0, P, b1, Xi, Z, none, none, t1);
+    sgemm(tt, sp, bi, bj, bi, QX_OP_N, QX_OP_C, -1.0, Xi, b2, P, Oij);
+    prefetched(touch);
+    prefetched(touch2);
     sync();
     if (any_s) {
-      if (sij.p) sgemm(tt, sp, bi, bj, bj, QX_OP_N, QX_OP_C, kOneS, t5, Xrj, kOneS, Oij, Oij);
+      if (sij.p) sgemm(tt, sp, bi, bj, bj, QX_OP_N, QX_OP_C, 1.0, t5, Xrj, Oij, Oij);
       sync();
     }
     // outputs: x_ji = -x_ij^H, the diagonal block, the density; team 0 the
@@ -558,12 +633,17 @@ __global__ __launch_bounds__(kSolveThreads) void rgf_small_kernel(SmallArgs g) {
       const M xr = blk(g.XR, g.sXR, e, g.lXR.diag[i], bi);
       if (xr.p) saxpby(tt, kThreads, bi, bi, kOneS, Zr, kZeroS, none, xr);
     }
-    if (want_r && want_r_off && team == 1) {
-      const M up = blk(g.XR, g.sXR, e, g.lXR.up[i], bj), lo = blk(g.XR, g.sXR, e, g.lXR.lo[i], bi);
-      if (up.p) saxpby(tt, kThreads, bi, bj, kMinusS, b3, kZeroS, none, up);
-      if (lo.p) sgemm(tt, sp, bj, bi, bi, QX_OP_N, QX_OP_N, kMinusS, b2, Xri, kZeroS, none, lo);
+    if (want_r && want_r_off) {
+      if (team == 1) {
+        const M up = blk(g.XR, g.sXR, e, g.lXR.up[i], bj), lo = blk(g.XR, g.sXR, e, g.lXR.lo[i], bi);
+        if (up.p) saxpby(tt, kThreads, bi, bj, kMinusS, b3, kZeroS, none, up);
+        if (lo.p) sgemm(tt, sp, bj, bi, bi, QX_OP_N, QX_OP_N, -1.0, b2, Xri, none, lo);
+      }
+      sync();  // before b2 and b3 are formed again
     }
-    sync();
+    // (otherwise the next layer's first products write only b1 and b2, which
+    // nobody reads here)
+    rj = 1 - rj;
   }
 }
 
@@ -571,6 +651,7 @@ __global__ __launch_bounds__(kSolveThreads) void rgf_small_kernel(SmallArgs g) {
 // rgf.hip), one workgroup per energy.
 struct SmallInvArgs {
   int N, NS, split;
+  int slot;  // elements of a workspace slot
   int bs[kSN];
   int64_t sA, sX;
   const z2* A;
@@ -586,16 +667,16 @@ struct SmallInvArgs {
 // sweep x_ji and x_ij run one per team.
 template <int SP>
 __global__ __launch_bounds__(kSolveThreads) void rgf_small_inv_kernel(SmallInvArgs g) {
-  __shared__ Shared sh;
+  __shared__ GjShared<GjWhole32> sh;
   const int64_t e = blockIdx.x;
   const int N = g.N;
   constexpr int sp = SP;
   int* info = g.info + e;
-  z2* W = g.ws + e * (int64_t)g.NS * kSB * kSB;
+  z2* W = g.ws + e * (int64_t)g.NS * g.slot;
   const int team = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 8));
   const int tt = threadIdx.x & (kThreads - 1);
   auto sync = [] { __syncthreads(); };
-  auto slot = [&](int s, int ld) { return M{W + (int64_t)s * kSB * kSB, ld}; };
+  auto slot = [&](int s, int ld) { return M{W + (int64_t)s * g.slot, ld}; };
   auto bs = [&](int i) { return g.bs[i]; };
   // slots: forward x_ii (0..N-1), full X_ii from the backward sweep
   // (N..2N-1; block N-1 keeps its forward slot), temporaries
@@ -620,12 +701,12 @@ __global__ __launch_bounds__(kSolveThreads) void rgf_small_inv_kernel(SmallInvAr
     const M t1 = slot(T1, bi), Xj = slot(F(j), bj);
     const bool ob = obc(j).p != nullptr;
     if (team == 0)
-      sgemm(tt, sp, bj, bi, bi, QX_OP_N, QX_OP_N, kOneS, Al(i), slot(F(i), bi), kZeroS, none, t1);
+      sgemm(tt, sp, bj, bi, bi, QX_OP_N, QX_OP_N, 1.0, Al(i), slot(F(i), bi), none, t1);
     else if (ob)
       saxpby(tt, kThreads, bj, bj, kOneS, Ad(j), kMinusS, obc(j), Xj);
     sync();
     if (team == 0)
-      sgemm(tt, sp, bj, bj, bi, QX_OP_N, QX_OP_N, kMinusS, t1, Au(i), kOneS, ob ? Xj : Ad(j), Xj);
+      sgemm(tt, sp, bj, bj, bi, QX_OP_N, QX_OP_N, -1.0, t1, Au(i), ob ? Xj : Ad(j), Xj);
     sync();
     sinv(bj, Xj, info, sh);
   }
@@ -645,19 +726,19 @@ __global__ __launch_bounds__(kSolveThreads) void rgf_small_inv_kernel(SmallInvAr
     const M up = blk(g.X, g.sX, e, g.lX.up[i], bj);
     // x_ji = -(x_jj a_ji) x_ii on team 0, x_ij = -(x_ii a_ij) x_jj on team 1
     if (team == 0)
-      sgemm(tt, sp, bj, bi, bj, QX_OP_N, QX_OP_N, kOneS, Xjj, Al(i), kZeroS, none, t1);
+      sgemm(tt, sp, bj, bi, bj, QX_OP_N, QX_OP_N, 1.0, Xjj, Al(i), none, t1);
     else
-      sgemm(tt, sp, bi, bj, bi, QX_OP_N, QX_OP_N, kOneS, Xii, Au(i), kZeroS, none, t2);
+      sgemm(tt, sp, bi, bj, bi, QX_OP_N, QX_OP_N, 1.0, Xii, Au(i), none, t2);
     sync();
     if (team == 0)
-      sgemm(tt, sp, bj, bi, bi, QX_OP_N, QX_OP_N, kMinusS, t1, Xii, kZeroS, none, Xji);
+      sgemm(tt, sp, bj, bi, bi, QX_OP_N, QX_OP_N, -1.0, t1, Xii, none, Xji);
     else if (up.p)
-      sgemm(tt, sp, bi, bj, bj, QX_OP_N, QX_OP_N, kMinusS, t2, Xjj, kZeroS, none, up);
+      sgemm(tt, sp, bi, bj, bj, QX_OP_N, QX_OP_N, -1.0, t2, Xjj, none, up);
     sync();
     // x_ii <- x_ii - x_ii a_ij x_ji
     const M Z = slot(full(i), bi);
     if (team == 0)
-      sgemm(tt, sp, bi, bi, bj, QX_OP_N, QX_OP_N, kMinusS, t2, Xji, kOneS, Xii, Z);
+      sgemm(tt, sp, bi, bi, bj, QX_OP_N, QX_OP_N, -1.0, t2, Xji, Xii, Z);
     sync();
     const M xd = blk(g.X, g.sX, e, g.lX.diag[i], bi);
     if (xd.p) saxpby(threadIdx.x, kSolveThreads, bi, bi, kOneS, Z, kZeroS, none, xd);
@@ -690,7 +771,7 @@ bool fits32(const qx_btd_layout* l, int N) {
 
 // Fused path of rgf_selected_solve for small blocks; returns false (and does
 // nothing) when the call is not eligible: complex128 arithmetic (4M or 3M),
-// at most 16 blocks of at most 32, offsets below 2^31, and QX_RGF_FUSED not 0.
+// at most 32 blocks of at most 32, offsets below 2^31, and QX_RGF_FUSED not 0.
 bool rgf_small_solve(qx_handle* h, hipStream_t st, const qx_btd_layout* la, const void* a,
                      const qx_btd_layout* lsl, const void* sl, const qx_btd_layout* lsg,
                      const void* sg, const void* const* obc_r, const void* const* obc_l,
@@ -715,7 +796,9 @@ bool rgf_small_solve(qx_handle* h, hipStream_t st, const qx_btd_layout* la, cons
   SmallArgs g;
   g.N = N;
   g.flags = (int)flags;
-  g.NS = 6 * N + 23;
+  g.NS = 3 * N + 15;
+  g.bmax = *std::max_element(la->block_sizes, la->block_sizes + N);
+  g.slot = g.bmax * g.bmax;
   g.split = prec == QX_PREC_C128_3M ? 3 : 4;
   int off = 0;
   for (int i = 0; i < kSN; ++i) {
@@ -746,7 +829,7 @@ bool rgf_small_solve(qx_handle* h, hipStream_t st, const qx_btd_layout* la, cons
   for (int q = 0; q < 3; ++q)
     for (int i = 0; i < kSN; ++i)
       g.obc[q][i] = (ob[q] && i < N) ? static_cast<const z2*>(ob[q][i]) : nullptr;
-  g.ws = static_cast<z2*>(h->ensure_ws((size_t)S * g.NS * kSB * kSB * sizeof(z2)));
+  g.ws = static_cast<z2*>(h->ensure_ws((size_t)S * g.NS * g.slot * sizeof(z2)));
   g.info = h->ensure_info(S);
   g.current = static_cast<z2*>(current);
   g.corner = static_cast<z2*>(corner);
@@ -798,6 +881,8 @@ bool rgf_small_inv(qx_handle* h, hipStream_t st, const qx_btd_layout* la, const 
   SmallInvArgs g;
   g.N = N;
   g.NS = 2 * N + 3;
+  const int bmax = *std::max_element(la->block_sizes, la->block_sizes + N);
+  g.slot = bmax * bmax;
   g.split = prec == QX_PREC_C128_3M ? 3 : 4;
   for (int i = 0; i < kSN; ++i) {
     g.bs[i] = i < N ? la->block_sizes[i] : 0;
@@ -809,7 +894,7 @@ bool rgf_small_inv(qx_handle* h, hipStream_t st, const qx_btd_layout* la, const 
   g.X = static_cast<z2*>(x);
   g.lA = make_lay(la, N);
   g.lX = make_lay(lx, N);
-  g.ws = static_cast<z2*>(h->ensure_ws((size_t)S * g.NS * kSB * kSB * sizeof(z2)));
+  g.ws = static_cast<z2*>(h->ensure_ws((size_t)S * g.NS * g.slot * sizeof(z2)));
   g.info = h->ensure_info(S);
   KernelTimer* timer = active_timer;
   hipEvent_t ev0 = nullptr;

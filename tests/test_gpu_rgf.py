@@ -544,6 +544,44 @@ def test_fused_small_block_path_matches_general(device, monkeypatch, precision):
         assert np.max(np.abs(got - ref)) <= 1e-12 * scale
 
 
+@pytest.mark.parametrize("block_sizes", [[3, 1], [5, 20, 32, 1, 31, 17, 8, 4], [6, 7] * 8 + [5],
+                                         [9, 4, 32, 3] * 8, [2] * 33],
+                         ids=["2", "8", "17", "32", "33"])
+@pytest.mark.parametrize("sigma", ["diagonal", "tridiagonal"])
+@pytest.mark.parametrize("offdiag", [False, True])
+def test_fused_equals_per_product_lengths(device, monkeypatch, block_sizes, sigma, offdiag):
+    """The fused kernel's blocks in LDS, whose places depend on the parity of
+    the layer, on Sigma off-diagonal blocks and on the optional outputs, up to
+    its largest block count (32; 33 takes the per-product path both times).
+    Same products in the same order but for the sums of the general sweep:
+    bound of the two-path test above."""
+    bs = np.array(block_sizes)
+    n, ne = len(bs), 3
+    coo = sps.coo_matrix(_bt_full(bs, seed=3 + n))
+    off = np.concatenate([[0], np.cumsum(bs)])
+    b = coo - coo.conj().T
+    if sigma == "diagonal":
+        b = sps.block_diag([b.tocsr()[o:p, o:p] for o, p in zip(off[:-1], off[1:])])
+    oa = ODSDBCOO.from_sparray(coo, bs, (ne,))
+    ob = ODSDBCOO.from_sparray(sps.coo_matrix(b), bs, (ne,))
+    gobc = OBCBlocks(n)
+    gobc.retarded[n - 1] = torch.full((ne, bs[-1], bs[-1]), 0.02 + 0.03j, dtype=torch.complex128,
+                                      device=device)
+    gobc.greater[0] = torch.full((ne, bs[0], bs[0]), -0.1j, dtype=torch.complex128, device=device)
+    outs = {}
+    for fused in ("1", "0"):
+        monkeypatch.setenv("QX_RGF_FUSED", fused)
+        a, bl, bg = to_gpu(oa, device), to_gpu(ob, device), to_gpu(ob, device)
+        corner = torch.zeros((ne, bs[0], bs[-1]), dtype=torch.complex128, device=device)
+        dens = torch.zeros((ne, int(bs.sum())), dtype=torch.float64, device=device)
+        xl, xg, xr, cur = RGF(100, retarded_offdiag=offdiag).selected_solve(
+            a, bl, bg, obc_blocks=gobc, return_retarded=True, return_current=True,
+            corner=corner, density=dens)
+        outs[fused] = [t.cpu().numpy() for t in (xl.data, xg.data, xr.data, cur, corner, dens)]
+    for got, ref in zip(outs["1"], outs["0"]):
+        assert np.max(np.abs(got - ref)) <= 1e-12 * np.max(np.abs(ref))
+
+
 @pytest.mark.parametrize("block_sizes", [[7], [1, 1], [32, 5], [1, 32, 1], [16] * 16,
                                          [32] * 3 + [1]],
                          ids=["N1", "b1x2", "32-5", "1-32-1", "16x16", "32x3-1"])
