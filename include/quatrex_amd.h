@@ -293,8 +293,8 @@ int qx_zgemm_ozaki(qx_handle* handle, void* stream, int64_t batch, int m, int n,
 #define QX_GEMM_LDS_128 128
 
 /* Execution tuning of a handle (no counterpart in the reference): streams =
- * concurrent sub-batches of one RGF call (1..8, default 4, env
- * QX_RGF_STREAMS); gemm_tile = one of QX_GEMM_* (env QX_ZGEMM_TILE,
+ * concurrent sub-batches of one RGF call at most (1..8, default 4, env
+ * QX_RGF_STREAMS; fewer where a block product of the call is small); gemm_tile = one of QX_GEMM_* (env QX_ZGEMM_TILE,
  * QX_ZGEMM_KERNEL and QX_ZGEMM_REG override it).  Used by the autotuner and
  * by callers that run several handles side by side. */
 int qx_set_tuning(qx_handle* handle, int streams, int gemm_tile);

@@ -171,9 +171,20 @@ thread_local int active_gemm_tile = 0;
 
 thread_local int split_part = 0;
 
-void run_split(qx_handle* h, hipStream_t st, int64_t S,
+// One sub-batch per 512 waves of a block product (32 x 32 tiles, half the
+// chip's SIMDs; a step launches two or three products at once): below that the
+// streams' launches cost more than their overlap gains, above it the inverses
+// of one hide behind the products of another.  1 / 4 sub-batches, measured
+// (solves, ms): 32 x 48 (energies x block, 64 waves a product) 1.9 / 2.5,
+// 64 x 64 (256) 2.4 / 3.5, 8 x 256 (512) 5.4 / 6.6, 128 x 64 (512) 2.9 / 3.9,
+// 256 x 64 (1024) 4.28 / 4.79 (2: 4.42), 64 x 128 (1024) 7.16 / 7.13 (2: 7.10),
+// 48 x 176 (1728) 17.1 / 16.0, 128 x 128 (2048) 7.8 / 7.1, 64 x 256 (4096)
+// 209 / 203.
+void run_split(qx_handle* h, hipStream_t st, int64_t S, int b,
                const std::function<void(hipStream_t, int64_t, int64_t)>& f) {
-  int P = (int)std::min<int64_t>(h->parts, std::max<int64_t>(1, S / 4));
+  const int64_t tiles = (b + 31) / 32, waves = S * tiles * tiles;
+  const int64_t most = std::min<int64_t>(S / 4, waves / 512);
+  const int P = (int)std::min<int64_t>(h->parts, std::max<int64_t>(1, most));
   if (P <= 1) {
     f(st, 0, S);
     return;

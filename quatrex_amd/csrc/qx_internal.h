@@ -314,12 +314,12 @@ extern thread_local int active_gemm_tile;
 // qx_inv_batched_noalloc (once per device; called by qx_create).
 void noalloc_init(int device);
 
-// Splits a batch of S matrices into up to `handle->parts` contiguous
-// sub-batches and runs f(stream, e0, n) for each concurrently: sub-batch 0 on
+// Splits a batch of S matrices (blocks of at most b) into up to
+// `handle->parts` contiguous sub-batches and runs f(stream, e0, n) for each concurrently: sub-batch 0 on
 // the caller's stream `st` in this thread, the others on handle-owned streams
 // from helper host threads.  Events order all sub-batches after the work
 // already queued on `st`, and `st` waits for all of them before returning.
-void run_split(qx_handle* h, hipStream_t st, int64_t S,
+void run_split(qx_handle* h, hipStream_t st, int64_t S, int b,
                const std::function<void(hipStream_t, int64_t, int64_t)>& f);
 // Index of the sub-batch the calling thread runs inside run_split (0 on the
 // caller's thread).

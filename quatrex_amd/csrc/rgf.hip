@@ -239,7 +239,7 @@ void rgf_selected_inv(qx_handle* h, hipStream_t st0, const qx_btd_layout* la,
   // arithmetic, unless the output shares memory with A; the other arithmetics
   // keep the reference's sequence of products
   const bool keep = (prec == QX_PREC_C128 || prec == QX_PREC_C128_3M) && !A0.overlaps(X0);
-  run_split(h, st0, Stot, [&](hipStream_t st, int64_t e0, int64_t S) {
+  run_split(h, st0, Stot, bmax, [&](hipStream_t st, int64_t e0, int64_t S) {
     const OzSubBatch oz(prec, oz_region, bmax, e0, S);
     const Btd A = A0.sub(e0), X = X0.sub(e0);
     const Slots W{ws, Stot, (int64_t)bmax * bmax, e0};
@@ -413,7 +413,7 @@ void rgf_selected_solve(qx_handle* h, hipStream_t st0, const qx_btd_layout* la,
   if (stagger) QX_HIP_CHECK(hipEventCreateWithFlags(&stg_ev, hipEventDisableTiming));
   std::promise<void> stg_set;
   std::shared_future<void> stg_ready = stg_set.get_future().share();
-  run_split(h, st0, Stot, [&](hipStream_t st, int64_t e0, int64_t S) {
+  run_split(h, st0, Stot, bmax, [&](hipStream_t st, int64_t e0, int64_t S) {
   const OzSubBatch oz(prec, oz_region, bmax, e0, S);
   const int part = split_part;
   // sub-batch 0 releases the others once its first inverse is enqueued, or
