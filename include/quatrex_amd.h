@@ -195,6 +195,14 @@ int qx_inv_batched_noalloc(qx_handle* handle, void* stream, int64_t batch, int n
                            int lds, int64_t stride_s, void* x, int ldx,
                            int64_t stride_x, int* info, int precision);
 
+/* x[e, q] = inv(sum_n w[n, q] a_n[e]) for batch systems and nq contour nodes
+ * (operator.py:113-179, w[n, q] = z_q^n).  a, stride_a: host arrays of n_terms
+ * (1..8) device stacks of d x d matrices and their matrix strides (0: one
+ * matrix for all systems); w: device, n_terms x nq; x: batch x nq x d x d. */
+int qx_operator_inverse(qx_handle* handle, void* stream, int64_t batch, int nq,
+                        int d, int n_terms, const void* const* a,
+                        const int64_t* stride_a, const void* w, void* x);
+
 /* Sancho-Rubio surface Green's function on (n, b, b) stacks.  Replaces
  * SanchoRubio.__call__ (src/qttools/boundary_conditions/obc/sancho_rubio.py:33-86):
  * batch-global stop when max_e ||(|alpha|+|beta|)||_F / 2 < tol.  Writes

@@ -73,7 +73,7 @@ EXPORTED_SYMBOLS = (
     "qx_sync_check", "qx_rgf_selected_inv", "qx_rgf_selected_solve", "qx_zgemm_batched",
     "qx_inv_batched", "qx_sancho_rubio", "qx_beyn_moments", "qx_timer_start", "qx_timer_stop",
     "qx_contact_self_energy", "qx_assemble_system_matrix", "qx_set_tuning", "qx_zgemm_ozaki",
-    "qx_inv_batched_noalloc", "qx_svd_batched", "qx_spectral_modes",
+    "qx_inv_batched_noalloc", "qx_svd_batched", "qx_spectral_modes", "qx_operator_inverse",
 )
 
 
@@ -140,6 +140,8 @@ def load() -> ctypes.CDLL:
             i64, ctypes.POINTER(f64), vp, i32, i64, i32]
         lib.qx_inv_batched.argtypes = [vp, vp, i64, i32, vp, i32, i64, vp, i32, i64, vp, i32,
                                        i64, i32]
+        lib.qx_operator_inverse.argtypes = [vp, vp, i64, i32, i32, i32, ctypes.POINTER(vp),
+                                            ctypes.POINTER(i64), vp, vp]
         lib.qx_inv_batched_noalloc.argtypes = [vp, vp, i64, i32, vp, i32, i64, vp, i32, i64,
                                                vp, i32, i64, vp, i32]
         lib.qx_svd_batched.argtypes = [vp, vp, i64, i32, i32, vp, i32, i64, vp, vp, vp, i32, f64,

@@ -569,6 +569,27 @@ int qx_inv_batched(qx_handle* h, void* stream, int64_t batch, int n, const void*
   });
 }
 
+int qx_operator_inverse(qx_handle* h, void* stream, int64_t batch, int nq, int d, int n_terms,
+                        const void* const* a, const int64_t* stride_a, const void* w, void* x) {
+  return guarded(h, [&]() {
+    QX_REQUIRE(h, "null handle");
+    QX_REQUIRE(batch >= 0 && nq >= 0 && d >= 1 && d <= qx::kInvMaxN, "operator: bad sizes");
+    QX_REQUIRE(a && stride_a && w && x, "operator: null argument");
+    const int64_t n = batch * nq, dd = (int64_t)d * d;
+    if (n == 0) return QX_OK;
+    int* info = h->ensure_info(n);
+    qx::z2* ws = static_cast<qx::z2*>(h->ensure_ws((size_t)(n * dd) * sizeof(qx::z2) +
+                                                   (size_t)(n * 3 * d) * sizeof(int)));
+    const qx::InvScratch scr{ws, dd, reinterpret_cast<int*>(ws + n * dd), 3 * (int64_t)d};
+    const hipStream_t st = static_cast<hipStream_t>(stream);
+    // the operators are formed where the inverse starts
+    const qx::Mat X(x, dd, d), T = qx::zinv_input(d, X, scr, QX_PREC_C128);
+    qx::operator_stack(st, batch, nq, d, n_terms, a, stride_a, w, T);
+    qx::zinv(st, n, d, T, qx::Mat(), X, info, QX_PREC_C128, scr);
+    return QX_OK;
+  });
+}
+
 int qx_sancho_rubio(qx_handle* h, void* stream, int64_t n, int b, const void* a_ii,
                     const void* a_ij, const void* a_ji, void* x_ii, int max_iterations, double tol,
                     int* iterations) {

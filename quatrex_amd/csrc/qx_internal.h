@@ -281,6 +281,11 @@ void max_value(hipStream_t s, int64_t n, const double* v, double* out);
 void contour_operator(hipStream_t s, int64_t batch, int nq, int b,
                       const Mat& aji, const Mat& aii, const Mat& aij,
                       const z2* z, const Mat& T);
+// T[e nq + q] = sum_n w[n nq + q] a_n[e], nt terms (host arrays of device
+// pointers and matrix strides, ld d; w on the device)
+constexpr int kOperatorTerms = 8;
+void operator_stack(hipStream_t s, int64_t batch, int nq, int d, int nt, const void* const* a,
+                    const int64_t* stride, const void* w, const Mat& T);
 // q0 += sum_q w0[q] Tinv[e, q]; q1 += sum_q w1[q] Tinv[e, q]
 void contour_accumulate(hipStream_t s, int64_t batch, int nq, int b,
                         const Mat& Tinv, const z2* w0, const z2* w1,

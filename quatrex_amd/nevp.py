@@ -93,7 +93,30 @@ def operator_inverse(a_xx, z, contour_type=None, in_type=None, num_threads: int 
         t = as_device(a, dev)
         dev = t.device
         ts.append(t)
-    zt = torch.as_tensor(np.asarray(z), dtype=torch.complex128, device=dev)
+    zc = torch.as_tensor(np.asarray(z), dtype=torch.complex128)
+    nb = max(t.shape[0] for t in ts) if ts and all(t.ndim == 4 for t in ts) else 0
+    d = ts[0].shape[-1] if nb else 0
+    # The operators in one pass, written where the inverse starts: stacks of
+    # square matrices with their nodes along the second axis, up to the inverse's
+    # largest size; any other broadcast takes the general sums below.
+    if (nb > 0 and len(ts) <= 8 and 1 <= d <= 512 and zc.ndim == 4 and zc.numel() > 0
+            and zc.shape == (1, zc.shape[1], 1, 1) and zc.shape[1] <= 65535
+            and dev.type == "cuda"
+            and all(type(t) is torch.Tensor and t.dtype == torch.complex128 and t.device == dev
+                    and t.shape in ((nb, 1, d, d), (1, 1, d, d)) and t.is_contiguous()
+                    and not t.is_conj() and not t.is_neg() for t in ts)):
+        nq = zc.shape[1]
+        w = torch.stack([zc.reshape(nq) ** n for n in range(-b, len(ts) - b)]).to(dev)
+        ptrs = (ctypes.c_void_p * len(ts))(*[t.data_ptr() for t in ts])
+        strides = (ctypes.c_int64 * len(ts))(*[d * d if t.shape[0] > 1 else 0 for t in ts])
+        out = torch.empty((nb, nq, d, d), dtype=torch.complex128, device=dev)
+        h, st = _lib.handle(dev), _lib.stream_ptr(dev)
+        rc = _lib.load().qx_operator_inverse(h, st, nb, nq, d, len(ts), ptrs, strides,
+                                             w.data_ptr(), out.data_ptr())
+        _lib.check(rc, h, "inv")
+        _lib.sync_check(dev, "inv")
+        return out
+    zt = zc.to(dev)
     op = sum(zt ** n * a for a, n in zip(ts, range(-b, b + 1)))
     return inv(op.contiguous())
 

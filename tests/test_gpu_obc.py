@@ -88,6 +88,33 @@ def test_obc_system_matches_oracle(device, mode):
         assert np.allclose(np_(r), rr, rtol=1e-3, atol=1e-9)
 
 
+@pytest.mark.parametrize("d,nq,terms", [(1, 1, 3), (33, 7, 3), (96, 8, 5), (129, 9, 3), (160, 17, 8)])
+@pytest.mark.parametrize("shared", [False, True])
+def test_operator_inverse_one_pass(device, d, nq, terms, shared):
+    """The operators formed in one pass (nodes in groups of eight, the first
+    stack shared by all systems or not) against the sums term by term, which
+    other layouts take; diagonally dominant at every node, so that the two
+    roundings of the operator differ by a few eps of the inverse."""
+    rng = np.random.default_rng(d + nq)
+    b = terms // 2
+    a = [0.1 * (rng.standard_normal((3, 1, d, d)) + 1j * rng.standard_normal((3, 1, d, d))) / d
+         for _ in range(terms)]
+    a[b] = a[b] + 4.0 * np.eye(d)
+    if shared:
+        a[0] = a[0][:1]
+    z = 1.2 * np.exp(2j * np.pi * np.arange(nq) / nq).reshape(1, nq, 1, 1)
+    ts = [torch.as_tensor(x, device=device) for x in a]
+    got = np_(operator_inverse(tuple(ts), z))
+    ref = np_(operator_inverse(tuple(t.transpose(-1, -2).contiguous().transpose(-1, -2)
+                                     for t in ts), z))
+    op = sum(z ** n * x for x, n in zip(a, range(-b, b + 1)))
+    assert got.shape == (3, nq, d, d)
+    assert rel_err(got, np.linalg.inv(op)) < 1e-12
+    assert rel_err(got, ref) < 1e-13
+    with pytest.raises(np.linalg.LinAlgError):
+        operator_inverse(tuple(torch.zeros_like(t) for t in ts), z)
+
+
 def test_operator_inverse(device):
     rng = np.random.default_rng(0)
     a_xx = tuple(rng.random((3, 1, 6, 6)) + 1j * rng.random((3, 1, 6, 6)) for _ in range(3))
