@@ -67,7 +67,7 @@ int sancho_rubio(qx_handle* h, hipStream_t st, int64_t n, int b, const void* a_i
   // their own: none is copied
   Mat eps(a_ii, bb, b), eps_s = eps, eps_inv = eps;
   Mat alpha(a_ji, bb, b), beta(a_ij, bb, b), na = M(5), nb = M(6);
-  const Mat start = zinv_input(b, g, scr, prec);
+  const Mat start = zinv_input(n, b, g, scr, prec);
   bool converged = false;
   for (int it = 0; it < max_iter && !converged; ++it) {
     if (iters) *iters = it + 1;
@@ -583,7 +583,7 @@ int qx_operator_inverse(qx_handle* h, void* stream, int64_t batch, int nq, int d
     const qx::InvScratch scr{ws, dd, reinterpret_cast<int*>(ws + n * dd), 3 * (int64_t)d};
     const hipStream_t st = static_cast<hipStream_t>(stream);
     // the operators are formed where the inverse starts
-    const qx::Mat X(x, dd, d), T = qx::zinv_input(d, X, scr, QX_PREC_C128);
+    const qx::Mat X(x, dd, d), T = qx::zinv_input(n, d, X, scr, QX_PREC_C128);
     qx::operator_stack(st, batch, nq, d, n_terms, a, stride_a, w, T);
     qx::zinv(st, n, d, T, qx::Mat(), X, info, QX_PREC_C128, scr);
     return QX_OK;

@@ -1232,20 +1232,32 @@ void launch_whole(hipStream_t s, int64_t batch, int n, const Mat& A, const Mat& 
 }  // namespace
 
 // Panel width: 32 columns; with the older panel kernels 16 above n = 256
-// (where two rows per thread double their per-column work).  QX_INV_NB=16|32|64
-// overrides for n <= 256 (16 runs the one-thread-per-row kernel; 64 the
-// column-group panel of eight waves of eight columns, whose rank-64 updates
-// pass over the matrix half as often).
-int inv_panel_width(int n) {
+// (where two rows per thread double their per-column work).  From 160 matrices
+// on the updates stream every matrix through HBM, and 64-column panels (eight
+// waves of eight columns, n <= 256) halve the passes over it: 256 x 256^2
+// 1.64 -> 1.40 ms, 160 x 256^2 1.16 -> 1.03, 256 x 192^2 0.80 -> 0.69, 256 x
+// 208^2 1.23 -> 1.17; not where the last panel would be nearly empty (300 x
+// 200^2 1.43 -> 1.56) or the matrix has fewer than three (512 x 160^2 1.05 ->
+// 1.13), nor below 160 matrices, where the look-ahead of the 32-column panels
+// wins (128 x 192^2 0.46 against 0.48), nor above 256, one panel per CU, where
+// the longer panels take a second round (384 x 256^2 2.31 -> 2.27, 640 x 256^2
+// 3.70 -> 3.62: not worth another order of summation).
+// QX_INV_NB=16|32|64 overrides for n <= 256 (16 runs the one-thread-per-row
+// kernel).
+int inv_panel_width(int64_t batch, int n, int precision) {
   const int forced_nb = forced_panel_width();
   if (n > 256) return inv_panel_kind() == 0 ? 32 : 16;
   if (forced_nb == 64 && inv_panel_kind() != 0) return 32;
-  return forced_nb ? forced_nb : 32;
+  if (forced_nb) return forced_nb;
+  const bool wide = batch >= 160 && batch <= 256 && n >= 192 && (n + 63) / 64 * 64 - n <= 48;
+  return wide && precision != QX_PREC_C64 && inv_panel_kind() == 0 && inv_group_width() == 4
+             ? 64
+             : 32;
 }
 
-Mat zinv_input(int n, const Mat& X, const InvScratch& scr, int precision) {
+Mat zinv_input(int64_t batch, int n, const Mat& X, const InvScratch& scr, int precision) {
   if (precision != QX_PREC_C64 && n <= inv_whole_max()) return X;
-  const int NB = inv_panel_width(n);
+  const int NB = inv_panel_width(batch, n, precision);
   const int npan = (n + NB - 1) / NB;
   // the panels ping-pong between X and the scratch buffer, the last one
   // writing the scratch buffer: an odd count starts in X, an even one in it
@@ -1276,7 +1288,7 @@ void zinv(hipStream_t s, int64_t batch, int n, const Mat& A, const Mat& S, const
     return;
   }
 
-  const int NB = inv_panel_width(n);
+  const int NB = inv_panel_width(batch, n, precision);
   const bool big = n > 256 && NB == 16;
   const int npan = (n + NB - 1) / NB;
   // start in the buffer that makes the last panel write the scratch buffer

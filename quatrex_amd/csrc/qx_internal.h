@@ -194,7 +194,7 @@ void spectral_modes(hipStream_t s, int64_t n, int b, int m, const z2* ws, const 
 // X = inv(A - S) with partial pivoting (S may be zero).  info[e] is set to a
 // nonzero value for an exactly singular matrix.  n <= kInvMaxN.  The scratch
 // holds, per matrix, an n x n complex buffer (buf + e * buf_stride) and 3 n
-// ints (ints + e * int_stride); A may alias X, or be zinv_input(n, X, scr, precision);
+// ints (ints + e * int_stride); A may alias X, or be zinv_input(batch, n, X, scr, precision);
 // X may not alias buf.
 constexpr int kInvMaxN = 512;
 struct InvScratch {
@@ -211,7 +211,7 @@ void zinv(hipStream_t s, int64_t batch, int n, const Mat& A, const Mat& S,
 // The buffer an inverse into X starts from (X itself or the scratch buffer):
 // a matrix formed there and passed as A (S zero) is inverted into X without
 // the initial copy.  precision: that of the inverse.
-Mat zinv_input(int n, const Mat& X, const InvScratch& scr, int precision);
+Mat zinv_input(int64_t batch, int n, const Mat& X, const InvScratch& scr, int precision);
 
 // Elementwise helpers on batched m x n blocks.
 // Y = a*A + b*B            (A, B may be zero matrices)

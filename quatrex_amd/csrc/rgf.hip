@@ -130,7 +130,7 @@ struct OzSubBatch {
 // entries are of the order of the FP32 rounding error and would be lost in
 // FP32), the small correction X R by the FP32 GEMM.  Mc and R are n x n
 // temporaries.
-// X = inv(M) for M in Ain, which is X or zinv_input(n, X, scr, ..): the products
+// X = inv(M) for M in Ain, which is X or zinv_input(S, n, X, scr, ..): the products
 // that form M write it there, so the inverse starts without a copy.
 //
 // Safety net of the mixed mode: since I - M X1 = (I - M X0)^2 for the
@@ -261,7 +261,7 @@ void rgf_selected_inv(qx_handle* h, hipStream_t st0, const qx_btd_layout* la,
 
     // Forward sweep (rgf.py:70-92).
     {
-      const Mat X0 = W.get(xd[0], bs(0)), M0 = zinv_input(bs(0), X0, scr, ip);
+      const Mat X0 = W.get(xd[0], bs(0)), M0 = zinv_input(S, bs(0), X0, scr, ip);
       fold(st, S, bs(0), bs(0), A.diag(0), -1.0, OR.get(0, bs(0)), M0);
       block_inv(st, S, bs(0), M0, X0, info, prec, scr, W.get(N + 6, bs(0)), W.get(N + 7, bs(0)),
                 mask);
@@ -270,7 +270,7 @@ void rgf_selected_inv(qx_handle* h, hipStream_t st0, const qx_btd_layout* la,
       const int j = i + 1, bi = bs(i), bj = bs(j);
       const Mat T1 = kept(i).zero() ? W.get(t1, bi) : kept(i);
       zgemm(st, S, bj, bi, bi, QX_OP_N, QX_OP_N, kOne, A.lower(i), W.get(xd[i], bi), kZero, T1, gp);
-      const Mat Xj = W.get(xd[j], bj), Mj = zinv_input(bj, Xj, scr, ip);
+      const Mat Xj = W.get(xd[j], bj), Mj = zinv_input(S, bj, Xj, scr, ip);
       Mat Ajj = A.diag(j);
       if (!OR.get(j, bj).zero()) {
         fold(st, S, bj, bj, A.diag(j), -1.0, OR.get(j, bj), Mj);
@@ -503,7 +503,7 @@ void rgf_selected_solve(qx_handle* h, hipStream_t st0, const qx_btd_layout* la,
   // ---- block 0 (rgf.py:207-231) ----
   {
     const int b0 = bs(0);
-    const Mat X0 = W.get(sr[0], b0), M0 = zinv_input(b0, X0, scr, ip);
+    const Mat X0 = W.get(sr[0], b0), M0 = zinv_input(S, b0, X0, scr, ip);
     fold(st, S, b0, b0, A.diag(0), -1.0, OR.get(0, b0), M0);
     block_inv(st, S, b0, M0, X0, info, prec, scr, W.get(NS1, b0), W.get(NS2, b0), mask);
     if (release.p) {
@@ -563,7 +563,7 @@ void rgf_selected_solve(qx_handle* h, hipStream_t st0, const qx_btd_layout* la,
     }
     // xr_jj = inv(a_jj - obc - a_ji xr_ii a_ij), the argument formed where
     // the inverse starts
-    const Mat Mj = zinv_input(bj, Xrj, scr, ip);
+    const Mat Mj = zinv_input(S, bj, Xrj, scr, ip);
     Mat Ajj = A.diag(j);
     if (!OR.get(j, bj).zero()) {
       fold(st, S, bj, bj, A.diag(j), -1.0, OR.get(j, bj), Mj);

@@ -366,6 +366,32 @@ def test_singular_block_raises(device):
     _inv(device, A, X, 0)
 
 
+@pytest.mark.parametrize("batch,n", [(159, 192), (160, 192), (161, 191), (160, 208), (256, 207),
+                                     (300, 255), (160, 256), (512, 193)])
+def test_wide_panel_rule(device, batch, n):
+    """Both sides of the line between 32- and 64-column panels (matrices per
+    call, size, filling of the last panel): residual of elimination with
+    partial pivoting, 16 n eps |A| |X|, and the 32-column panels to the
+    conditioning of the matrices times eps."""
+    g = torch.Generator(device=device).manual_seed(batch + n)
+    A = torch.randn((batch, n, n), dtype=torch.complex128, device=device, generator=g)
+    A[:, 0, 0] = 0.0
+    outs = []
+    for nb in (None, "32"):
+        with pytest.MonkeyPatch.context() as mp:
+            if nb:
+                mp.setenv("QX_INV_NB", nb)
+            X = torch.empty_like(A)
+            _inv(device, A, X, 0)
+            outs.append(X)
+    eps = np.finfo(float).eps
+    for e in (0, batch // 2, batch - 1):
+        a, x = A[e].cpu().numpy(), outs[0][e].cpu().numpy()
+        kappa = np.linalg.norm(a) * np.linalg.norm(x)
+        assert np.linalg.norm(x @ a - np.eye(n)) <= 16 * n * eps * kappa
+        assert rel_err(x, outs[1][e].cpu().numpy()) <= 32 * n * eps * kappa
+
+
 @pytest.mark.parametrize("m,n,k", [(32, 32, 16), (96, 32, 16), (32, 160, 48), (96, 96, 96),
                                    (97, 65, 33), (33, 161, 20), (160, 224, 64), (288, 320, 32),
                                    (320, 257, 17)])
