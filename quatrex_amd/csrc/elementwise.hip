@@ -458,7 +458,7 @@ struct TraceArgs {
 // coalesced.  The partial sums of a matrix's row tiles go to `part` and are
 // added in order by trace_sum_kernel, so a result does not depend on how many
 // matrices share the launch.  (One workgroup per matrix with strided reads of
-// Y and W: 282 us for 12 matrices of 176; 48 n^2.. 64 n^2 bytes are streamed.)
+// Y and W: 282 us for 12 matrices of 176; 64 n^2 bytes are streamed.)
 __global__ __launch_bounds__(NT) void trace_kernel(TraceArgs g, int tn, z2* part, int64_t sp) {
   __shared__ z2 ty_[TS][TS + 1], tw_[TS][TS + 1];
   __shared__ double red[NT / 64];

@@ -18,9 +18,10 @@
 // Why one wave per matrix: a column is a serial chain (pivot search, exchange
 // of the pivot row, reciprocal, elimination) of about 110 instructions at one
 // row per lane, each 4 cycles of issue.  Eight waves that share the columns
-// repeat the reciprocal and the exchange in every wave (2500 cycles per
-// column at 256 rows); four waves that share the rows pay two dependent LDS
-// round trips and a barrier per column (1600 cycles).
+// repeat the exchange in every wave (1850 to 2700 cycles per column at 256
+// rows, the owner of the next column one ahead); four waves that share the
+// rows pay two dependent LDS round trips and a barrier per column (1600
+// cycles).
 #pragma once
 
 #include "qx_internal.h"
