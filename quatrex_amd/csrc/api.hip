@@ -90,9 +90,7 @@ int sancho_rubio(qx_handle* h, hipStream_t st, int64_t n, int b, const void* a_i
     zgemm_triple(st, n, b, b, b, QX_OP_N, QX_OP_N, kOne, kOne, ab, aa, bb2, prec);
     zgemm_one(st, n, b, b, b, QX_OP_N, QX_OP_N, kOne, kOne, ba, prec);
     absnorm2(st, n, b, na, nb, dnorm);
-    max_value(st, n, dnorm, h->word_dev);
-    QX_HIP_CHECK(hipMemcpyAsync(h->word_host, h->word_dev, sizeof(double), hipMemcpyDeviceToHost,
-                                st));
+    max_value(st, n, dnorm, h->word_host);  // pinned: no copy between kernel and wait
     QX_HIP_CHECK(hipStreamSynchronize(st));
     converged = *static_cast<volatile double*>(h->word_host) / 2.0 < tol;
     // the couplings of the next iteration; the caller's are never written
