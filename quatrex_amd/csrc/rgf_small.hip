@@ -854,7 +854,7 @@ bool rgf_small_solve(qx_handle* h, hipStream_t st, const qx_btd_layout* la, cons
       const double bi = la->block_sizes[i], bj = la->block_sizes[i + 1];
       fl += 3.0 * cube(bj, bi, bi) + 3.0 * cube(bj, bj, bi) + 4.0 * cube(bj, bj, bj)  // forward
             + cube(bj, bj, bj)                                                          // inverse
-            + cube(bi, bj, bi) + cube(bj, bi, bj) + cube(bi, bj, bj) + cube(bi, bi, bj)  // b1..b4
+            + cube(bi, bj, bi) + cube(bj, bi, bj) + cube(bi, bi, bj)  // b1, b2, b4
             + 3.0 * cube(bi, bi, bi) + 2.0 * cube(bi, bj, bj) + 2.0 * cube(bi, bi, bj) +
             2.0 * cube(bi, bj, bi);
     }
