@@ -372,6 +372,8 @@ void rgf_selected_solve(qx_handle* h, hipStream_t st0, const qx_btd_layout* la,
   QX_REQUIRE(N >= 1, "selected_solve: need at least one block");
   if (Stot == 0) return;
   const int bmax = block_limits(la, "selected_solve");
+  const Btd A0(la, a), SL0(lsl, sl), SG0(lsg, sg), XL0(lxl, xl), XG0(lxg, xg),
+      XR0(want_r ? lxr : nullptr, want_r ? xr : nullptr);
   if (rgf_small_solve(h, st0, la, a, lsl, sl, lsg, sg, obc_r, obc_l, obc_g, lxl, xl, lxg, xg,
                       want_r ? lxr : nullptr, want_r ? xr : nullptr, want_cur ? current : nullptr,
                       corner, density, ldos, flags, prec))
@@ -380,8 +382,6 @@ void rgf_selected_solve(qx_handle* h, hipStream_t st0, const qx_btd_layout* la,
   int* info_all = h->ensure_info(Stot);
   int* mask_all = prec == QX_PREC_MIXED ? h->ensure_mask(Stot) : nullptr;
   char* oz_region = reinterpret_cast<char*>(ws) + rgf_slot_bytes(la, true, bmax);
-  const Btd A0(la, a), SL0(lsl, sl), SG0(lsg, sg), XL0(lxl, xl), XG0(lxg, xg),
-      XR0(want_r ? lxr : nullptr, want_r ? xr : nullptr);
 
   const int gp = gemm_precision(prec), ip = inv_precision(prec);
   // The odd sub-batches start after sub-batch 0's first block inverse, so
@@ -395,9 +395,14 @@ void rgf_selected_solve(qx_handle* h, hipStream_t st0, const qx_btd_layout* la,
   // The backward sweep with three products per quantity holds for
   // skew-Hermitian Σ^≶ and is taken when the device finds them so; the check
   // needs one wait for the device, so only a caller that allows it
-  // (QX_SOLVE_SKEW_CHECK) and does not record a graph gets it.  The
+  // (QX_SOLVE_SKEW_CHECK) and does not record a graph gets it.  It reads the
+  // G^≶ output blocks of the step before, so they have to share no memory with
+  // each other or with G^R (a caller may pass one container for two quantities
+  // of which it needs one; the general sweep reads workspace slots).  The
   // reduced-precision products keep the reference's sequence.
-  bool skew_on = (flags & QX_SOLVE_SKEW_CHECK) != 0 && N > 1 && xl != xg &&
+  const bool apart = !XL0.overlaps(XG0) &&
+                     !(want_r && (XR0.overlaps(XL0) || XR0.overlaps(XG0)));
+  bool skew_on = (flags & QX_SOLVE_SKEW_CHECK) != 0 && N > 1 && apart &&
                  (prec == QX_PREC_C128 || prec == QX_PREC_C128_3M);
   if (skew_on) {
     hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;

@@ -768,3 +768,30 @@ def test_selected_inv_output_forms(device, monkeypatch, bs, form, precision):
             if 0 <= j < len(bs) and (i == j or form != "diag"):
                 assert rel_err(got[0].blocks[i, j].cpu().numpy(), ref.blocks[i, j]) < 1e-10
     assert torch.equal(torch.view_as_real(got[0].data), torch.view_as_real(got[1].data))
+
+
+@pytest.mark.parametrize("shared", ["lesser", "greater"])
+@pytest.mark.parametrize("same", ["pointer", "part"])
+@pytest.mark.parametrize("block_sizes", [[64, 40, 64, 64]], ids=["4x64"])
+def test_retarded_and_lesser_or_greater_in_one_container(device, block_sizes, shared, same):
+    """A caller that does not need one of G^<, G^> hands the container of G^R
+    for it as well: G^R, written last, and the other quantity are those of
+    separate containers.  The same where the two only share a part: the stack
+    of the unneeded quantity starts one energy later in one tensor."""
+    bs, ne = np.array(block_sizes), 6
+    a, sl, sg, obc, container, _ = _skew_case(device, bs, "diag", "btd", ne)
+    outs = []
+    for apart in (True, False):
+        xl, xg, xr = container(), container(), container()
+        if not apart:
+            both = torch.zeros((ne + 1, xr.nnz), dtype=torch.complex128, device=device)
+            xr = DSDBCOO(both[:ne], xr.rows, xr.cols, bs, (ne,))
+            dump = xr if same == "pointer" else DSDBCOO(both[1:], xr.rows, xr.cols, bs, (ne,))
+            xl, xg = (dump, xg) if shared == "lesser" else (xl, dump)
+        RGF(ne, retarded_offdiag=True).selected_solve(a, sl, sg, obc_blocks=obc, out=(xl, xg, xr),
+                                                      return_retarded=True)
+        outs.append((xr, xg if shared == "lesser" else xl))
+    (r0, q0), (r1, q1) = outs
+    assert rel_err(q1.data.cpu().numpy(), q0.data.cpu().numpy()) < 1e-10
+    if same == "pointer":
+        assert rel_err(r1.data.cpu().numpy(), r0.data.cpu().numpy()) < 1e-10
