@@ -374,7 +374,15 @@ void rgf_selected_solve(qx_handle* h, hipStream_t st0, const qx_btd_layout* la,
   const int bmax = block_limits(la, "selected_solve");
   const Btd A0(la, a), SL0(lsl, sl), SG0(lsg, sg), XL0(lxl, xl), XG0(lxg, xg),
       XR0(want_r ? lxr : nullptr, want_r ? xr : nullptr);
-  if (rgf_small_solve(h, st0, la, a, lsl, sl, lsg, sg, obc_r, obc_l, obc_g, lxl, xl, lxg, xg,
+  // One container for G^R and a quantity the caller does not need: G^R is
+  // written last.  The fused kernel keeps that order within an energy, so it is
+  // left out where an energy's G^R shares memory with another energy's G^≶.
+  auto crossed = [&](const Btd& x) {
+    return want_r && XR0.overlaps(x) &&
+           !(XR0.base == x.base && XR0.L->stack_stride == x.L->stack_stride);
+  };
+  if (!crossed(XL0) && !crossed(XG0) &&
+      rgf_small_solve(h, st0, la, a, lsl, sl, lsg, sg, obc_r, obc_l, obc_g, lxl, xl, lxg, xg,
                       want_r ? lxr : nullptr, want_r ? xr : nullptr, want_cur ? current : nullptr,
                       corner, density, ldos, flags, prec))
     return;

@@ -56,6 +56,7 @@ struct SLay {
 struct SmallArgs {
   int N, flags, NS, split;
   int bmax, slot;  // largest block, elements of a workspace slot (bmax^2)
+  int shared;      // G^R in the container of G^< or G^>
   int bs[kSN];
   int orb[kSN];  // first orbital of each block (density row offsets)
   int64_t n_orb;
@@ -533,6 +534,7 @@ __global__ __launch_bounds__(kSolveThreads) void rgf_small_kernel(SmallArgs g) {
     const M Xq = XQ(tq), od = Od(tq, N - 1);
     if (g.density && team == 0) sdiag_imag(tt, kThreads, bn, Xq, g.density + e * g.n_orb + g.orb[N - 1]);
     if (od.p) sherm(tt, kThreads, bn, bn, 0.0, 0.5, Xq, -0.5, Xq, od);
+    if (g.shared) sync();  // G^R is written last
     if (want_r && team == 0) {
       const M xr = blk(g.XR, g.sXR, e, g.lXR.diag[N - 1], bn);
       if (xr.p) saxpby(tt, kThreads, bn, bn, kOneS, lds(rj), kZeroS, none, xr);
@@ -629,6 +631,7 @@ __global__ __launch_bounds__(kSolveThreads) void rgf_small_kernel(SmallArgs g) {
     if (!skip_lower[q - 1] && low.p) sherm(tt, kThreads, bj, bi, 0.0, 0.0, none, -1.0, Oij, low);
     if (od.p) sherm(tt, kThreads, bi, bi, 0.0, 0.5, Z, -0.5, Z, od);
     if (g.density && q == 1) sdiag_imag(tt, kThreads, bi, Z, g.density + e * g.n_orb + g.orb[i]);
+    if (g.shared) sync();  // G^R is written last
     if (want_r && team == 0) {
       const M xr = blk(g.XR, g.sXR, e, g.lXR.diag[i], bi);
       if (xr.p) saxpby(tt, kThreads, bi, bi, kOneS, Zr, kZeroS, none, xr);
@@ -799,6 +802,7 @@ bool rgf_small_solve(qx_handle* h, hipStream_t st, const qx_btd_layout* la, cons
   g.NS = 3 * N + 15;
   g.bmax = *std::max_element(la->block_sizes, la->block_sizes + N);
   g.slot = g.bmax * g.bmax;
+  g.shared = xr && (xr == xl || xr == xg);
   g.split = prec == QX_PREC_C128_3M ? 3 : 4;
   int off = 0;
   for (int i = 0; i < kSN; ++i) {

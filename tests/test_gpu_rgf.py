@@ -772,7 +772,8 @@ def test_selected_inv_output_forms(device, monkeypatch, bs, form, precision):
 
 @pytest.mark.parametrize("shared", ["lesser", "greater"])
 @pytest.mark.parametrize("same", ["pointer", "part"])
-@pytest.mark.parametrize("block_sizes", [[64, 40, 64, 64]], ids=["4x64"])
+@pytest.mark.parametrize("block_sizes", [[64, 40, 64, 64], [20, 32, 9, 32] * 5, [20, 32, 9]],
+                         ids=["4x64", "20x32", "3x32"])
 def test_retarded_and_lesser_or_greater_in_one_container(device, block_sizes, shared, same):
     """A caller that does not need one of G^<, G^> hands the container of G^R
     for it as well: G^R, written last, and the other quantity are those of
