@@ -184,8 +184,7 @@ void herm(hipStream_t s, int64_t batch, int m, int n, double cy, double ca,
              cc, D.p, D.stride, D.ld, batch,
              a2.p, a2.stride, a2.ld, b2.p, b2.stride, b2.ld, y2.p, y2.stride, y2.ld};
   const int64_t blocks = (two ? 2 : 1) * batch * g.tm * g.tn;
-  QX_REQUIRE(blocks < (int64_t(1) << 31), "herm: grid too large");
-  hipLaunchKernelGGL(herm_kernel, dim3((unsigned)blocks), dim3(NT), 0, s, g);
+  hipLaunchKernelGGL(herm_kernel, dim3(groups(blocks, NT, "herm")), dim3(NT), 0, s, g);
   QX_HIP_CHECK(hipGetLastError());
 }
 
@@ -751,8 +750,7 @@ void ew_contact_sigma(hipStream_t s, int64_t batch, int n, const Mat& S, const d
   QX_REQUIRE(S.ld == n && L.ld == n && G.ld == n, "contact_sigma: matrices must be dense n x n");
   const int tn = (n + TS - 1) / TS;
   const int64_t blocks = batch * tn * tn;
-  QX_REQUIRE(blocks < (int64_t(1) << 31), "contact_sigma: grid too large");
-  hipLaunchKernelGGL(contact_sigma_kernel, dim3((unsigned)blocks), dim3(NT), 0, s, S.p, S.stride,
+  hipLaunchKernelGGL(contact_sigma_kernel, dim3(groups(blocks, NT, "contact_sigma")), dim3(NT), 0, s, S.p, S.stride,
                      n, f, L.p, L.stride, G.p, G.stride, tn);
   QX_HIP_CHECK(hipGetLastError());
 }
@@ -772,11 +770,10 @@ void ew_assemble(hipStream_t s, int64_t batch, int64_t nnz, const z2* z, const z
   if (batch <= 0 || nnz <= 0) return;
   QX_REQUIRE(A && (z || !S), "assemble: null argument");
   const int64_t gx = (nnz + NT - 1) / NT;
-  QX_REQUIRE(gx < (int64_t(1) << 31), "assemble: grid too large");
   constexpr int64_t per = int64_t(65535) * kAsmE;  // energies per launch (grid.y limit)
   for (int64_t e = 0; e < batch; e += per) {
     const int64_t n = std::min(per, batch - e);
-    const dim3 grid((unsigned)gx, (unsigned)((n + kAsmE - 1) / kAsmE));
+    const dim3 grid(groups(gx, NT, "assemble"), (unsigned)((n + kAsmE - 1) / kAsmE));
     if (Sig)
       hipLaunchKernelGGL(assemble_kernel<true>, grid, dim3(NT), 0, s, z + (S ? e : 0), S, T,
                          Sig + e * sSig, sSig, A + e * sA, sA, nnz, n);
@@ -831,8 +828,7 @@ void ew_skew_update(hipStream_t s, int64_t batch, int n, const Mat& X0, const Ma
              {X0.stride, x1.stride}, {P0.stride, p1.stride}, {Y0.stride, y1.stride},
              {X0.ld, x1.ld}, {P0.ld, p1.ld}, {Y0.ld, y1.ld}, dens, dens_stride};
   const int64_t blocks = (two ? 2 : 1) * batch * (tn * (tn + 1) / 2);
-  QX_REQUIRE(blocks < (int64_t(1) << 31), "skew_update: grid too large");
-  hipLaunchKernelGGL(skew_update_kernel, dim3((unsigned)blocks), dim3(NT), 0, s, g);
+  hipLaunchKernelGGL(skew_update_kernel, dim3(groups(blocks, NT, "skew_update")), dim3(NT), 0, s, g);
   QX_HIP_CHECK(hipGetLastError());
 }
 
@@ -848,10 +844,13 @@ void skew_check(hipStream_t s, int64_t batch, const std::vector<SkewBlock>& bloc
       g.n[k] = blocks[b0 + k].n;
     }
     g.flag = flag;
-    const int64_t wgs = batch * g.blocks;
-    QX_REQUIRE(wgs < (int64_t(1) << 31), "skew_check: grid too large");
-    hipLaunchKernelGGL(skew_check_kernel, dim3((unsigned)wgs), dim3(NT), 0, s, g);
-    QX_HIP_CHECK(hipGetLastError());
+    const int64_t most = max_groups(NT) / kSkewBlocks;  // matrices per launch
+    for (int64_t e = 0; e < batch; e += most) {
+      const unsigned wgs = (unsigned)(std::min(batch - e, most) * g.blocks);
+      hipLaunchKernelGGL(skew_check_kernel, dim3(wgs), dim3(NT), 0, s, g);
+      QX_HIP_CHECK(hipGetLastError());
+      for (int k = 0; k < g.blocks; ++k) g.p[k] += most * g.stride[k];
+    }
   }
 }
 
@@ -879,13 +878,12 @@ void trace_diff(hipStream_t s, int64_t batch, int n, const Mat& X, const Mat& Y,
   if (batch <= 0) return;
   const int tn = (n + TS - 1) / TS;
   QX_REQUIRE(!part.zero() && part.stride >= tn, "trace_diff: scratch too small");
-  QX_REQUIRE(batch * tn < (int64_t(1) << 31), "trace_diff: grid too large");
   TraceArgs g{n, X.p, Y.p, Z.p, W.p, X.stride, Y.stride, Z.stride, W.stride,
               X.ld, Y.ld, Z.ld, W.ld, out, out_stride};
   if (X.zero() || Y.zero()) g.X = nullptr;
   if (Z.zero() || W.zero()) g.Z = nullptr;
-  hipLaunchKernelGGL(trace_kernel, dim3((unsigned)(batch * tn)), dim3(NT), 0, s, g, tn, part.p,
-                     part.stride);
+  hipLaunchKernelGGL(trace_kernel, dim3(groups(batch * tn, NT, "trace_diff")), dim3(NT), 0, s, g,
+                     tn, part.p, part.stride);
   hipLaunchKernelGGL(trace_sum_kernel, dim3((unsigned)((batch + NT - 1) / NT)), dim3(NT), 0, s,
                      part.p, part.stride, tn, out, out_stride, batch);
   QX_HIP_CHECK(hipGetLastError());
@@ -894,9 +892,12 @@ void trace_diff(hipStream_t s, int64_t batch, int n, const Mat& X, const Mat& Y,
 void absnorm2(hipStream_t s, int64_t batch, int n, const Mat& A, const Mat& B,
               double* out) {
   if (batch <= 0) return;
-  hipLaunchKernelGGL(absnorm_kernel, dim3((unsigned)batch), dim3(NTN), 0, s, n, A.p,
-                     A.stride, A.ld, B.p, B.stride, B.ld, out);
-  QX_HIP_CHECK(hipGetLastError());
+  for (int64_t e = 0; e < batch; e += max_groups(NTN)) {
+    const unsigned wgs = (unsigned)std::min(batch - e, max_groups(NTN));
+    hipLaunchKernelGGL(absnorm_kernel, dim3(wgs), dim3(NTN), 0, s, n, A.p + e * A.stride, A.stride,
+                       A.ld, B.p + e * B.stride, B.stride, B.ld, out + e);
+    QX_HIP_CHECK(hipGetLastError());
+  }
 }
 
 void max_value(hipStream_t s, int64_t n, const double* v, double* out) {
@@ -908,8 +909,7 @@ void max_value(hipStream_t s, int64_t n, const double* v, double* out) {
 void ew_ns_check(hipStream_t s, int64_t batch, int n, const Mat& R, double tol, int* flagged,
                  int* info) {
   if (batch <= 0) return;
-  QX_REQUIRE(batch < (int64_t(1) << 31), "ns_check: batch too large");
-  hipLaunchKernelGGL(ns_check_kernel, dim3((unsigned)batch), dim3(NT), 0, s, n, R.p, R.stride,
+  hipLaunchKernelGGL(ns_check_kernel, dim3(groups(batch, NT, "ns_check")), dim3(NT), 0, s, n, R.p, R.stride,
                      R.ld, tol, flagged, info);
   QX_HIP_CHECK(hipGetLastError());
 }

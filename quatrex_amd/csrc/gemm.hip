@@ -619,9 +619,7 @@ template <typename T, int SPLIT, int BM, int BN, int WM, int WN>
 void launch_shape(hipStream_t s, int64_t batch, int opA, int opB, GemmArgs g) {
   g.tilesM = (g.m + BM - 1) / BM;
   g.tilesN = (g.n + BN - 1) / BN;
-  const int64_t blocks = batch * g.tilesM * g.tilesN;
-  QX_REQUIRE(blocks < (int64_t(1) << 31), "zgemm: grid too large");
-  dim3 grid((unsigned)blocks), block(64 * WM * WN);
+  const dim3 block(64 * WM * WN), grid(groups(batch * g.tilesM * g.tilesN, block.x, "zgemm"));
   KernelTimer* timer = active_timer;
   hipEvent_t ev0 = nullptr;
   if (timer) timer->begin(s, &ev0);
@@ -661,9 +659,8 @@ void launch_reg(hipStream_t s, int64_t batch, int opA, int opB, GemmArgs g) {
   g.tilesN = (g.n + BN - 1) / BN;
   g.count = (unsigned)batch;
   const int64_t waves = batch * g.tilesM * g.tilesN;
-  QX_REQUIRE(waves < (int64_t(1) << 31), "zgemm: grid too large");
   const bool full = g.m % BM == 0 && g.n % BN == 0 && g.k % (4 * D) == 0;
-  dim3 grid((unsigned)((waves + 3) / 4)), block(256);
+  const dim3 grid(groups((waves + 3) / 4, 256, "zgemm")), block(256);
   KernelTimer* timer = active_timer;
   hipEvent_t ev0 = nullptr;
   if (timer) timer->begin(s, &ev0);

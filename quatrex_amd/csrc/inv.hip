@@ -1070,7 +1070,7 @@ void with_rows_per_lane(int n, const F& f) {
 
 template <typename T, int NB>
 void launch_panel_cg(hipStream_t s, int64_t batch, int n, const PanelArgs& pa) {
-  const dim3 grid((unsigned)batch);
+  const dim3 grid(groups(batch, 512, "inv"));
   if constexpr (NB == 64) {
     // eight waves of eight columns, four rows per lane (n <= 256)
     hipLaunchKernelGGL((inv_panel_cg<T, 4, 8, 64>), grid, dim3(512), 0, s, pa);
@@ -1104,9 +1104,8 @@ bool inv_lookahead() {
 // An update launch of the look-ahead (32-deep chunks, as inv_step).
 template <typename T>
 void launch_update(hipStream_t s, int64_t batch, const UpdArgs& ua) {
-  const int64_t blocks = batch * ua.tiles;
-  QX_REQUIRE(blocks < (int64_t(1) << 31), "inv: grid too large");
-  hipLaunchKernelGGL((inv_update<T, 32, 32, 1>), dim3((unsigned)blocks), dim3(NT), 0, s, ua);
+  hipLaunchKernelGGL((inv_update<T, 32, 32, 1>), dim3(groups(batch * ua.tiles, NT, "inv")), dim3(NT),
+                     0, s, ua);
 }
 
 template <typename T>
@@ -1144,12 +1143,10 @@ void run_inverse_lookahead(hipStream_t s, int64_t batch, int n, const Mat (&B)[2
     ur.tiles = tn * (tn - 1);
     const int64_t total = batch * ur.tiles;
     const int np = (int)((batch + 7) / 8 * 8);
-    const int64_t blocks = np + (total + 1) / 2;
-    QX_REQUIRE(blocks < (int64_t(1) << 31), "inv: grid too large");
+    const dim3 grid(groups(np + (total + 1) / 2, 512, "inv"));
     const PanelArgs pn = panel_args(p + 1);
     with_rows_per_lane(n, [&](auto r) {
-      hipLaunchKernelGGL((inv_step<T, r()>), dim3((unsigned)blocks), dim3(512), 0, s, pn, ur,
-                         (int)batch, np, total);
+      hipLaunchKernelGGL((inv_step<T, r()>), grid, dim3(512), 0, s, pn, ur, (int)batch, np, total);
     });
   }
 }
@@ -1175,19 +1172,19 @@ void run_inverse(hipStream_t s, int64_t batch, int n, const Mat& X, const InvScr
       if (NB == 32 && kind == 0)
         launch_panel_cg<T, 32>(s, batch, n, pa);
       else if (NB == 32 && RPT == 1 && kind == 4)
-        hipLaunchKernelGGL((inv_panel4<T>), dim3((unsigned)batch), dim3(NT4), 0, s, pa);
+        hipLaunchKernelGGL((inv_panel4<T>), dim3(groups(batch, NT4, "inv")), dim3(NT4), 0, s, pa);
       else
-        hipLaunchKernelGGL((inv_panel<T, NB, RPT>), dim3((unsigned)batch), dim3(NT), 0, s, pa);
+        hipLaunchKernelGGL((inv_panel<T, NB, RPT>), dim3(groups(batch, NT, "inv")), dim3(NT), 0, s,
+                           pa);
     }
     if (n > nbw) {
       UpdArgs ua{n, k0, nbw, tn * tn, B[cur].p, B[cur].stride, B[cur].ld,
                  B[nxt].p, B[nxt].stride, B[nxt].ld, scr.ints, scr.int_stride, mask};
-      const int64_t blocks = batch * tn * tn;
-      QX_REQUIRE(blocks < (int64_t(1) << 31), "inv: grid too large");
+      const dim3 grid(groups(batch * tn * tn, NT, "inv"));
       if (narrow_update(batch))
-        hipLaunchKernelGGL((inv_update<T, NB, 16, 4>), dim3((unsigned)blocks), dim3(NT), 0, s, ua);
+        hipLaunchKernelGGL((inv_update<T, NB, 16, 4>), grid, dim3(NT), 0, s, ua);
       else
-        hipLaunchKernelGGL((inv_update<T, NB, 32, 1>), dim3((unsigned)blocks), dim3(NT), 0, s, ua);
+        hipLaunchKernelGGL((inv_update<T, NB, 32, 1>), grid, dim3(NT), 0, s, ua);
     }
     cur = nxt;
   }
@@ -1220,9 +1217,12 @@ int inv_whole_max() {
 
 void launch_whole(hipStream_t s, int64_t batch, int n, const Mat& A, const Mat& S, const Mat& X,
                   int* info, const int* mask) {
-#define QX_WHOLE(G)                                                                          \
-  hipLaunchKernelGGL((inv_whole<G>), dim3((unsigned)batch), dim3(G::THREADS), 0, s, n, A.p,  \
-                     A.stride, A.ld, S.p, S.stride, S.ld, X.p, X.stride, X.ld, info, mask)
+#define QX_WHOLE(G)                                                                              \
+  for (int64_t e = 0; e < batch; e += max_groups(G::THREADS))                                    \
+  hipLaunchKernelGGL((inv_whole<G>), dim3((unsigned)min(batch - e, max_groups(G::THREADS))),     \
+                     dim3(G::THREADS), 0, s, n, A.p + e * A.stride, A.stride, A.ld,              \
+                     S.p ? S.p + e * S.stride : nullptr, S.stride, S.ld, X.p + e * X.stride,     \
+                     X.stride, X.ld, info + e, mask ? mask + e : nullptr)
   if (n <= 32) QX_WHOLE(GjWhole32);
   else if (n <= 64) QX_WHOLE(GjWhole64);
   else if (n <= 96) QX_WHOLE(GjWhole96);

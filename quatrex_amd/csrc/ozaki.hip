@@ -296,10 +296,10 @@ void zgemm_ozaki(hipStream_t s, int64_t batch, int m, int n, int k, int opA, int
   if (timer) timer->begin(s, &ev0);
   // line i of op(A) = row i of A, or conj of column i of A for A^H;
   // line j of op(B) = column j of B, or conj of row j of B for B^H
-  hipLaunchKernelGGL(ozaki_split_kernel, dim3((unsigned)(batch * m)), dim3(ONT), 0, s, A.p,
+  hipLaunchKernelGGL(ozaki_split_kernel, dim3(groups(batch * m, ONT, "zgemm_ozaki")), dim3(ONT), 0, s, A.p,
                      A.stride, A.ld, opA == QX_OP_C ? 1 : 0, opA == QX_OP_C ? 1 : 0, m, k,
                      k_pad, slices, dA, sAd, ea, (int64_t)m);
-  hipLaunchKernelGGL(ozaki_split_kernel, dim3((unsigned)(batch * n)), dim3(ONT), 0, s, B.p,
+  hipLaunchKernelGGL(ozaki_split_kernel, dim3(groups(batch * n, ONT, "zgemm_ozaki")), dim3(ONT), 0, s, B.p,
                      B.stride, B.ld, opB == QX_OP_N ? 1 : 0, opB == QX_OP_C ? 1 : 0, n, k,
                      k_pad, slices, dB, sBd, eb, (int64_t)n);
   OzArgs g;
@@ -327,11 +327,11 @@ void zgemm_ozaki(hipStream_t s, int64_t batch, int m, int n, int k, int opA, int
   g.tilesN = (n + OBN - 1) / OBN;
   g.beta_zero = ((beta.re == 0.0 && beta.im == 0.0) || Cin.zero()) ? 1 : 0;
   const int64_t blocks = batch * g.tilesM * g.tilesN;
-  QX_REQUIRE(blocks < (int64_t(1) << 31), "zgemm_ozaki: grid too large");
+  const dim3 grid(groups(blocks, ONT, "zgemm_ozaki"));
   switch (slices) {
 #define QX_OZ_CASE(S)                                                                   \
   case S:                                                                               \
-    hipLaunchKernelGGL(ozaki_gemm_kernel<S>, dim3((unsigned)blocks), dim3(ONT), 0, s, g); \
+    hipLaunchKernelGGL(ozaki_gemm_kernel<S>, grid, dim3(ONT), 0, s, g);                 \
     break;
     QX_OZ_CASE(2)
     QX_OZ_CASE(3)

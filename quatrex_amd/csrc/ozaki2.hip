@@ -444,12 +444,11 @@ void zgemm_oz2(hipStream_t s, int64_t batch, int m, int n, int k, int opA, int o
   // line i of op(A): row i of A, or conj of column i of A for A^H;
   // line j of op(B): column j of B, or conj of row j of B for B^H
   const int64_t ga = batch * ((m + 7) / 8), gb = batch * ((n + 7) / 8);
-  QX_REQUIRE(ga < (int64_t(1) << 31) && gb < (int64_t(1) << 31), "zgemm_oz2: grid too large");
-  hipLaunchKernelGGL(oz2_split_kernel, dim3((unsigned)ga), dim3(256), 0, s, x.A.p, x.A.stride,
-                     x.A.ld, opA == QX_OP_C ? 1 : 0, opA == QX_OP_C ? 1 : 0, m, k, k_pad, c, Ra,
+  hipLaunchKernelGGL(oz2_split_kernel, dim3(groups(ga, 256, "zgemm_oz2")), dim3(256), 0, s, x.A.p,
+                     x.A.stride, x.A.ld, opA == QX_OP_C ? 1 : 0, opA == QX_OP_C ? 1 : 0, m, k, k_pad, c, Ra,
                      sRa, ea, (int64_t)m);
-  hipLaunchKernelGGL(oz2_split_kernel, dim3((unsigned)gb), dim3(256), 0, s, x.B.p, x.B.stride,
-                     x.B.ld, opB == QX_OP_N ? 1 : 0, opB == QX_OP_C ? 1 : 0, n, k, k_pad, c, Rb,
+  hipLaunchKernelGGL(oz2_split_kernel, dim3(groups(gb, 256, "zgemm_oz2")), dim3(256), 0, s, x.B.p,
+                     x.B.stride, x.B.ld, opB == QX_OP_N ? 1 : 0, opB == QX_OP_C ? 1 : 0, n, k, k_pad, c, Rb,
                      sRb, eb, (int64_t)n);
   Oz2Args g{};
   g.m = m;
@@ -484,8 +483,7 @@ void zgemm_oz2(hipStream_t s, int64_t batch, int m, int n, int k, int opA, int o
   g.V = V;
   g.c = c;
   const int64_t blocks = batch * g.tilesM * g.tilesN;
-  QX_REQUIRE(blocks * nmod < (int64_t(1) << 31), "zgemm_oz2: grid too large");
-  const dim3 mgrid((unsigned)(blocks * nmod));
+  const dim3 mgrid(groups(blocks * nmod, 256, "zgemm_oz2"));
   switch (k_pad / 64) {
 #define QX_OZ_MOD(NK)                                                   \
   case NK:                                                              \

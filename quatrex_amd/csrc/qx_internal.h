@@ -84,6 +84,15 @@ struct Error {
     if (!(cond)) throw ::qx::Error{QX_EINVAL, (msg)};                        \
   } while (0)
 
+// A launch counts its threads along x in 32 bits and drops what is beyond them
+// without an error: the most workgroups of `threads` threads it can take, and a
+// grid that is refused above it.
+constexpr int64_t max_groups(int threads) { return ((int64_t(1) << 32) - 1) / threads; }
+inline unsigned groups(int64_t n, int threads, const char* what) {
+  QX_REQUIRE(n <= max_groups(threads), std::string(what) + ": grid too large");
+  return (unsigned)n;
+}
+
 // ---- kernels (launchers) --------------------------------------------------
 
 // Fused selected inversion for stacks of small blocks (rgf_small.hip);

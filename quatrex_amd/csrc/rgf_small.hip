@@ -57,6 +57,7 @@ struct SmallArgs {
   int N, flags, NS, split;
   int bmax, slot;  // largest block, elements of a workspace slot (bmax^2)
   int shared;      // G^R in the container of G^< or G^>
+  int64_t e0;      // energy of the launch's first workgroup
   int bs[kSN];
   int orb[kSN];  // first orbital of each block (density row offsets)
   int64_t n_orb;
@@ -386,7 +387,7 @@ const Cplx kOneS{1.0, 0.0}, kMinusS{-1.0, 0.0}, kZeroS{0.0, 0.0};
 template <int SP>
 __global__ __launch_bounds__(kSolveThreads) void rgf_small_kernel(SmallArgs g) {
   __shared__ Shared sh;
-  const int64_t e = blockIdx.x;
+  const int64_t e = g.e0 + blockIdx.x;
   const int N = g.N;
   constexpr int sp = SP;
   const bool want_r = (g.flags & QX_SOLVE_RETARDED) != 0;
@@ -654,7 +655,8 @@ __global__ __launch_bounds__(kSolveThreads) void rgf_small_kernel(SmallArgs g) {
 // rgf.hip), one workgroup per energy.
 struct SmallInvArgs {
   int N, NS, split;
-  int slot;  // elements of a workspace slot
+  int slot;    // elements of a workspace slot
+  int64_t e0;  // energy of the launch's first workgroup
   int bs[kSN];
   int64_t sA, sX;
   const z2* A;
@@ -671,7 +673,7 @@ struct SmallInvArgs {
 template <int SP>
 __global__ __launch_bounds__(kSolveThreads) void rgf_small_inv_kernel(SmallInvArgs g) {
   __shared__ GjShared<GjWhole32> sh;
-  const int64_t e = blockIdx.x;
+  const int64_t e = g.e0 + blockIdx.x;
   const int N = g.N;
   constexpr int sp = SP;
   int* info = g.info + e;
@@ -841,11 +843,14 @@ bool rgf_small_solve(qx_handle* h, hipStream_t st, const qx_btd_layout* la, cons
   KernelTimer* timer = active_timer;
   hipEvent_t ev0 = nullptr;
   if (timer) timer->begin(st, &ev0);
-  if (g.split == 3)
-    hipLaunchKernelGGL(rgf_small_kernel<3>, dim3((unsigned)S), dim3(kSolveThreads), 0, st, g);
-  else
-    hipLaunchKernelGGL(rgf_small_kernel<4>, dim3((unsigned)S), dim3(kSolveThreads), 0, st, g);
-  QX_HIP_CHECK(hipGetLastError());
+  for (g.e0 = 0; g.e0 < S; g.e0 += max_groups(kSolveThreads)) {
+    const dim3 grid((unsigned)std::min(S - g.e0, max_groups(kSolveThreads)));
+    if (g.split == 3)
+      hipLaunchKernelGGL(rgf_small_kernel<3>, grid, dim3(kSolveThreads), 0, st, g);
+    else
+      hipLaunchKernelGGL(rgf_small_kernel<4>, grid, dim3(kSolveThreads), 0, st, g);
+    QX_HIP_CHECK(hipGetLastError());
+  }
   if (timer) {
     // matrix flops of the products and inverses the kernel runs when no
     // optional term is present (no current, corner, Σ off-diagonal blocks or
@@ -903,11 +908,14 @@ bool rgf_small_inv(qx_handle* h, hipStream_t st, const qx_btd_layout* la, const 
   KernelTimer* timer = active_timer;
   hipEvent_t ev0 = nullptr;
   if (timer) timer->begin(st, &ev0);
-  if (g.split == 3)
-    hipLaunchKernelGGL(rgf_small_inv_kernel<3>, dim3((unsigned)S), dim3(kSolveThreads), 0, st, g);
-  else
-    hipLaunchKernelGGL(rgf_small_inv_kernel<4>, dim3((unsigned)S), dim3(kSolveThreads), 0, st, g);
-  QX_HIP_CHECK(hipGetLastError());
+  for (g.e0 = 0; g.e0 < S; g.e0 += max_groups(kSolveThreads)) {
+    const dim3 grid((unsigned)std::min(S - g.e0, max_groups(kSolveThreads)));
+    if (g.split == 3)
+      hipLaunchKernelGGL(rgf_small_inv_kernel<3>, grid, dim3(kSolveThreads), 0, st, g);
+    else
+      hipLaunchKernelGGL(rgf_small_inv_kernel<4>, grid, dim3(kSolveThreads), 0, st, g);
+    QX_HIP_CHECK(hipGetLastError());
+  }
   if (timer) {
     // matrix flops of its products and inverses (8 m n k, 8 n^3), counted as
     // GEMM work of this one launch

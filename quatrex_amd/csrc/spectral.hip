@@ -94,8 +94,8 @@ void spectral_modes(hipStream_t s, int64_t n, int b, int m, const z2* ws, const 
   ModeArgs g{n, b, m, ws, vs, am, a0, ap, min_decay, max_decay, min_propagation,
              residual_tolerance, eta_decay, residual_normalization ? 1 : 0, mask, res, dk};
   const int64_t blocks = (n * m + 255) / 256;
-  QX_REQUIRE(blocks < (int64_t(1) << 31), "spectral_modes: too many modes");
-  hipLaunchKernelGGL(spectral_modes_kernel, dim3((unsigned)blocks), dim3(256), 0, s, g);
+  hipLaunchKernelGGL(spectral_modes_kernel, dim3(groups(blocks, 256, "spectral_modes")), dim3(256),
+                     0, s, g);
   QX_HIP_CHECK(hipGetLastError());
 }
 

@@ -188,7 +188,6 @@ void svd_tall(hipStream_t s, int64_t n, int d, int m, const Mat& A, const Mat& U
   QX_REQUIRE(!A.zero() && !U.zero() && S && !V.zero(), "svd: null operand");
   QX_REQUIRE(max_sweeps >= 1 && tol > 0.0, "svd: bad iteration limits");
   if (n <= 0) return;
-  QX_REQUIRE(n < (int64_t(1) << 31), "svd: batch too large");
   QX_REQUIRE(ws_bytes >= svd_workspace_bytes(n, d, m), "svd: workspace too small");
   SvdArgs g;
   g.d = d;
@@ -208,7 +207,8 @@ void svd_tall(hipStream_t s, int64_t n, int d, int m, const Mat& A, const Mat& U
   g.sV = V.stride;
   g.sweeps = sweeps;
   QX_REQUIRE(U.ld == m && V.ld == m, "svd: U and V must be contiguous (leading dimension = cols)");
-  hipLaunchKernelGGL(jacobi_svd_kernel, dim3((unsigned)n), dim3(kSvdThreads), 0, s, g);
+  hipLaunchKernelGGL(jacobi_svd_kernel, dim3(groups(n, kSvdThreads, "svd")), dim3(kSvdThreads), 0,
+                     s, g);
   QX_HIP_CHECK(hipGetLastError());
 }
 
