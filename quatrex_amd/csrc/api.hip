@@ -178,11 +178,15 @@ thread_local int split_part = 0;
 // 256 x 64 (1024) 4.28 / 4.79 (2: 4.42), 64 x 128 (1024) 7.16 / 7.13 (2: 7.10),
 // 48 x 176 (1728) 17.1 / 16.0, 128 x 128 (2048) 7.8 / 7.1, 64 x 256 (4096)
 // 209 / 203.
-void run_split(qx_handle* h, hipStream_t st, int64_t S, int b,
-               const std::function<void(hipStream_t, int64_t, int64_t)>& f) {
+int split_count(const qx_handle* h, int64_t S, int b) {
   const int64_t tiles = (b + 31) / 32, waves = S * tiles * tiles;
   const int64_t most = std::min<int64_t>(S / 4, waves / 512);
-  const int P = (int)std::min<int64_t>(h->parts, std::max<int64_t>(1, most));
+  return (int)std::min<int64_t>(h->parts, std::max<int64_t>(1, most));
+}
+
+void run_split(qx_handle* h, hipStream_t st, int64_t S, int b,
+               const std::function<void(hipStream_t, int64_t, int64_t)>& f) {
+  const int P = split_count(h, S, b);
   if (P <= 1) {
     f(st, 0, S);
     return;

@@ -328,8 +328,10 @@ extern thread_local int active_gemm_tile;
 // qx_inv_batched_noalloc (once per device; called by qx_create).
 void noalloc_init(int device);
 
-// Splits a batch of S matrices (blocks of at most b) into up to
-// `handle->parts` contiguous sub-batches and runs f(stream, e0, n) for each concurrently: sub-batch 0 on
+// Sub-batches run_split makes of S matrices with blocks of at most b.
+int split_count(const qx_handle* h, int64_t S, int b);
+// Splits a batch of S matrices (blocks of at most b) into split_count, at most
+// `handle->parts`, contiguous sub-batches and runs f(stream, e0, n) for each concurrently: sub-batch 0 on
 // the caller's stream `st` in this thread, the others on handle-owned streams
 // from helper host threads.  Events order all sub-batches after the work
 // already queued on `st`, and `st` waits for all of them before returning.

@@ -422,13 +422,28 @@ void rgf_selected_solve(qx_handle* h, hipStream_t st0, const qx_btd_layout* la,
     skew_on = cap == hipStreamCaptureStatusNone;
   }
   if (skew_on) h->ensure_words();
+  // Each sub-batch checks its own blocks and all wait for every answer: one
+  // sweep for the whole call, so that the number of sub-batches changes no bit.
+  // true: the sub-batch's answer is on its way (its event is recorded).
+  std::vector<std::promise<bool>> votes(skew_on ? split_count(h, Stot, bmax) : 0);
+  std::vector<std::shared_future<bool>> voted;
+  for (auto& v : votes) voted.push_back(v.get_future().share());
   hipEvent_t stg_ev = nullptr;
   if (stagger) QX_HIP_CHECK(hipEventCreateWithFlags(&stg_ev, hipEventDisableTiming));
   std::promise<void> stg_set;
   std::shared_future<void> stg_ready = stg_set.get_future().share();
   run_split(h, st0, Stot, bmax, [&](hipStream_t st, int64_t e0, int64_t S) {
-  const OzSubBatch oz(prec, oz_region, bmax, e0, S);
   const int part = split_part;
+  // a sub-batch that leaves early with an error has no answer
+  struct Vote {
+    std::promise<bool>* p;
+    void cast(bool queued) {
+      if (p) p->set_value(queued);
+      p = nullptr;
+    }
+    ~Vote() { cast(false); }
+  } vote{skew_on ? &votes[part] : nullptr};
+  const OzSubBatch oz(prec, oz_region, bmax, e0, S);
   // sub-batch 0 releases the others once its first inverse is enqueued, or
   // when it leaves early with an error
   struct Release {
@@ -554,6 +569,7 @@ void rgf_selected_solve(qx_handle* h, hipStream_t st0, const qx_btd_layout* la,
     QX_HIP_CHECK(hipMemcpyAsync(h->word_host + part, flag, sizeof(int), hipMemcpyDeviceToHost,
                                 st));
     QX_HIP_CHECK(hipEventRecord(h->part_ev[part], st));
+    vote.cast(true);
   }
 
   // ---- forward sweep (rgf.py:234-295) ----
@@ -648,10 +664,12 @@ void rgf_selected_solve(qx_handle* h, hipStream_t st0, const qx_btd_layout* la,
     if (lds) ew_diag_imag(st, S, bn, W.get(sr[N - 1], bn), lds + orb_off[N - 1], n_orb, kLdos);
   }
 
-  bool skew = false;
-  if (skew_on) {
-    QX_HIP_CHECK(hipEventSynchronize(h->part_ev[part]));
-    skew = *reinterpret_cast<const volatile int*>(h->word_host + part) == 0;
+  bool skew = skew_on;
+  for (size_t k = 0; skew && k < voted.size(); ++k) {
+    skew = voted[k].get();
+    if (!skew) break;
+    QX_HIP_CHECK(hipEventSynchronize(h->part_ev[k]));
+    skew = *reinterpret_cast<const volatile int*>(h->word_host + k) == 0;
   }
   // full[qi]: G^≶_jj of the step before (the caller's output block, projected,
   // in the skew-Hermitian sweep where it is written, else a workspace slot)
