@@ -1244,14 +1244,16 @@ void launch_whole(hipStream_t s, int64_t batch, int n, const Mat& A, const Mat& 
 // wins (128 x 192^2 0.46 against 0.48), nor above 256, one panel per CU, where
 // the longer panels take a second round (384 x 256^2 2.31 -> 2.27, 640 x 256^2
 // 3.70 -> 3.62: not worth another order of summation).
+// steady calls (the block inverses of the RGF, whose sub-batches and batches
+// would else decide over the bits of a result) keep 32.
 // QX_INV_NB=16|32|64 overrides for n <= 256 (16 runs the one-thread-per-row
 // kernel).
-int inv_panel_width(int64_t batch, int n, int precision) {
+int inv_panel_width(int64_t batch, int n, int precision, bool steady) {
   const int forced_nb = forced_panel_width();
   if (n > 256) return inv_panel_kind() == 0 ? 32 : 16;
   if (forced_nb == 64 && inv_panel_kind() != 0) return 32;
   if (forced_nb) return forced_nb;
-  const bool wide = batch >= 160 && batch <= 256 && n >= 192 && (n + 63) / 64 * 64 - n <= 48;
+  const bool wide = !steady && batch >= 160 && batch <= 256 && n >= 192 && (n + 63) / 64 * 64 - n <= 48;
   return wide && precision != QX_PREC_C64 && inv_panel_kind() == 0 && inv_group_width() == 4
              ? 64
              : 32;
@@ -1259,7 +1261,7 @@ int inv_panel_width(int64_t batch, int n, int precision) {
 
 Mat zinv_input(int64_t batch, int n, const Mat& X, const InvScratch& scr, int precision) {
   if (precision != QX_PREC_C64 && n <= inv_whole_max()) return X;
-  const int NB = inv_panel_width(batch, n, precision);
+  const int NB = inv_panel_width(batch, n, precision, scr.steady);
   const int npan = (n + NB - 1) / NB;
   // the panels ping-pong between X and the scratch buffer, the last one
   // writing the scratch buffer: an odd count starts in X, an even one in it
@@ -1290,7 +1292,7 @@ void zinv(hipStream_t s, int64_t batch, int n, const Mat& A, const Mat& S, const
     return;
   }
 
-  const int NB = inv_panel_width(batch, n, precision);
+  const int NB = inv_panel_width(batch, n, precision, scr.steady);
   const bool big = n > 256 && NB == 16;
   const int npan = (n + NB - 1) / NB;
   // start in the buffer that makes the last panel write the scratch buffer

@@ -211,6 +211,9 @@ struct InvScratch {
   int64_t buf_stride;
   int* ints;
   int64_t int_stride;
+  // 32-column panels whatever the number of matrices (inv_panel_width): callers
+  // whose results are not to depend on how a stack is cut into calls
+  bool steady = false;
 };
 // A non-null mask restricts the inverse to the matrices with mask[e] != 0;
 // the others (X included) are left untouched.

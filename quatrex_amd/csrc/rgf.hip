@@ -72,11 +72,12 @@ struct Slots {
   int64_t cap;  // elements per matrix
   int64_t e0;
   Mat get(int k, int ld) const { return Mat(base + (int64_t)k * S * cap + e0 * cap, cap, ld); }
-  // inverse scratch: complex buffer in slot k, pivot ints in slot k + 1
+  // inverse scratch: complex buffer in slot k, pivot ints in slot k + 1; the
+  // panels do not depend on the energies of a sub-batch
   InvScratch inv(int k) const {
     return InvScratch{base + (int64_t)k * S * cap + e0 * cap, cap,
                       reinterpret_cast<int*>(base + (int64_t)(k + 1) * S * cap + e0 * cap),
-                      4 * cap};
+                      4 * cap, true};
   }
 };
 

@@ -75,11 +75,12 @@ def _same_bits(device, call, counts):
             assert torch.equal(x, y), (streams, name)
 
 
-# (energies, block sizes): ranges of unequal lengths
-STACKS = [(518, [64, 48, 64])]
+# (energies, block sizes): ranges of unequal lengths; whole inverses, and panels
+# on a stack that a call in one range passes to the inverse as 250 matrices
+STACKS = [(518, [64, 48, 64]), (250, [208, 256, 200])]
 
 
-@pytest.mark.parametrize("n_e,sizes", STACKS, ids=["518x64"])
+@pytest.mark.parametrize("n_e,sizes", STACKS, ids=["518x64", "250x256"])
 @pytest.mark.parametrize("precision", ["c128", "c128-3m", "mixed"])
 @pytest.mark.parametrize("sigma", ["skew", "one-not-skew"])
 def test_solve_bits(device, n_e, sizes, precision, sigma):
@@ -105,7 +106,7 @@ def test_solve_bits(device, n_e, sizes, precision, sigma):
     _same_bits(device, call, (2, 3, 4))
 
 
-@pytest.mark.parametrize("n_e,sizes", STACKS, ids=["518x64"])
+@pytest.mark.parametrize("n_e,sizes", STACKS, ids=["518x64", "250x256"])
 @pytest.mark.parametrize("precision", ["c128", "c128-3m", "mixed"])
 def test_inverse_bits(device, n_e, sizes, precision):
     """selected_inv with boundary blocks, new output and output over A."""
