@@ -1236,14 +1236,20 @@ void launch_whole(hipStream_t s, int64_t batch, int n, const Mat& A, const Mat& 
 // Panel width: 32 columns; with the older panel kernels 16 above n = 256
 // (where two rows per thread double their per-column work).  From 160 matrices
 // on the updates stream every matrix through HBM, and 64-column panels (eight
-// waves of eight columns, n <= 256) halve the passes over it: 256 x 256^2
-// 1.64 -> 1.40 ms, 160 x 256^2 1.16 -> 1.03, 256 x 192^2 0.80 -> 0.69, 256 x
-// 208^2 1.23 -> 1.17; not where the last panel would be nearly empty (300 x
-// 200^2 1.43 -> 1.56) or the matrix has fewer than three (512 x 160^2 1.05 ->
-// 1.13), nor below 160 matrices, where the look-ahead of the 32-column panels
-// wins (128 x 192^2 0.46 against 0.48), nor above 256, one panel per CU, where
-// the longer panels take a second round (384 x 256^2 2.31 -> 2.27, 640 x 256^2
-// 3.70 -> 3.62: not worth another order of summation).
+// waves of eight columns, n <= 256) halve the passes over it.  32 / 64 columns,
+// us per call:
+//   matrices        128        160        192        256        257        512
+//   n = 192     463/ 496   547/ 524   654/ 581   809/ 680   869/ 933  1399/1315
+//   n = 208     671/ 747   835/ 855   961/ 959  1229/1171  1320/1470  2179/2294
+//   n = 224     713/ 793   894/ 904  1092/1066  1305/1244  1407/1561  2316/2427
+//   n = 240     829/ 847  1095/1004  1304/1146  1512/1322  1628/1658  2694/2577
+//   n = 256     880/ 879  1173/1076  1390/1200  1621/1398  1739/1749  2911/2800
+// The lines: 160 matrices (below, the look-ahead of the 32-column panels wins or
+// is close), 192 where the last panel is at most half full, never where it is
+// nearly empty (300 x 200^2 1.43 -> 1.56 ms) or the matrix has fewer than three
+// (512 x 160^2 1.05 -> 1.13); and 256, the CUs of the chip, each with one panel:
+// beyond it the longer panels take a second round, which 4 % at 512 matrices of
+// some sizes do not repay at 257 to 320.
 // steady calls (the block inverses of the RGF, whose sub-batches and batches
 // would else decide over the bits of a result) keep 32.
 // QX_INV_NB=16|32|64 overrides for n <= 256 (16 runs the one-thread-per-row
@@ -1253,7 +1259,9 @@ int inv_panel_width(int64_t batch, int n, int precision, bool steady) {
   if (n > 256) return inv_panel_kind() == 0 ? 32 : 16;
   if (forced_nb == 64 && inv_panel_kind() != 0) return 32;
   if (forced_nb) return forced_nb;
-  const bool wide = !steady && batch >= 160 && batch <= 256 && n >= 192 && (n + 63) / 64 * 64 - n <= 48;
+  const int last = (n - 1) % 64 + 1;  // columns of the last 64-column panel
+  const bool wide = !steady && batch >= (last > 32 ? 160 : 192) && batch <= 256 && n >= 192 &&
+                    last >= 16;
   return wide && precision != QX_PREC_C64 && inv_panel_kind() == 0 && inv_group_width() == 4
              ? 64
              : 32;

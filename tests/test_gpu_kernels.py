@@ -490,3 +490,22 @@ def test_whole_inverse_singular_raises(device, n):
     with pytest.raises(np.linalg.LinAlgError):
         _inv(device, A, X, 0)
     assert np.array_equal(X[0].cpu().numpy(), np.eye(n))
+
+
+@pytest.mark.parametrize("batch,n,wide", [(159, 240, False), (160, 240, True), (160, 208, False),
+                                          (191, 224, False), (192, 224, True), (192, 208, True),
+                                          (256, 207, False), (257, 256, False), (256, 191, False)])
+def test_wide_panel_lines(device, monkeypatch, batch, n, wide):
+    """Which calls take 64-column panels: the bits are those of the width forced,
+    and the two widths differ."""
+    g = torch.Generator(device=device).manual_seed(n)
+    A = torch.randn((batch, n, n), dtype=torch.complex128, device=device, generator=g)
+    outs = []
+    for nb in (None, "32", "64"):
+        if nb:
+            monkeypatch.setenv("QX_INV_NB", nb)
+        X = torch.empty_like(A)
+        _inv(device, A, X, 0)
+        outs.append(torch.view_as_real(X))
+    assert torch.equal(outs[0], outs[2 if wide else 1])
+    assert not torch.equal(outs[1], outs[2])
