@@ -960,8 +960,12 @@ __global__ __launch_bounds__(512) void inv_step(PanelArgs pa, UpdArgs ua, int ba
   update_tile<T, 32, 32>(ua, u, in && update_live(ua, u), threadIdx.x & (NT - 1), sh.u[half]);
 }
 
-// Whole matrices in registers (gj_core.h): shapes for n <= 64, 96, 128
-// (GjWhole32 there).
+// Whole matrices in registers (gj_core.h): shapes for n <= 4, 64, 96, 128
+// (GjWhole32 there).  Up to 4 the call is bound by the launch of its workgroups
+// and by how many fit a CU, so they are two waves with 10 KB of LDS; one
+// sub-panel holds the matrix, and the bits are those of GjWhole32 (65536
+// matrices, GjWhole32 -> GjWhole4: n = 1 209 -> 52 us, n = 4 290 -> 85).
+typedef GjShape<1, 1, 1, 1, 4> GjWhole4;
 typedef GjShape<4, 1, 4, 1, 8> GjWhole64;
 typedef GjShape<6, 1, 6, 2, 8> GjWhole96;
 typedef GjShape<8, 1, 8, 2, 8> GjWhole128;
@@ -1203,9 +1207,9 @@ void run_inverse(hipStream_t s, int64_t batch, int n, const Mat& X, const InvScr
 // none).  At 128 the line is where the matrix still fits the registers of one
 // CU (256 KB of accumulators).  us per call against the split panel and update
 // kernels (n <= 32: against one workgroup of four waves per matrix):
-//   64 x 32^2 20 / 30, 1024 x 32^2 29 / 58, 64 x 64^2 44 / 107, 1024 x 64^2
-//   164 / 330, 32 x 96^2 109 / 159, 256 x 96^2 123 / 241, 32 x 128^2 168 /
-//   224, 512 x 128^2 373 / 618.
+//   65536 x 1^2 52 / 118, 65536 x 4^2 85 / 278, 64 x 32^2 20 / 30, 1024 x 32^2
+//   29 / 58, 64 x 64^2 44 / 107, 1024 x 64^2 164 / 330, 32 x 96^2 109 / 159,
+//   256 x 96^2 123 / 241, 32 x 128^2 168 / 224, 512 x 128^2 373 / 618.
 // Panels of larger matrices held and factored the same way (32 columns of 256
 // rows) took 42 us instead of 47, and the step with its own update longer than
 // the look-ahead's: 32 x 256^2 497-553 against 490, so those stay as they are.
@@ -1223,7 +1227,8 @@ void launch_whole(hipStream_t s, int64_t batch, int n, const Mat& A, const Mat& 
                      dim3(G::THREADS), 0, s, n, A.p + e * A.stride, A.stride, A.ld,              \
                      S.p ? S.p + e * S.stride : nullptr, S.stride, S.ld, X.p + e * X.stride,     \
                      X.stride, X.ld, info + e, mask ? mask + e : nullptr)
-  if (n <= 32) QX_WHOLE(GjWhole32);
+  if (n <= 4) QX_WHOLE(GjWhole4);
+  else if (n <= 32) QX_WHOLE(GjWhole32);
   else if (n <= 64) QX_WHOLE(GjWhole64);
   else if (n <= 96) QX_WHOLE(GjWhole96);
   else QX_WHOLE(GjWhole128);

@@ -101,7 +101,7 @@ def test_sancho_rubio_of_many_leads(device):
 
 
 def test_inverse_of_many_matrices(device):
-    """Workgroups of 192 threads: 22369621 matrices fill a launch."""
-    x = torch.arange(1, 22369621 + 4, dtype=torch.float64, device=device)
+    """Workgroups of 128 threads: 33554431 matrices fill a launch."""
+    x = torch.arange(1, 33554431 + 4, dtype=torch.float64, device=device)
     got = inv((x + 0j).reshape(-1, 1, 1)).reshape(-1)
     assert float((got * x - 1).abs().max()) < 1e-15 * 4
