@@ -386,29 +386,42 @@ __global__ __launch_bounds__(NT) void diag_imag_kernel(const z2* X, int64_t sX, 
 }
 
 // System matrix on the nnz pattern: A[e, k] = z_e S_k + T_k - Sig[e, k].
-// A workgroup covers NT consecutive entries of kAsmE energies: S and T are read
-// once for them, the Sigma loads of all are in flight together, and nothing is
-// divided by nnz (one thread per element of a flat grid: two 64-bit divisions
-// each, 3.4 TB/s at 256 energies of 866 k entries).  Streaming, 32 bytes per
-// entry and energy.
-constexpr int kAsmE = 8;
-template <bool SIG>
+// A thread covers one entry of E energies: S and T are read once for them, their
+// Sigma loads are in flight together.  The grid is entries by groups of energies,
+// flat below kAsmFlat entries, where one 32-bit division finds the thread's place
+// (one thread per element of a flat grid: two 64-bit divisions each).
+// Streaming, 32 bytes per entry and energy with Sigma, 16 without.
+// With Sigma E = 4 and stores past the caches, else E = 8: eight loads and eight
+// stores in rows a power of two apart evict each other.  us, one thread per
+// element / E = 8 / as it is (a grid of entries by energies at 30 entries: 18):
+//   energies x entries   with Sigma           without
+//   64 x 262144           98 / 108 /  88       39 /  45
+//   64 x 262656          147 / 101 /  96      113 /  49
+//   256 x 100000         194 / 159 / 145       91 /  76
+//   256 x 866304        1674 /1326 /1258      988 / 624
+//   100000 x 30         15.5 /15.4 /16.5     11.0 / 9.7
+constexpr int64_t kAsmFlat = 2048;
+template <bool SIG, int E>
 __global__ __launch_bounds__(NT) void assemble_kernel(const z2* z, const z2* S, const z2* T,
                                                       const z2* Sig, int64_t sSig, z2* A,
-                                                      int64_t sA, int64_t nnz, int64_t batch) {
-  const int64_t k = blockIdx.x * (int64_t)NT + threadIdx.x;
-  const int64_t e0 = blockIdx.y * (int64_t)kAsmE;
-  if (k >= nnz) return;
-  const int ne = (int)(batch - e0 < kAsmE ? batch - e0 : kAsmE);
-  z2 sg[kAsmE];
+                                                      int64_t sA, unsigned nnz, int64_t batch) {
+  unsigned k = blockIdx.x * (unsigned)NT + threadIdx.x, grp = blockIdx.y;
+  if (nnz < kAsmFlat) {
+    grp = k / nnz;
+    k -= grp * nnz;
+  }
+  const int64_t e0 = grp * (int64_t)E;
+  if (k >= nnz || e0 >= batch) return;
+  const int ne = (int)(batch - e0 < E ? batch - e0 : E);
+  z2 sg[E];
   if constexpr (SIG) {
 #pragma unroll
-    for (int u = 0; u < kAsmE; ++u) sg[u] = Sig[(e0 + (u < ne ? u : 0)) * sSig + k];
+    for (int u = 0; u < E; ++u) sg[u] = Sig[(e0 + (u < ne ? u : 0)) * sSig + k];
   }
   const z2 sk = S ? S[k] : make_double2(0.0, 0.0);
   const z2 tk = T ? T[k] : make_double2(0.0, 0.0);
 #pragma unroll
-  for (int u = 0; u < kAsmE; ++u) {
+  for (int u = 0; u < E; ++u) {
     if (u < ne) {
       double vr = 0.0, vi = 0.0;
       if (S) {
@@ -424,7 +437,14 @@ __global__ __launch_bounds__(NT) void assemble_kernel(const z2* z, const z2* S, 
         vr -= sg[u].x;
         vi -= sg[u].y;
       }
-      A[(e0 + u) * sA + k] = make_double2(vr, vi);
+      double* a = &A[(e0 + u) * sA + k].x;
+      if constexpr (SIG) {
+        typedef double d2 __attribute__((ext_vector_type(2)));
+        __builtin_nontemporal_store(d2{vr, vi}, reinterpret_cast<d2*>(a));
+      } else {
+        a[0] = vr;
+        a[1] = vi;
+      }
     }
   }
 }
@@ -769,18 +789,24 @@ void ew_assemble(hipStream_t s, int64_t batch, int64_t nnz, const z2* z, const z
                  const z2* T, const z2* Sig, int64_t sSig, z2* A, int64_t sA) {
   if (batch <= 0 || nnz <= 0) return;
   QX_REQUIRE(A && (z || !S), "assemble: null argument");
-  const int64_t gx = (nnz + NT - 1) / NT;
-  constexpr int64_t per = int64_t(65535) * kAsmE;  // energies per launch (grid.y limit)
-  for (int64_t e = 0; e < batch; e += per) {
-    const int64_t n = std::min(per, batch - e);
-    const dim3 grid(groups(gx, NT, "assemble"), (unsigned)((n + kAsmE - 1) / kAsmE));
-    if (Sig)
-      hipLaunchKernelGGL(assemble_kernel<true>, grid, dim3(NT), 0, s, z + (S ? e : 0), S, T,
-                         Sig + e * sSig, sSig, A + e * sA, sA, nnz, n);
-    else
-      hipLaunchKernelGGL(assemble_kernel<false>, grid, dim3(NT), 0, s, z + (S ? e : 0), S, T,
-                         Sig, sSig, A + e * sA, sA, nnz, n);
-    QX_HIP_CHECK(hipGetLastError());
+  constexpr int64_t kMost = int64_t(1) << 28;  // threads of a launch
+  for (int64_t k = 0; k < nnz; k += kMost) {
+    const int64_t len = std::min(kMost, nnz - k);
+    const bool flat = len < kAsmFlat;
+    auto launch = [&](auto kernel, int per) {  // energies per thread
+      const int64_t rows = std::min<int64_t>(kMost / len, flat ? kMost : 65535);
+      for (int64_t e = 0; e < batch; e += rows * per) {
+        const int64_t n = std::min(rows * per, batch - e), grp = (n + per - 1) / per;
+        const dim3 grid((unsigned)(((flat ? grp * len : len) + NT - 1) / NT),
+                        flat ? 1u : (unsigned)grp);
+        hipLaunchKernelGGL(kernel, grid, dim3(NT), 0, s, z + (S ? e : 0), S ? S + k : nullptr,
+                           T ? T + k : nullptr, Sig ? Sig + e * sSig + k : nullptr, sSig,
+                           A + e * sA + k, sA, (unsigned)len, n);
+        QX_HIP_CHECK(hipGetLastError());
+      }
+    };
+    if (Sig) launch(assemble_kernel<true, 4>, 4);
+    else launch(assemble_kernel<false, 8>, 8);
   }
 }
 

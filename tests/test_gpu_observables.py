@@ -134,3 +134,60 @@ def test_assembly_kernel_edges(device, batch, nnz, terms):
     got = out.cpu().numpy()
     assert np.allclose(got[:batch], want, rtol=1e-15, atol=4e-15)
     assert np.all(got[batch] == 7.0)
+
+
+@pytest.mark.parametrize("with_sigma", [True, False])
+@pytest.mark.parametrize("batch,nnz", [(3, 29), (1001, 30), (4097, 7), (5, 300), (65537, 1), (9, 2047),
+                                       (9, 2048), (9, 2305)])
+def test_assembly_small_patterns(device, batch, nnz, with_sigma):
+    """Patterns shorter than a workgroup (its threads cover several groups of
+    energies) and around the line of the flat grid, with strides above nnz and in place over Sigma; entries outside
+    are left alone.  Two roundings a term: 4 eps of the terms' sizes."""
+    from quatrex_amd import _lib
+
+    g = torch.Generator(device=device).manual_seed(batch + nnz)
+    cn = lambda *s: torch.randn(*s, dtype=torch.complex128, generator=g, device=device)  # noqa: E731
+    z, s, t, sig = cn(batch), cn(nnz), cn(nnz), cn(batch, nnz + 2)
+    want = z[:, None] * s + t
+    out = sig.clone()
+    size = (z[:, None] * s).abs() + t.abs()
+    if with_sigma:
+        want, size = want - sig[:, :nnz], size + sig[:, :nnz].abs()
+    h = _lib.handle(device)
+    rc = _lib.load().qx_assemble_system_matrix(
+        h, _lib.stream_ptr(device), batch, nnz, z.data_ptr(), s.data_ptr(), t.data_ptr(),
+        out.data_ptr() if with_sigma else None, nnz + 2, out.data_ptr(), nnz + 2)
+    _lib.check(rc, h, "assemble")
+    assert bool(((out[:, :nnz] - want).abs() <= 4 * np.finfo(float).eps * size).all())
+    assert torch.equal(torch.view_as_real(out[:, nnz:]), torch.view_as_real(sig[:, nnz:]))
+
+
+@pytest.mark.parametrize("with_sigma", [True, False])
+@pytest.mark.parametrize("shape", ["energies", "rows", "entries"])
+def test_assembly_of_more_than_one_launch(device, shape, with_sigma):
+    """A launch takes 2^28 threads and a grid 65535 rows: stacks and patterns beyond one, the second
+    launch's first and last elements among those looked at."""
+    from quatrex_amd import _lib
+
+    line = 1 << 28
+    if shape == "energies":
+        batch, nnz = (4 if with_sigma else 8) * line + 9, 1
+    elif shape == "rows":  # of a grid, 65535 at most
+        batch, nnz = (4 if with_sigma else 8) * 65535 + 9, 2048
+    else:
+        batch, nnz = 2, line + 9
+    n = batch * nnz
+    z = torch.arange(batch, dtype=torch.float64, device=device) + 0j
+    s = torch.ones(nnz, dtype=torch.complex128, device=device)
+    t = torch.arange(nnz, dtype=torch.float64, device=device) * 1j
+    out = torch.full((n,), 0.5, dtype=torch.complex128, device=device)
+    h = _lib.handle(device)
+    rc = _lib.load().qx_assemble_system_matrix(
+        h, _lib.stream_ptr(device), batch, nnz, z.data_ptr(), s.data_ptr(), t.data_ptr(),
+        out.data_ptr() if with_sigma else None, nnz, out.data_ptr(), nnz)
+    _lib.check(rc, h, "assemble")
+    less = 0.5 if with_sigma else 0.0
+    for lo in range(0, n, line):
+        i = torch.arange(lo, min(lo + line, n), device=device)
+        want = torch.complex((i // nnz).double() - less, (i % nnz).double())
+        assert torch.equal(torch.view_as_real(out[lo:lo + line]), torch.view_as_real(want))
