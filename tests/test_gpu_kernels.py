@@ -537,3 +537,60 @@ def test_whole_inverse_smallest_bits(device, n):
     A[3, :, 0] = 0.0
     with pytest.raises(np.linalg.LinAlgError):
         _inv(device, A, X, 0)
+
+
+@pytest.mark.parametrize("n", [40, 64, 65, 100, 128])
+@pytest.mark.parametrize("batch", [5, 260])
+def test_split_inverse_variants_up_to_128(device, monkeypatch, n, batch):
+    """complex128 matrices up to 128 on the split kernels, which their whole
+    inverse leaves unused by default: 16- and 32-deep chunks of the update, and
+    the look-ahead or not, sum the same products in the same order."""
+    rng = np.random.default_rng(11 * n + batch)
+    a = _cplx(rng, (batch, n, n))
+    a[:, 0, 0] = 0.0  # a row interchange at the first pivot
+    A = torch.as_tensor(a, device=device)
+    monkeypatch.setenv("QX_INV_WHOLE", "0")
+
+    def run():
+        X = torch.empty_like(A)
+        _inv(device, A, X, 0)
+        return X.cpu().numpy()
+
+    outs = []
+    for depth in ("16", "32"):
+        monkeypatch.setenv("QX_INV_UPDATE", depth)
+        for look in ("1", "0"):
+            monkeypatch.setenv("QX_INV_LOOKAHEAD", look)
+            outs.append(run())
+    monkeypatch.delenv("QX_INV_UPDATE")
+    monkeypatch.delenv("QX_INV_LOOKAHEAD")
+    monkeypatch.delenv("QX_INV_WHOLE")
+    whole = run()
+    for x in outs[1:]:
+        assert np.array_equal(outs[0].view(np.uint64), x.view(np.uint64))
+    assert not np.array_equal(whole, outs[0])  # other kernels indeed
+    for e in range(2):
+        tol = 1e-15 * np.linalg.cond(a[e]) * n
+        assert rel_err(outs[0][e], np.linalg.inv(a[e])) < tol
+        assert rel_err(whole[e], outs[0][e]) < 2 * tol
+
+
+@pytest.mark.parametrize("n", [3, 20, 32])
+@pytest.mark.parametrize("batch", [1, 5, 9])
+def test_smallest_whole_inverse_against_split_kernels(device, monkeypatch, n, batch):
+    """n <= 32 with a subtracted matrix: the whole inverse against the split
+    panels, same pivot rule, results to rounding."""
+    rng = np.random.default_rng(10 * n + batch)
+    a, s = _cplx(rng, (batch, n, n)), 0.1 * _cplx(rng, (batch, n, n))
+    A, S = torch.as_tensor(a, device=device), torch.as_tensor(s, device=device)
+    outs = []
+    for whole in ("32", "0"):
+        monkeypatch.setenv("QX_INV_WHOLE", whole)
+        X = torch.empty_like(A)
+        _inv(device, A, X, 0, S)
+        outs.append(X.cpu().numpy())
+    assert not np.array_equal(outs[0], outs[1])
+    for e in range(batch):
+        tol = 1e-15 * np.linalg.cond(a[e] - s[e]) * max(n, 4)
+        assert rel_err(outs[0][e], outs[1][e]) < tol
+        assert rel_err(outs[0][e], np.linalg.inv(a[e] - s[e])) < tol
