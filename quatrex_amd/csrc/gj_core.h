@@ -1,7 +1,8 @@
-// Gauss-Jordan elimination of a panel held in MFMA result registers (gfx950,
-// double precision), shared by the batched inverses.
+// Gauss-Jordan inverse of a matrix held in MFMA result registers (gfx950,
+// double precision), for the batched inverse up to 128 and the fused
+// small-block solves.
 //
-// A workgroup of one factoring wave (wave 0) and MW update waves holds a panel
+// A workgroup of one factoring wave (wave 0) and MW update waves holds a matrix
 // of up to 16 RT MW rows and 16 CT columns: update wave u the rows
 // 16 RT u .. in RT x CT tiles of the v_mfma_f64_16x16x4_f64 result layout.
 // The columns are eliminated in sub-panels of SB = 4 or 8:
@@ -51,6 +52,9 @@ __device__ __forceinline__ double gj_lane_read(double v, int l) {
   const unsigned hi = (unsigned)__builtin_amdgcn_readlane((int)(b >> 32), l);
   return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
 }
+__device__ __forceinline__ float gj_lane_read(float v, int l) {
+  return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), l));
+}
 
 // MW update waves of RT x CT tiles, RL rows per lane of the factoring wave,
 // sub-panels of SB columns.
@@ -71,14 +75,12 @@ struct GjShared {
   z2 prow[G::SB][G::C];     // pivot rows, the B operand of the update
   z2 rcp[G::SB];            // pivot reciprocals of a sub-panel
   int step_of[G::LS];       // sub-panel step of a pivot row, or -1
-  int perm[G::C];           // position interchanged with k0 + column
   int piv[G::C];            // pivot row of a column
   int pos[G::LS];           // final position of a row
 };
 
 // One wave factors columns [0, ns) of the sub-panel sub, the columns k, k + 1,
-// ... of the matrix (panel columns col0, ...): the pivot of column k + c is
-// the row of largest |re| + |im| (pivot_key) among the rows at positions >=
+// ... of the matrix: the pivot of column k + c is the row of largest |re| + |im| (pivot_key) among the rows at positions >=
 // k + c.  pos[j]: the position of row lane + 64 j, -1 for the rows >= n.
 // The scaling of a pivot row by its reciprocal is deferred to the end of the
 // sub-panel (its multiplier is taken as zero and its active entry as 1; the
@@ -86,7 +88,7 @@ struct GjShared {
 // and step_of the pivot rows' steps.
 template <typename G>
 __device__ __forceinline__ void gj_factor(GjShared<G>& sh, z2 (*sub)[G::LS], int n, int k,
-                                          int col0, int ns, int (&pos)[G::RL], int* info) {
+                                          int ns, int (&pos)[G::RL], int* info) {
   constexpr int RL = G::RL, SB = G::SB;
   const int lane = threadIdx.x & 63;
   double xr[RL][SB], xi[RL][SB];
@@ -137,8 +139,7 @@ __device__ __forceinline__ void gj_factor(GjShared<G>& sh, z2 (*sub)[G::LS], int
       complex_recip(ar[c], ai[c], vr, vi);
       if (lane == 0) {
         sh.rcp[c] = make_double2(vr, vi);
-        sh.perm[col0 + c] = q;
-        sh.piv[col0 + c] = p;
+        sh.piv[k + c] = p;
       }
 #pragma unroll
       for (int j = 0; j < RL; ++j) {
@@ -214,13 +215,12 @@ __device__ __forceinline__ void gj_update(const GjShared<G>& sh, const z2 (*sub)
   }
 }
 
-// Eliminates the columns k0 .. k0 + nbw - 1 (nbw <= 16 CT) of n rows; called
-// by the factoring wave.  Passes the workgroup barriers of gj_update_waves.
+// Eliminates the n columns; called by the factoring wave.  Passes the workgroup
+// barriers of gj_update_waves.
 template <typename G>
-__device__ __forceinline__ void gj_factor_wave(GjShared<G>& sh, int n, int k0, int nbw,
-                                               int* info) {
+__device__ __forceinline__ void gj_factor_wave(GjShared<G>& sh, int n, int* info) {
   const int lane = threadIdx.x & 63;
-  const int nsub = (nbw + G::SB - 1) / G::SB;
+  const int nsub = (n + G::SB - 1) / G::SB;
   int pos[G::RL];
 #pragma unroll
   for (int j = 0; j < G::RL; ++j) pos[j] = lane + 64 * j < n ? lane + 64 * j : -1;
@@ -229,8 +229,7 @@ __device__ __forceinline__ void gj_factor_wave(GjShared<G>& sh, int n, int k0, i
 #pragma unroll 1
   for (int s = 0; s < nsub; ++s) {
     __syncthreads();  // the sub-panel's columns are in LDS
-    gj_factor<G>(sh, sh.sub[s & 1], n, k0 + s * G::SB, s * G::SB, min(G::SB, nbw - s * G::SB),
-                 pos, info);
+    gj_factor<G>(sh, sh.sub[s & 1], n, s * G::SB, min(G::SB, n - s * G::SB), pos, info);
     __syncthreads();  // the reduced sub-panel is in LDS
     __syncthreads();  // the pivot rows are in LDS
   }
@@ -240,9 +239,9 @@ __device__ __forceinline__ void gj_factor_wave(GjShared<G>& sh, int n, int k0, i
   __syncthreads();
 }
 
-// The same for update wave u: acr / aci hold its rows of the panel (rows >= n
-// and columns >= nbw zero).  Ends with a barrier after which sh.perm, sh.piv
-// and sh.pos are complete.
+// The same for update wave u: acr / aci hold its rows of the matrix (rows and
+// columns >= n zero).  Ends with a barrier after which sh.piv and sh.pos are
+// complete.
 //
 // The loop over the sub-panels stays rolled: unrolled, the code outgrows the
 // instruction cache (128 rows: 185 -> 705 us).  Accumulators are therefore
@@ -252,11 +251,11 @@ __device__ __forceinline__ void gj_factor_wave(GjShared<G>& sh, int n, int k0, i
 template <typename G>
 __device__ __forceinline__ void gj_update_waves(GjShared<G>& sh, int u,
                                                 gj_acc (&acr)[G::CT][G::RT],
-                                                gj_acc (&aci)[G::CT][G::RT], int nbw) {
+                                                gj_acc (&aci)[G::CT][G::RT], int n) {
   constexpr int RT = G::RT, CT = G::CT, SB = G::SB;
   const int lane = threadIdx.x & 63, l16 = lane & 15, l4 = lane >> 4;
   const int row0 = 16 * RT * u;
-  const int nsub = (nbw + SB - 1) / SB;
+  const int nsub = (n + SB - 1) / SB;
   // the columns of sub-panel s of the own rows to LDS
   auto extract = [&](int s) {
     auto* sub = sh.sub[s & 1];
@@ -280,7 +279,7 @@ __device__ __forceinline__ void gj_update_waves(GjShared<G>& sh, int u,
     // pivot rows to LDS and out of the accumulators; the sub-panel's own
     // columns are replaced by the reduced ones (zero accumulator, identity in
     // the B operand)
-    const int c0 = s * SB, ns = min(SB, nbw - c0);
+    const int c0 = s * SB, ns = min(SB, n - c0);
     int st[RT][4];
 #pragma unroll
     for (int i = 0; i < RT; ++i)
@@ -345,7 +344,7 @@ __device__ __forceinline__ void gj_invert(int n, const z2* A, int lda, const z2*
   const int lane = threadIdx.x & 63;
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   if (w == 0) {
-    gj_factor_wave<G>(sh, n, 0, n, info);
+    gj_factor_wave<G>(sh, n, info);
   } else if (w <= G::MW) {
     const int l16 = lane & 15, l4 = lane >> 4, row0 = 16 * RT * (w - 1);
     gj_acc acr[CT][RT], aci[CT][RT];

@@ -9,7 +9,8 @@
 // Algorithm: blocked in-place Gauss-Jordan elimination split into kernels so
 // that the O(n^3) part runs on every CU of the chip while the sequential
 // pivoting chain stays short:
-//   for each panel of NB = 32 columns (QX_INV_NB=64: 64 for n <= 256)
+//   for each panel of NB = 32 columns (64 for some numbers of matrices of up
+//   to 256: inv_panel_width)
 //     panel kernel  (one workgroup per matrix): by default inv_panel_cg, in
 //        which each wave holds a group of the panel's columns for all rows
 //        and the rows never move (one barrier per column; see the kernel);
@@ -17,9 +18,10 @@
 //        threads per row for n <= 256, inv_panel4; QX_INV_PANEL=1: one or two
 //        rows per thread, 16-column panels above n = 256, inv_panel).  The
 //        pivot of a column is the first row of maximal |re| + |im| among the
-//        unreduced rows, compared through a 32-bit key (float magnitude with
-//        9 low mantissa bits replaced by the row index).  The reduced panel,
-//        the pivot rows and the composed row gather sig are written out.
+//        unreduced rows, compared through a 32-bit key (pivot_key: the upper
+//        word of the magnitude's double, the row in its 9 low bits).  The
+//        reduced panel, the pivot rows and the composed row gather sig are
+//        written out.
 //     update kernel (64 x 64 tiles of every matrix, MFMA; the rank-NB sum
 //        staged through LDS in 16- or 32-deep k-chunks): the other columns
 //        receive the row interchanges and the rank-NB update in one pass,
@@ -457,19 +459,6 @@ __global__ __launch_bounds__(NT4) void inv_panel4(PanelArgs g) {
   panel_gathers<NT4>(perm_l, n, k0, nbw, tid, sig, idx);
 }
 
-// Wave-wide unsigned max with DPP only: quad and row butterflies give every
-// lane its row's maximum, row_bcast:15 / row_bcast:31 carry the row maxima
-// up to lane 63, which is read once.  Every lane of the wave must be active.
-__device__ inline unsigned wave_max_bcast(unsigned v) {
-  v = max(v, (unsigned)__builtin_amdgcn_update_dpp(0, (int)v, 0xB1, 0xf, 0xf, false));   // quad xor 1
-  v = max(v, (unsigned)__builtin_amdgcn_update_dpp(0, (int)v, 0x4E, 0xf, 0xf, false));   // quad xor 2
-  v = max(v, (unsigned)__builtin_amdgcn_update_dpp(0, (int)v, 0x124, 0xf, 0xf, false));  // row_ror 4
-  v = max(v, (unsigned)__builtin_amdgcn_update_dpp(0, (int)v, 0x128, 0xf, 0xf, false));  // row_ror 8
-  v = max(v, (unsigned)__builtin_amdgcn_update_dpp(0, (int)v, 0x142, 0xa, 0xf, false));  // row_bcast:15
-  v = max(v, (unsigned)__builtin_amdgcn_update_dpp(0, (int)v, 0x143, 0xc, 0xf, false));  // row_bcast:31
-  return (unsigned)__builtin_amdgcn_readlane((int)v, 63);
-}
-
 // Panel kernel with column groups (n <= 64 RPL, NB-column panels): wave w of
 // the NB / CW waves holds columns CW w .. CW w + CW - 1 of the panel for all
 // rows, lane l the rows l + 64 j (j < RPL).  Rows stay in their registers;
@@ -507,17 +496,6 @@ __device__ inline unsigned wave_max_bcast(unsigned v) {
 // Pivot choice (largest |re| + |im| through the 32-bit key, ties to the lower
 // row), arithmetic and outputs are those of the other panel kernels up to
 // rounding; ties are broken by the row's index at the start of the panel.
-// Value of v in lane l of the wave (l uniform).
-__device__ inline double lane_read(double v, int l) {
-  const long long b = __double_as_longlong(v);
-  const unsigned lo = (unsigned)__builtin_amdgcn_readlane((int)b, l);
-  const unsigned hi = (unsigned)__builtin_amdgcn_readlane((int)(b >> 32), l);
-  return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
-}
-__device__ inline float lane_read(float v, int l) {
-  return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), l));
-}
-
 template <typename T, int RPL, int CW, int NB>
 struct PanelCgShared {
   T col_r[2][64 * RPL], col_i[2][64 * RPL];
@@ -573,8 +551,8 @@ __device__ __forceinline__ void panel_cg(const PanelArgs& g, int64_t e,
 #pragma unroll
         for (int c = 0; c < CW; ++c) {
           if (c == own) continue;
-          ar[c] = lane_read(xr[j][c], pl);
-          ai[c] = lane_read(xi[j][c], pl);
+          ar[c] = gj_lane_read(xr[j][c], pl);
+          ai[c] = gj_lane_read(xi[j][c], pl);
         }
       }
     }
@@ -625,7 +603,7 @@ __device__ __forceinline__ void panel_cg(const PanelArgs& g, int64_t e,
       const unsigned kj = pivot_key((double)xr[j][ca], (double)xi[j][ca], r);
       key = max(key, pos[j] >= k ? kj : 0u);
     }
-    key = wave_max_bcast(key);
+    key = gj_wave_max(key);
     // a candidate always exists (n - k rows), so p < n; min() keeps every
     // index inside the panel whatever the key holds
     const int p = min(511 - (int)(key & 0x1FFu), n - 1);
@@ -636,8 +614,8 @@ __device__ __forceinline__ void panel_cg(const PanelArgs& g, int64_t e,
 #pragma unroll
     for (int j = 0; j < RPL; ++j) {
       if (j == pj) {
-        pvr = (double)lane_read(xr[j][ca], pl);
-        pvi = (double)lane_read(xi[j][ca], pl);
+        pvr = (double)gj_lane_read(xr[j][ca], pl);
+        pvi = (double)gj_lane_read(xi[j][ca], pl);
         q = __builtin_amdgcn_readlane(pos[j], pl);
       }
     }

@@ -1,8 +1,8 @@
 // Fused selected solve for small blocks (gfx950): one workgroup per energy.
 //
-// Same algorithm, outputs and operation order as the general sweep of
-// rgf_selected_solve in rgf.hip (reference
-// src/qttools/greens_function_solver/rgf.py:164-414), for stacks whose blocks
+// Same algorithm and outputs as rgf_selected_solve in rgf.hip, in the operation
+// order of its general sweep (four products per lesser / greater block backward;
+// reference src/qttools/greens_function_solver/rgf.py:164-414), for stacks whose blocks
 // are all at most kSB = 32 wide and at most kSN = 32 long.  At such sizes every
 // block product is a few microseconds of matrix-core work, so the general path
 // (one launch per product over the whole stack) is bound by launch latency;
