@@ -122,3 +122,27 @@ def test_inverse_bits(device, n_e, sizes, precision):
         return {"x": x.data, "in place": y.data}
 
     _same_bits(device, call, (2, 3, 4))
+
+
+@pytest.mark.parametrize("n_e,sizes", STACKS, ids=["518x64", "250x256"])
+def test_offset_of_the_ranges_bits(device, monkeypatch, n_e, sizes):
+    """The odd ranges start after the first one's first block inverse
+    (QX_RGF_STAGGER): the bits of ranges started together, over several calls on
+    one handle."""
+    a = _stack(device, sizes, n_e, 1, False)
+    sl, sg = _stack(device, sizes, n_e, 2, True), _stack(device, sizes, n_e, 3, True)
+
+    def call():
+        out = [empty_btd(sizes, (n_e,), device=device)[0] for _ in range(3)]
+        for _ in range(3):
+            RGF(n_e).selected_solve(a, sl, sg, out=tuple(out), return_retarded=True)
+        return {k: m.data for k, m in enumerate(out)}
+
+    outs = []
+    for stagger in ("1", "0"):
+        monkeypatch.setenv("QX_RGF_STAGGER", stagger)
+        outs.append(_on_streams(device, 4, call))
+    (ref, launches), (got, n) = outs
+    assert n == launches == 4 * _on_streams(device, 1, call)[1]
+    for k in ref:
+        assert torch.equal(torch.view_as_real(got[k]), torch.view_as_real(ref[k]))
