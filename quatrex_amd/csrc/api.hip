@@ -185,7 +185,8 @@ int split_count(const qx_handle* h, int64_t S, int b) {
 }
 
 void run_split(qx_handle* h, hipStream_t st, int64_t S, int b,
-               const std::function<void(hipStream_t, int64_t, int64_t)>& f) {
+               const std::function<void(hipStream_t, int64_t, int64_t)>& f,
+               const std::function<void(int)>& lost) {
   const int P = split_count(h, S, b);
   if (P <= 1) {
     f(st, 0, S);
@@ -218,6 +219,7 @@ void run_split(qx_handle* h, hipStream_t st, int64_t S, int b,
         f(h->streams[k - 1], e0[k], e0[k + 1] - e0[k]);
       } catch (...) {
         err[k] = std::current_exception();
+        if (lost) lost(k);
       }
       active_timer = nullptr;
     });
@@ -227,6 +229,7 @@ void run_split(qx_handle* h, hipStream_t st, int64_t S, int b,
     f(st, 0, e0[1]);
   } catch (...) {
     err[0] = std::current_exception();
+    if (lost) lost(0);
   }
   for (auto& t : threads) t.join();
   for (int k = 1; k < P; ++k) {

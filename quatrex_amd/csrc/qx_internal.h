@@ -333,13 +333,16 @@ void noalloc_init(int device);
 
 // Sub-batches run_split makes of S matrices with blocks of at most b.
 int split_count(const qx_handle* h, int64_t S, int b);
-// Splits a batch of S matrices (blocks of at most b) into split_count, at most
-// `handle->parts`, contiguous sub-batches and runs f(stream, e0, n) for each concurrently: sub-batch 0 on
+// Splits a batch of S matrices (blocks of at most b) into split_count contiguous
+// sub-batches and runs f(stream, e0, n) for each concurrently: sub-batch 0 on
 // the caller's stream `st` in this thread, the others on handle-owned streams
 // from helper host threads.  Events order all sub-batches after the work
 // already queued on `st`, and `st` waits for all of them before returning.
+// lost(k) is called where sub-batch k ends with an error (one that others wait
+// for is never silent).
 void run_split(qx_handle* h, hipStream_t st, int64_t S, int b,
-               const std::function<void(hipStream_t, int64_t, int64_t)>& f);
+               const std::function<void(hipStream_t, int64_t, int64_t)>& f,
+               const std::function<void(int)>& lost = nullptr);
 // Index of the sub-batch the calling thread runs inside run_split (0 on the
 // caller's thread).
 extern thread_local int split_part;

@@ -10,6 +10,7 @@
 // stored (e.g. Sigma_{i,i+1} of a block-diagonal self-energy) are skipped:
 // they are exactly zero.
 #include <algorithm>
+#include <chrono>
 #include <cstdlib>
 #include <cstring>
 #include <future>
@@ -425,25 +426,21 @@ void rgf_selected_solve(qx_handle* h, hipStream_t st0, const qx_btd_layout* la,
   if (skew_on) h->ensure_words();
   // Each sub-batch checks its own blocks and all wait for every answer: one
   // sweep for the whole call, so that the number of sub-batches changes no bit.
-  // true: the sub-batch's answer is on its way (its event is recorded).
+  // true: the sub-batch's answer is on its way (its event is recorded); false:
+  // the sub-batch ended with an error before.
   std::vector<std::promise<bool>> votes(skew_on ? split_count(h, Stot, bmax) : 0);
   std::vector<std::shared_future<bool>> voted;
   for (auto& v : votes) voted.push_back(v.get_future().share());
+  auto lost = [&](int k) {
+    if (skew_on && voted[k].wait_for(std::chrono::seconds(0)) != std::future_status::ready)
+      votes[k].set_value(false);
+  };
   hipEvent_t stg_ev = nullptr;
   if (stagger) QX_HIP_CHECK(hipEventCreateWithFlags(&stg_ev, hipEventDisableTiming));
   std::promise<void> stg_set;
   std::shared_future<void> stg_ready = stg_set.get_future().share();
   run_split(h, st0, Stot, bmax, [&](hipStream_t st, int64_t e0, int64_t S) {
   const int part = split_part;
-  // a sub-batch that leaves early with an error has no answer
-  struct Vote {
-    std::promise<bool>* p;
-    void cast(bool queued) {
-      if (p) p->set_value(queued);
-      p = nullptr;
-    }
-    ~Vote() { cast(false); }
-  } vote{skew_on ? &votes[part] : nullptr};
   const OzSubBatch oz(prec, oz_region, bmax, e0, S);
   // sub-batch 0 releases the others once its first inverse is enqueued, or
   // when it leaves early with an error
@@ -570,7 +567,7 @@ void rgf_selected_solve(qx_handle* h, hipStream_t st0, const qx_btd_layout* la,
     QX_HIP_CHECK(hipMemcpyAsync(h->word_host + part, flag, sizeof(int), hipMemcpyDeviceToHost,
                                 st));
     QX_HIP_CHECK(hipEventRecord(h->part_ev[part], st));
-    vote.cast(true);
+    votes[part].set_value(true);
   }
 
   // ---- forward sweep (rgf.py:234-295) ----
@@ -862,7 +859,7 @@ void rgf_selected_solve(qx_handle* h, hipStream_t st0, const qx_btd_layout* la,
     gr[i] = Zr;
     if (lds) ew_diag_imag(st, S, bi, gr[i], lds + orb_off[i], n_orb, kLdos);
   }
-  });
+  }, lost);
   // released once the waits enqueued on it have been satisfied
   if (stg_ev) QX_HIP_CHECK(hipEventDestroy(stg_ev));
 }
