@@ -69,6 +69,19 @@ struct GjShape {
   static constexpr int THREADS = 64 * (MW + 1);
 };
 
+// Whether products are summed before they are subtracted from the matrix (one
+// rounding of the matrix's size per column in the factoring wave and per
+// sub-panel in the update) instead of fused into it (two per column).  Up to 32
+// rows the kernel before this one summed.  Error against it, geometric mean over
+// 600 matrices, fused / summed: n = 20 1.13 to 1.18 / 1.02 to 1.06, n = 32 1.13 to
+// 1.20 / 1.04 (what is left are the sub-panels' composite coefficients).  It costs
+// 0 to 2 % (256 x 32^2 21.1 -> 21.3 us; a solve of 16 energies, 8 blocks of 32
+// 533 -> 540).  Above 32 the kernels before fused as well (n = 48, 64: the same
+// error, n = 128: 0.83 of theirs), and at 64 the registers of the sums halve the
+// workgroups of a CU (4096 x 64^2 551 -> 751 us).
+template <typename G>
+constexpr bool gj_exact = G::CT <= 2;
+
 template <typename G>
 struct GjShared {
   z2 sub[2][G::SB][G::LS];  // sub-panel columns, alternating buffers
@@ -151,8 +164,13 @@ __device__ __forceinline__ void gj_factor(GjShared<G>& sh, z2 (*sub)[G::LS], int
             xr[j][u] = -mr;
             xi[j][u] = -mi;
           } else {
-            xr[j][u] = fma(-mr, ar[u], fma(mi, ai[u], xr[j][u]));
-            xi[j][u] = fma(-mr, ai[u], fma(-mi, ar[u], xi[j][u]));
+            if constexpr (gj_exact<G>) {
+              xr[j][u] -= fma(mr, ar[u], -(mi * ai[u]));
+              xi[j][u] -= fma(mr, ai[u], mi * ar[u]);
+            } else {
+              xr[j][u] = fma(-mr, ar[u], fma(mi, ai[u], xr[j][u]));
+              xi[j][u] = fma(-mr, ai[u], fma(-mi, ar[u], xi[j][u]));
+            }
           }
         }
         // interchange k + c <-> q: row p moves to position k + c
@@ -191,10 +209,19 @@ __device__ __forceinline__ void gj_factor(GjShared<G>& sh, z2 (*sub)[G::LS], int
 
 // Update waves: the rank-SB update by sub-panel `sub` of the column tile that
 // starts at panel column col.
+//
+// gj_exact: the rank-SB sum is formed from zero and then added (see there).
 template <typename G>
 __device__ __forceinline__ void gj_update(const GjShared<G>& sh, const z2 (*sub)[G::LS], int row0,
                                           int l16, int l4, int col, gj_acc (&cr)[G::RT],
                                           gj_acc (&ci)[G::RT]) {
+  constexpr bool SUM = gj_exact<G>;
+  gj_acc sr[G::RT], si[G::RT];
+#pragma unroll
+  for (int i = 0; i < G::RT; ++i) {
+    sr[i] = SUM ? gj_acc{0.0, 0.0, 0.0, 0.0} : cr[i];
+    si[i] = SUM ? gj_acc{0.0, 0.0, 0.0, 0.0} : ci[i];
+  }
 #pragma unroll
   for (int ks = 0; ks < G::SB / 4; ++ks) {
     __builtin_amdgcn_sched_barrier(0);  // operands of one k-step at a time: registers
@@ -204,14 +231,19 @@ __device__ __forceinline__ void gj_update(const GjShared<G>& sh, const z2 (*sub)
     for (int i = 0; i < G::RT; ++i) a[i] = sub[4 * ks + l4][row0 + 16 * i + l16];
 #pragma unroll
     for (int i = 0; i < G::RT; ++i) {
-      cr[i] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[i].x, b.x, cr[i], 0, 0, 0);
-      ci[i] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[i].x, b.y, ci[i], 0, 0, 0);
+      sr[i] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[i].x, b.x, sr[i], 0, 0, 0);
+      si[i] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[i].x, b.y, si[i], 0, 0, 0);
     }
 #pragma unroll
     for (int i = 0; i < G::RT; ++i) {
-      cr[i] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[i].y, b.y, cr[i], 0, 0, 1);
-      ci[i] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[i].y, b.x, ci[i], 0, 0, 0);
+      sr[i] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[i].y, b.y, sr[i], 0, 0, 1);
+      si[i] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[i].y, b.x, si[i], 0, 0, 0);
     }
+  }
+#pragma unroll
+  for (int i = 0; i < G::RT; ++i) {
+    cr[i] = SUM ? cr[i] + sr[i] : sr[i];
+    ci[i] = SUM ? ci[i] + si[i] : si[i];
   }
 }
 
