@@ -69,18 +69,23 @@ struct GjShape {
   static constexpr int THREADS = 64 * (MW + 1);
 };
 
-// Whether products are summed before they are subtracted from the matrix (one
+// Whether products are summed before they are subtracted from the matrix, one
 // rounding of the matrix's size per column in the factoring wave and per
-// sub-panel in the update) instead of fused into it (two per column).  Up to 32
-// rows the kernel before this one summed.  Error against it, geometric mean over
-// 600 matrices, fused / summed: n = 20 1.13 to 1.18 / 1.02 to 1.06, n = 32 1.13 to
-// 1.20 / 1.04 (what is left are the sub-panels' composite coefficients).  It costs
-// 0 to 2 % (256 x 32^2 21.1 -> 21.3 us; a solve of 16 energies, 8 blocks of 32
-// 533 -> 540).  Above 32 the kernels before fused as well (n = 48, 64: the same
-// error, n = 128: 0.83 of theirs), and at 64 the registers of the sums halve the
-// workgroups of a CU (4096 x 64^2 551 -> 751 us).
+// sub-panel in the update, or fused into it, two per column.  Error against the
+// kernels before this one, which summed up to 32 rows and fused above; geometric
+// means over 400 to 2000 matrices (+- 0.01 to 0.02):
+//            fused           update summed   both summed
+//   n = 20   1.16            1.06            1.02
+//   n = 32   1.15 to 1.20    1.07            1.03 to 1.04
+//   n = 48   1.02 to 1.04    0.90 to 0.93
+//   n = 64   0.99 to 1.05    0.89 to 0.92
+//   n = 128  0.78 to 0.84
+// (What is left at 32 are the sub-panels' composite coefficients.)  Up to 32 the
+// sums cost 0 to 2 % of an inverse (256 x 32^2 20.7 -> 21.3 us; a solve of 16
+// energies, 8 blocks of 32 533 -> 540); at 64 the registers of the update's halve
+// the workgroups of a CU (4096 x 64^2 551 -> 751 us).
 template <typename G>
-constexpr bool gj_exact = G::CT <= 2;
+constexpr bool kSums = G::CT <= 2;
 
 template <typename G>
 struct GjShared {
@@ -164,7 +169,7 @@ __device__ __forceinline__ void gj_factor(GjShared<G>& sh, z2 (*sub)[G::LS], int
             xr[j][u] = -mr;
             xi[j][u] = -mi;
           } else {
-            if constexpr (gj_exact<G>) {
+            if constexpr (kSums<G>) {
               xr[j][u] -= fma(mr, ar[u], -(mi * ai[u]));
               xi[j][u] -= fma(mr, ai[u], mi * ar[u]);
             } else {
@@ -210,12 +215,12 @@ __device__ __forceinline__ void gj_factor(GjShared<G>& sh, z2 (*sub)[G::LS], int
 // Update waves: the rank-SB update by sub-panel `sub` of the column tile that
 // starts at panel column col.
 //
-// gj_exact: the rank-SB sum is formed from zero and then added (see there).
+// kSums: the rank-SB sum is formed from zero and then added.
 template <typename G>
 __device__ __forceinline__ void gj_update(const GjShared<G>& sh, const z2 (*sub)[G::LS], int row0,
                                           int l16, int l4, int col, gj_acc (&cr)[G::RT],
                                           gj_acc (&ci)[G::RT]) {
-  constexpr bool SUM = gj_exact<G>;
+  constexpr bool SUM = kSums<G>;
   gj_acc sr[G::RT], si[G::RT];
 #pragma unroll
   for (int i = 0; i < G::RT; ++i) {

@@ -578,8 +578,16 @@ __device__ __forceinline__ void panel_cg(const PanelArgs& g, int64_t e,
     for (int j = 0; j < RPL; ++j) {
 #pragma unroll
       for (int c = 0; c < CW; ++c) {
-        xr[j][c] = fma(-fr[j], sr[c], fma(fi[j], si[c], xr[j][c]));
-        xi[j][c] = fma(-fr[j], si[c], fma(-fi[j], sr[c], xi[j][c]));
+        if constexpr (NB == 64) {
+          // the product first (inv_panel_width); the empty asm ends each element's
+          // temporaries, which the compiler otherwise keeps all and spills
+          xr[j][c] -= fma(fr[j], sr[c], -(fi[j] * si[c]));
+          xi[j][c] -= fma(fr[j], si[c], fi[j] * sr[c]);
+          asm volatile("" : "+v"(xr[j][c]), "+v"(xi[j][c]));
+        } else {
+          xr[j][c] = fma(-fr[j], sr[c], fma(fi[j], si[c], xr[j][c]));
+          xi[j][c] = fma(-fr[j], si[c], fma(-fi[j], sr[c], xi[j][c]));
+        }
       }
     }
   };
@@ -807,24 +815,33 @@ __device__ __forceinline__ void update_tile(const UpdArgs& g, const UpdTile& u, 
   if (tid < 64) sig_r[tid] = (r0 + tid < n) ? sig[r0 + tid] : 0;
   if (tid < NB) sig_k[tid] = (tid < nbw) ? sig[k0 + tid] : 0;
   __syncthreads();
-  // C init: gathered rows, pivot rows zeroed.  Issued before the operand
-  // staging below so that both sets of loads are in flight together.
-  acc_t aR[2][2], aI[2][2];
+  // C: gathered rows, pivot rows zeroed.  The accumulators start from it; a
+  // rank-64 sum (inv_panel_width) starts from zero and C is added to it.
+  constexpr bool SUM = NB == 64;
+  acc_t aR[2][2], aI[2][2], cR[2][2], cI[2][2];
+#define QX_LOAD_C(DR, DI)                                                                \
+  _Pragma("unroll") for (int i = 0; i < 2; ++i)                                          \
+  _Pragma("unroll") for (int j = 0; j < 2; ++j)                                          \
+  _Pragma("unroll") for (int q = 0; q < 4; ++q) {                                        \
+    const int rl = wm * 32 + i * 16 + MM::row(lane, q);                                  \
+    const int r = r0 + rl;                                                               \
+    const int c = c0 + wn * 32 + j * 16 + (lane & 15);                                   \
+    /* unconditional loads from clamped addresses: all in flight together */             \
+    const bool ok = live && r < n && c < n && !(r >= k0 && r < k0 + nbw);                \
+    const z2 v = Xc[ok ? (int64_t)sig_r[rl] * g.ldc + c : 0];                            \
+    DR[i][j][q] = ok ? (T)v.x : (T)0;                                                    \
+    DI[i][j][q] = ok ? (T)v.y : (T)0;                                                    \
+  }
+  if constexpr (SUM) {
 #pragma unroll
-  for (int i = 0; i < 2; ++i)
+    for (int i = 0; i < 2; ++i)
 #pragma unroll
-    for (int j = 0; j < 2; ++j)
-#pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        const int rl = wm * 32 + i * 16 + MM::row(lane, q);
-        const int r = r0 + rl;
-        const int c = c0 + wn * 32 + j * 16 + (lane & 15);
-        // unconditional loads from clamped addresses: all in flight together
-        const bool ok = live && r < n && c < n && !(r >= k0 && r < k0 + nbw);
-        const z2 v = Xc[ok ? (int64_t)sig_r[rl] * g.ldc + c : 0];
-        aR[i][j][q] = ok ? (T)v.x : (T)0;
-        aI[i][j][q] = ok ? (T)v.y : (T)0;
-      }
+      for (int j = 0; j < 2; ++j) aR[i][j] = aI[i][j] = acc_t{0, 0, 0, 0};
+  } else {
+    // before the operand staging below, so that both sets of loads are in
+    // flight together
+    QX_LOAD_C(aR, aI)
+  }
   // per chunk: A = reduced panel rows of this tile, B = gathered pivot rows;
   // all loads first (unconditional, clamped addresses), then the LDS writes
   constexpr int NS = 64 * KW / NT;
@@ -855,6 +872,11 @@ __device__ __forceinline__ void update_tile(const UpdArgs& g, const UpdTile& u, 
       Bs[1][k2][c] = (T)vb[it].y;
     }
     __syncthreads();
+    if constexpr (SUM) {
+      if (kc + KW >= NB) {  // C beside the last chunk's products
+        QX_LOAD_C(cR, cI)
+      }
+    }
 #pragma unroll
     for (int kq = 0; kq < KW / 4; ++kq) {
       const int kr = kq * 4 + (lane >> 4);
@@ -882,6 +904,16 @@ __device__ __forceinline__ void update_tile(const UpdArgs& g, const UpdTile& u, 
           aI[i][j] = MM::mma(a_i[i], b_r[j], aI[i][j]);
         }
     }
+  }
+#undef QX_LOAD_C
+  if constexpr (SUM) {
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+      for (int j = 0; j < 2; ++j) {
+        aR[i][j] += cR[i][j];
+        aI[i][j] += cI[i][j];
+      }
   }
   if (!live) return;
 #pragma unroll
@@ -1164,7 +1196,8 @@ void run_inverse(hipStream_t s, int64_t batch, int n, const Mat& X, const InvScr
                  B[nxt].p, B[nxt].stride, B[nxt].ld, scr.ints, scr.int_stride, mask};
       const dim3 grid(groups(batch * tn * tn, NT, "inv"));
       if (narrow_update(batch))
-        hipLaunchKernelGGL((inv_update<T, NB, 16, 4>), grid, dim3(NT), 0, s, ua);
+        // (three waves per SIMD where the sum and C are both held)
+        hipLaunchKernelGGL((inv_update<T, NB, 16, NB == 64 ? 3 : 4>), grid, dim3(NT), 0, s, ua);
       else
         hipLaunchKernelGGL((inv_update<T, NB, 32, 1>), grid, dim3(NT), 0, s, ua);
     }
@@ -1221,18 +1254,22 @@ void launch_whole(hipStream_t s, int64_t batch, int n, const Mat& A, const Mat& 
 // on the updates stream every matrix through HBM, and 64-column panels (eight
 // waves of eight columns, n <= 256) halve the passes over it.  32 / 64 columns,
 // us per call:
-//   matrices        128        160        192        256        257        512
-//   n = 192     463/ 496   547/ 524   654/ 581   809/ 680   869/ 933  1399/1315
-//   n = 208     671/ 747   835/ 855   961/ 959  1229/1171  1320/1470  2179/2294
-//   n = 224     713/ 793   894/ 904  1092/1066  1305/1244  1407/1561  2316/2427
-//   n = 240     829/ 847  1095/1004  1304/1146  1512/1322  1628/1658  2694/2577
-//   n = 256     880/ 879  1173/1076  1390/1200  1621/1398  1739/1749  2911/2800
-// The lines: 160 matrices (below, the look-ahead of the 32-column panels wins or
-// is close), 192 where the last panel is at most half full, never where it is
-// nearly empty (300 x 200^2 1.43 -> 1.56 ms) or the matrix has fewer than three
-// (512 x 160^2 1.05 -> 1.13); and 256, the CUs of the chip, each with one panel:
-// beyond it the longer panels take a second round, which 4 % at 512 matrices of
-// some sizes do not repay at 257 to 320.
+//   matrices        144        160        192        224        256        257
+//   n = 192     500/ 538   546/ 551   654/ 615   780/ 665   812/ 708   870/1002
+//   n = 208     801/ 834   834/ 886   963/ 987  1208/1146  1230/1187  1321/1529
+//   n = 224     866/ 889   894/ 936  1092/1098  1293/1227  1306/1262  1408/1627
+//   n = 240     997/ 935  1095/1046  1302/1191  1551/1315  1513/1338  1629/1726
+//   n = 256    1103/1048  1170/1119  1393/1247  1669/1375  1630/1408  1740/1810
+// The lines: 160 matrices, 224 where the last panel is at most half full, never
+// where it is nearly empty (300 x 200^2 1.43 -> 1.56 ms) or the matrix has fewer
+// than three (512 x 160^2 1.05 -> 1.13); and 256, the CUs of the chip, each with
+// one panel: beyond it the longer panels take a second round.
+// A panel's composite coefficients grow less accurate with its width, so the
+// 64-column panels and their rank-64 updates sum products before they subtract
+// them: error against 32 columns, geometric means over 500 matrices (+- 0.02),
+// 192: 0.93 to 0.97, 208: 1.00, 224 to 256: 1.02 to 1.05 (fused product by
+// product 1.01 to 1.03, 1.11, 1.09 to 1.16; 1.40 ms instead of 1.41 at 256 x
+// 256^2).
 // steady calls (the block inverses of the RGF, whose sub-batches and batches
 // would else decide over the bits of a result) keep 32.
 // QX_INV_NB=16|32|64 overrides for n <= 256 (16 runs the one-thread-per-row
@@ -1243,7 +1280,7 @@ int inv_panel_width(int64_t batch, int n, int precision, bool steady) {
   if (forced_nb == 64 && inv_panel_kind() != 0) return 32;
   if (forced_nb) return forced_nb;
   const int last = (n - 1) % 64 + 1;  // columns of the last 64-column panel
-  const bool wide = !steady && batch >= (last > 32 ? 160 : 192) && batch <= 256 && n >= 192 &&
+  const bool wide = !steady && batch >= (last > 32 ? 160 : 224) && batch <= 256 && n >= 192 &&
                     last >= 16;
   return wide && precision != QX_PREC_C64 && inv_panel_kind() == 0 && inv_group_width() == 4
              ? 64

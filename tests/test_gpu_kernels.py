@@ -493,7 +493,7 @@ def test_whole_inverse_singular_raises(device, n):
 
 
 @pytest.mark.parametrize("batch,n,wide", [(159, 240, False), (160, 240, True), (160, 208, False),
-                                          (191, 224, False), (192, 224, True), (192, 208, True),
+                                          (223, 224, False), (224, 224, True), (224, 208, True),
                                           (256, 207, False), (257, 256, False), (256, 191, False)])
 def test_wide_panel_lines(device, monkeypatch, batch, n, wide):
     """Which calls take 64-column panels: the bits are those of the width forced,
@@ -596,26 +596,53 @@ def test_smallest_whole_inverse_against_split_kernels(device, monkeypatch, n, ba
         assert rel_err(outs[0][e], np.linalg.inv(a[e] - s[e])) < tol
 
 
-@pytest.mark.parametrize("n", [24, 32])
-def test_whole_inverse_rounding(device, monkeypatch, n):
-    """Up to 32 rows products are summed before they are subtracted: over 600
-    matrices E + i eta - H, H Hermitian, the geometric mean of the error (against
-    the inverse refined in extended precision) is no larger than that of the
-    split panels, which choose the same pivots and fuse product by product."""
-    rng = np.random.default_rng(n)
-    x = _cplx(rng, (600, n, n))
-    h = (x + x.conj().transpose(0, 2, 1)) / 2 / np.sqrt(n)
-    a = (rng.uniform(-1, 1, 600) + 1e-3j)[:, None, None] * np.eye(n) - h
-    A = torch.as_tensor(a, device=device)
-    ref = np.linalg.inv(a).astype(np.clongdouble)
-    wide, eye = a.astype(np.clongdouble), np.eye(n)
-    for _ in range(2):
-        ref = ref + ref @ (eye - wide @ ref)
-    log_error = {}
-    for whole in ("32", "0"):
-        monkeypatch.setenv("QX_INV_WHOLE", whole)
+def _inverse_error(A, X):
+    """Log of the relative error of X as the inverse of A, per matrix: |X R| / |X|
+    with the residual R = I - A X from products of 22-bit slices, whose sums over
+    up to 256 terms are exact in double precision."""
+    def slices(m, dim):
+        scale = torch.exp2(torch.ceil(torch.log2(m.abs().amax(dim, keepdim=True))))
+        out, rest = [], m / scale
+        for k in (1, 2, 3):
+            s = torch.round(rest * 2.0 ** (22 * k)) / 2.0 ** (22 * k)
+            out.append(s * scale)
+            rest = rest - s
+        return out
+
+    def products(a, b):
+        sa, sb = slices(a.contiguous(), -1), slices(b.contiguous(), -2)
+        return [(i + j, sa[i] @ sb[j]) for i in range(3) for j in range(3) if i + j < 4]
+
+    re = products(A.real, X.real) + [(k, -p) for k, p in products(A.imag, X.imag)]
+    im = products(A.real, X.imag) + products(A.imag, X.real)
+    r = torch.eye(A.shape[-1], dtype=torch.float64, device=A.device).expand(A.shape)
+    i = torch.zeros_like(r)
+    for _, p in sorted(re, key=lambda t: t[0]):
+        r = r - p
+    for _, p in sorted(im, key=lambda t: t[0]):
+        i = i - p
+    e = X @ torch.complex(r, i)
+    return (torch.linalg.norm(e, dim=(-2, -1)) / torch.linalg.norm(X, dim=(-2, -1))).log()
+
+
+@pytest.mark.parametrize("n,batch,knob,values,most", [
+    (24, 1000, "QX_INV_WHOLE", ("32", "0"), -0.05), (32, 1000, "QX_INV_WHOLE", ("32", "0"), -0.05),
+    (208, 250, "QX_INV_NB", ("64", "32"), 0.07), (256, 250, "QX_INV_NB", ("64", "32"), 0.07)])
+def test_inverse_rounding(device, monkeypatch, n, batch, knob, values, most):
+    """Where products are summed before they are subtracted (whole inverses up to
+    32 rows, 64-column panels) the error is not above that of the 32-column panels
+    beside them, which choose the same pivots and fuse product by product: mean of
+    the logarithm over matrices E + i eta - H, H Hermitian, standard error 0.01 and
+    0.03.  Fused they were 0.03 to 0.06 and 0.10 to 0.17 above."""
+    g = torch.Generator(device=device).manual_seed(n)
+    x = torch.randn((batch, n, n), dtype=torch.complex128, device=device, generator=g)
+    h = (x + x.conj().transpose(1, 2)) / (2 * n) ** 0.5
+    e = 2 * torch.rand((batch, 1, 1), dtype=torch.float64, device=device, generator=g) - 1
+    A = (e + 1e-3j) * torch.eye(n, device=device) - h
+    log = []
+    for v in values:
+        monkeypatch.setenv(knob, v)
         X = torch.empty_like(A)
         _inv(device, A, X, 0)
-        e = np.abs(X.cpu().numpy() - ref).astype(float)
-        log_error[whole] = np.log((e ** 2).sum((1, 2))) / 2
-    assert (log_error["32"] - log_error["0"]).mean() <= 0.0
+        log.append(_inverse_error(A, X))
+    assert float((log[0] - log[1]).mean()) <= most
