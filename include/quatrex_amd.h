@@ -72,10 +72,11 @@ extern "C" {
 #define QX_SOLVE_SKIP_LOWER_L 8u     /* lesser output is symmetric-stored      */
 #define QX_SOLVE_SKIP_LOWER_G 16u    /* greater output is symmetric-stored     */
 /* The call may wait for the device once: it checks whether every diagonal
- * S^{<>} block and lesser / greater boundary block is skew-Hermitian (to 64
- * eps of its largest entry) and, if so, runs the backward sweep with three
- * products per quantity and block instead of four (complex128 arithmetic; same
- * results to rounding).  Ignored while the stream records a graph. */
+ * S^{<>} block and lesser / greater boundary block of all its energies is
+ * skew-Hermitian (to 64 eps of its largest entry) and, if so, runs the backward
+ * sweep with three products per quantity and block instead of four (complex128
+ * arithmetic; same results to rounding).  Ignored while the stream records a
+ * graph and where the memory of two outputs overlaps. */
 #define QX_SOLVE_SKEW_CHECK 32u
 
 typedef struct qx_handle qx_handle;
@@ -302,7 +303,8 @@ int qx_zgemm_ozaki(qx_handle* handle, void* stream, int64_t batch, int m, int n,
 
 /* Execution tuning of a handle (no counterpart in the reference): streams =
  * concurrent sub-batches of one RGF call at most (1..8, default 4, env
- * QX_RGF_STREAMS; fewer where a block product of the call is small); gemm_tile = one of QX_GEMM_* (env QX_ZGEMM_TILE,
+ * QX_RGF_STREAMS; fewer where a block product of the call is small; same
+ * results bitwise); gemm_tile = one of QX_GEMM_* (env QX_ZGEMM_TILE,
  * QX_ZGEMM_KERNEL and QX_ZGEMM_REG override it).  Used by the autotuner and
  * by callers that run several handles side by side. */
 int qx_set_tuning(qx_handle* handle, int streams, int gemm_tile);

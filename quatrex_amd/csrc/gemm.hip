@@ -590,7 +590,8 @@ __device__ __forceinline__ void zgemm_wave(const GemmArgs& g, const GemmSet& P, 
 // a matrix takes ceil(m / 16 TM) x ceil(n / 16 TN) of them, and only its last
 // 32 rows and columns are padded, not its last 64.  96 products of n x n,
 // padded to 64 -> to 32: n = 80 25 -> 17 us, 96 30 -> 18, 132 71 -> 54,
-// 160 84 -> 64, 205 160 -> 135, 416 930 -> 777; multiples of 64 as before.
+// 160 84 -> 64, 205 160 -> 135, 416 930 -> 777; multiples of 64 to 5 % (1024 of
+// 64 x 64 A B 42 -> 44, A B^H 46 -> 43.5; 512 of 256 983 -> 978, 967 -> 960).
 // Half tiles for the waves at the edges (padding to 16) gained nothing: the
 // time of a wave with few MFMAs is the latency of its loads, and the four waves
 // drift apart in L1 (176: 91 -> 92 us, 161: 86 -> 90).

@@ -26,12 +26,13 @@
 // - A barrier closes every step, which makes its writes visible to the other
 //   waves of the workgroup.
 //
-// Bound by the chain of steps: of about 65 us per layer of 32 the inverse takes
-// 17 and each of the 15 product steps 1.5 to 5, for under 1 of matrix-core
-// work.  With all blocks in L2 and 16 blocks at most, before -> now: 16
-// energies of 8 blocks of 32 677 -> 536 us, 300 of 11 blocks of 20 1101 -> 879;
-// against one launch per product: 16 of 32 x 32 2.0 ms (4.9), 512 of 32 x 32
-// 4.3 (9.4), 64 of 24 x 16 0.9 (2.6), 1024 of 16 x 32 4.2 (6.3).
+// Bound by the chain of steps: of about 51 us per layer of 32 (59 with the layer
+// current) the inverse takes 17 and each of the 15 product steps 1.5 to 5, for
+// under 1 of matrix-core work.  Calls, with all blocks in L2 and 16 blocks at
+// most before -> now: 16 energies of 8 blocks of 32 677 -> 540 us, 300 of 11
+// blocks of 20 1101 -> 894; against one launch per product: 16 of 32 x 32 2.0 ms
+// (4.9), 512 of 32 x 32 4.3 (9.4), 64 of 24 x 16 0.9 (2.6), 1024 of 16 x 32 4.2
+// (6.3).
 #include <algorithm>
 #include <cstdlib>
 
